@@ -64,6 +64,24 @@ int kvq_kivi_quant(const void* x, int x_dtype, int64_t B, int64_t H, int64_t T, 
                    float* xhat, void* stream);
 
 /* ------------------------------------------------------------------------------------------
+ * A1  A whole context into the decode cache in two launches: what KIVIMethod leaves at a horizon
+ * (STRATA_KV.py:801-823, no sinks).  k, v: (B, H, T, 128) of one dtype with element strides, channels
+ * contiguous.  Rows [0, n_q = T - window) are coded at 4 bits as kvq_kivi_quant codes them (key groups over
+ * all T rows) into the layouts of kvq_kivi_decode: kc (BH, cap_t, 64) pack_codes rows (the codes of every
+ * row of the key groups that hold a packed row), k_lo / k_sc (BH, cap_t / group_k, 128), vc value tiles
+ * (BH, cap_t / 32, 2048), vmeta (BH, cap_t / 32, 128 / group_v, 32, 2).  The last `window` rows go to
+ * k_exact / v_exact (BH, cap_e, 128): row n_q + i at slot i, or with `ring` (cap_e == window) at slot
+ * (n_q + i) % cap_e.  Every byte of the outputs is written; what holds no row is zero.
+ * group_k, group_v in {32, 64, 128}; cap_t a multiple of 32 and group_k; pointers and strides (in
+ * bytes) multiples of 16; token strides >= 128 elements.
+ * ---------------------------------------------------------------------------------------- */
+int kvq_kivi_compress(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb,
+                      int64_t v_sh, int64_t v_st, int dtype, int64_t B, int64_t H, int64_t T, int64_t d,
+                      int64_t window, int group_k, int group_v, int64_t cap_t, uint8_t* kc, uint16_t* k_lo,
+                      uint16_t* k_sc, uint8_t* vc, uint16_t* vmeta, void* k_exact, void* v_exact,
+                      int64_t cap_e, int ring, void* stream);
+
+/* ------------------------------------------------------------------------------------------
  * A3  Bit packing.  kvq_pack_codes replaces pack_codes (STRATA_KV.py:2728-2732): `count`
  * uint8 codes (< 2^bits) -> ceil(count*bits/8) bytes, first code in the most significant bits,
  * last byte zero padded.  kvq_unpack_codes is its inverse.  bits in {1, 2, 4, 8}.

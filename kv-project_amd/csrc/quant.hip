@@ -529,6 +529,26 @@ __device__ __forceinline__ uint32_t code_word4(const float (&v)[8], const float 
   return w;
 }
 
+// The same rounding for eight channels of one group: t[k] the clamped code as a float.
+__device__ __forceinline__ void codes4(const float (&v)[8], float lo, float sc, float rc, float (&t)[8]) {
+  bool near = false;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float p = __fmul_rn(__fsub_rn(v[k], lo), rc);
+    t[k] = rintf(p);
+    near |= fabsf(p - t[k]) > 0.4999f;
+  }
+  if (__builtin_expect(__any(near), 0)) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float dd = __fsub_rn(v[k], lo);
+      if (fabsf(__fmul_rn(dd, rc) - t[k]) > 0.4999f) t[k] = rintf(__fdiv_rn(dd, sc));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) t[k] = fminf(fmaxf(t[k], 0.0f), 15.0f);
+}
+
 // Keys: item = (group gi, b*h), group <= 4 RPL rows; per-channel min / max over the rows of the
 // lane, then over the four row lanes (permlane swaps).
 template <int DT, int RPL>
@@ -662,6 +682,244 @@ __global__ __launch_bounds__(256) void kivi_quant_values_p4(
         sc_out[mrow + static_cast<int64_t>(r) * NG] = f32_to_f16(s1);
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// A whole context straight into the decode cache (PackedKIVICache's layout, 4 bits, d == 128): every
+// output byte is written once, padding included, so nothing has to be cleared, packed, copied or
+// re-tiled behind these two launches.  Bound by memory: rows in, codes and metadata out.  At
+// 4 x 8 x 32845 bf16 rows a side (0.69 GB) the pair takes 136 us, 5.1 TB/s (a plain 2 GiB copy reaches
+// 4.9); the quantisers, the packed rows' copy into the cache, the value re-tiling and the fills that
+// it replaces, 19 launches, took 595 us.
+
+// Keys: an item is one key group of one (b, h), every group of the cache's capacity: the first n_gq hold
+// rows (all `group` of them, up to T: a group that straddles the window is coded over its rows), the
+// others are written as zeros.  WPI wavefronts share an item (lane (s, rq) of wavefront w: channels
+// 8s .. 8s+7 of rows 4 RPL w + rq + 4 j), so that a lane holds at most 64 registers of rows at every
+// group size and type; with WPI > 1 the wavefronts' ranges meet in LDS.
+template <int DT, int RPL, int WPI>
+__global__ __launch_bounds__(256) void kivi_compress_keys(const void* __restrict__ x, int H, int64_t sb, int64_t sh,
+                                                          int64_t st, int T, int n_gq, int cap_g,
+                                                          uint8_t* __restrict__ kc, uint16_t* __restrict__ k_lo,
+                                                          uint16_t* __restrict__ k_sc, int64_t n_items) {
+  constexpr int D = 128, G = 4 * RPL * WPI, ES = DT == KVQ_F32 ? 4 : 2, NL = ES / 2;
+  __shared__ float red[WPI > 1 ? 2 : 1][WPI > 1 ? 4 : 1][WPI > 1 ? D : 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave % WPI;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * (4 / WPI) + wave / WPI;
+  const bool live = item < n_items;                 // no early exit: the wavefronts of an item meet at a barrier
+  const int s = lane & 15, rq = lane >> 4;
+  const int64_t bh = live ? item / cap_g : 0;
+  const int gi = live ? static_cast<int>(item - bh * cap_g) : 0;
+  const int64_t b = bh / H, h = bh - b * H;
+  const int64_t t0 = static_cast<int64_t>(gi) * G;
+  const int rv = live && gi < n_gq ? static_cast<int>(min(static_cast<int64_t>(G), T - t0)) : 0;   // rows held
+  const char* src = static_cast<const char*>(x) + (b * sb + h * sh + (rv > 0 ? t0 : 0) * st) * ES;
+  const uint32_t rstride = static_cast<uint32_t>(st * ES);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, static_cast<uint32_t>(rv) * rstride);
+  const int r0 = 4 * RPL * w + rq;
+  u32x4 raw[RPL * NL];                              // rows read once: non-temporal loads; past the rows: zeros
+#pragma unroll
+  for (int j = 0; j < RPL; ++j)
+#pragma unroll
+    for (int e = 0; e < NL; ++e)
+      raw[j * NL + e] = __builtin_amdgcn_raw_buffer_load_b128(rs, (r0 + 4 * j) * rstride + s * 8 * ES + 16 * e, 0, 2);
+  auto row = [&](int j, float (&v)[8]) {
+    if constexpr (DT == KVQ_F32) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = __uint_as_float(raw[j * NL + k / 4][k % 4]);
+    } else {
+      cvt_slab<DT>(raw[j], v);
+    }
+  };
+  float mn[8], mx[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    mn[k] = INFINITY;
+    mx[k] = -INFINITY;
+  }
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) {
+    const bool ok = r0 + 4 * j < rv;
+    float v[8];
+    row(j, v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      mn[k] = fminf(mn[k], ok ? v[k] : INFINITY);
+      mx[k] = fmaxf(mx[k], ok ? v[k] : -INFINITY);
+    }
+  }
+  // the rows are converted again when coded: only the raw words stay live across the reduction
+#pragma unroll
+  for (int j = 0; j < RPL * NL; ++j) asm volatile("" : "+v"(raw[j]));
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    mn[k] = xmin32(xmin16(mn[k]));
+    mx[k] = xmax32(xmax16(mx[k]));
+  }
+  if constexpr (WPI > 1) {
+    if (rq == 0) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        red[0][wave][8 * s + k] = mn[k];
+        red[1][wave][8 * s + k] = mx[k];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < WPI; ++o) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        mn[k] = fminf(mn[k], red[0][wave - w + o][8 * s + k]);
+        mx[k] = fmaxf(mx[k], red[1][wave - w + o][8 * s + k]);
+      }
+    }
+  }
+  if (!live) return;
+  float lo[8], sc[8], rc[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float l = as_stored(mn[k]);
+    const float q = fmaxf(as_stored(__fdiv_rn(__fsub_rn(mx[k], l), 15.0f)), kMinScale);
+    lo[k] = l;
+    sc[k] = q;
+    rc[k] = __builtin_amdgcn_rcpf(q);
+  }
+  if (rq == 0 && w == 0) {
+    const int64_t mo = item * D + s * 8;
+    u32x4 wl = {0, 0, 0, 0}, ws = {0, 0, 0, 0};
+    if (rv > 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        wl[k] = f32_to_f16(lo[2 * k]) | (static_cast<uint32_t>(f32_to_f16(lo[2 * k + 1])) << 16);
+        ws[k] = f32_to_f16(sc[2 * k]) | (static_cast<uint32_t>(f32_to_f16(sc[2 * k + 1])) << 16);
+      }
+    }
+    *reinterpret_cast<u32x4*>(k_lo + mo) = wl;
+    *reinterpret_cast<u32x4*>(k_sc + mo) = ws;
+  }
+  uint32_t* dst = reinterpret_cast<uint32_t*>(kc + (item * G + r0) * (D / 2)) + s;
+  if (rv == 0) {
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) __builtin_nontemporal_store(0u, &dst[4 * j * (D / 8)]);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) {
+    float v[8];
+    row(j, v);
+    const uint32_t cw = code_word4(v, lo, sc, rc);
+    __builtin_nontemporal_store(r0 + 4 * j < rv ? cw : 0u, &dst[4 * j * (D / 8)]);            // written once
+  }
+}
+
+// Word of a value chunk's LDS image: 4 words of padding behind every 64, so that the 64 lanes of a write
+// (word (s / 8) 256 + (16 g + 8 (s & 1) + k) 4 + (s / 2) % 4 of lane (g, s)) fall on 64 banks and the
+// 16-byte reads in word order stay aligned.
+__device__ __forceinline__ int v_image(int word) { return word + 4 * (word >> 6); }
+constexpr int kVImage = 512 + 4 * 8;
+
+// Values and exact rows.  The first item_blocks workgroups: a wavefront per CH chunks of 32 tokens.
+// Lane (g, s) loads channels 8s .. 8s+7 of the eight tokens of slots 8g .. 8g+7 (each load instruction
+// four whole rows), so the eight codes of a channel that share a word of the value tile meet in one lane
+// and only the words cross lanes (through LDS, to leave in 16-byte stores); a group of 8 L channels is
+// L lanes.  Tokens past n_q and chunks past the context are zeros.  The other workgroups copy the
+// exact rows, 16 bytes a thread: slot i holds token n_q + i, or with a ring the token n_q + j at
+// (n_q + j) % cap_e; slots without one are zeros.
+template <int DT, int L, int CH>
+__global__ __launch_bounds__(256) void kivi_compress_values(
+    const void* __restrict__ x, const void* __restrict__ kx, int H, int64_t sb, int64_t sh, int64_t st, int64_t k_sb,
+    int64_t k_sh, int64_t k_st, int64_t n_q, int window, int64_t n_chunks, uint8_t* __restrict__ vc,
+    uint16_t* __restrict__ vmeta, int64_t items_bh, int64_t n_items, unsigned item_blocks, u32x4* __restrict__ k_exact,
+    u32x4* __restrict__ v_exact, int64_t cap_e, int ring, int64_t exact_units) {
+  constexpr int D = 128, ES = DT == KVQ_F32 ? 4 : 2, NL = ES / 2, NG = D / (8 * L), UR = D * ES / 16;
+  __shared__ uint32_t image[4][kVImage];
+  if (blockIdx.x >= item_blocks) {
+    int64_t u = static_cast<int64_t>(blockIdx.x - item_blocks) * 256 + threadIdx.x;
+    if (u >= 2 * exact_units) return;
+    const bool val = u >= exact_units;
+    u -= val ? exact_units : 0;
+    const int64_t row = u / UR, bh = row / cap_e, slot = row - bh * cap_e, b = bh / H, h = bh - b * H;
+    const int c = static_cast<int>(u - row * UR);
+    int64_t i = slot;
+    if (ring) {
+      i = slot - n_q % cap_e;
+      i += i < 0 ? cap_e : 0;
+    }
+    u32x4 w = {0, 0, 0, 0};
+    if (i < window) {
+      const char* src = static_cast<const char*>(val ? x : kx);
+      const int64_t e = val ? b * sb + h * sh + (n_q + i) * st : b * k_sb + h * k_sh + (n_q + i) * k_st;
+      w = *reinterpret_cast<const u32x4*>(src + e * ES + 16 * c);
+    }
+    (val ? v_exact : k_exact)[u] = w;
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+  if (item >= n_items) return;
+  const int s = lane & 15, g = lane >> 4;
+  const int64_t bh = item / items_bh, chunk0 = (item - bh * items_bh) * CH, t0 = chunk0 * 32;
+  const int64_t b = bh / H, h = bh - b * H;
+  const int rv = static_cast<int>(max(static_cast<int64_t>(0), min(static_cast<int64_t>(32 * CH), n_q - t0)));
+  const char* src = static_cast<const char*>(x) + (b * sb + h * sh + (rv > 0 ? t0 : 0) * st) * ES;
+  const uint32_t rstride = static_cast<uint32_t>(st * ES);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, static_cast<uint32_t>(rv) * rstride);
+  u32x4 raw[CH][8 * NL];                            // rows read once: non-temporal loads; past n_q: zeros
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < NL; ++e)
+        raw[c][j * NL + e] = __builtin_amdgcn_raw_buffer_load_b128(
+            rs, (32 * c + 16 * (j >> 2) + 4 * g + (j & 3)) * rstride + s * 8 * ES + 16 * e, 0, 2);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    if (chunk0 + c >= n_chunks) return;
+    uint32_t word[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    u32x4 meta[2];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bool ok = 32 * c + 16 * (j >> 2) + 4 * g + (j & 3) < rv;
+      float v[8], mn = INFINITY, mx = -INFINITY;
+      if constexpr (DT == KVQ_F32) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = __uint_as_float(raw[c][j * NL + k / 4][k % 4]);
+      } else {
+        cvt_slab<DT>(raw[c][j], v);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        mn = fminf(mn, v[k]);
+        mx = fmaxf(mx, v[k]);
+      }
+      run_minmax<L>(mn, mx);
+      const float l1 = as_stored(mn);
+      const float s1 = fmaxf(as_stored(__fdiv_rn(__fsub_rn(mx, l1), 15.0f)), kMinScale);
+      float t[8];
+      codes4(v, l1, s1, __builtin_amdgcn_rcpf(s1), t);
+      // nibble (j & 1) 4 + j / 2 holds slot j (kSlotOfNibble's inverse)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) word[k] |= (ok ? static_cast<uint32_t>(t[k]) : 0u) << (16 * (j & 1) + 4 * (j >> 1));
+      meta[j >> 2][j & 3] = ok ? f32_to_f16(s1) | (static_cast<uint32_t>(f32_to_f16(l1)) << 16) : 0u;
+    }
+    const int64_t ck = bh * n_chunks + chunk0 + c;
+    if (s % L == 0) {
+      u32x4* m = reinterpret_cast<u32x4*>(vmeta + (ck * NG + s / L) * 64 + 16 * g);
+      m[0] = meta[0];
+      m[1] = meta[1];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      image[wave][v_image((s >> 3) * 256 + (16 * g + 8 * (s & 1) + k) * 4 + ((s >> 1) & 3))] = word[k];
+    wave_lds_fence();
+    const u32x4 o0 = *reinterpret_cast<const u32x4*>(&image[wave][v_image(4 * lane)]);
+    const u32x4 o1 = *reinterpret_cast<const u32x4*>(&image[wave][v_image(256 + 4 * lane)]);
+    u32x4* dst = reinterpret_cast<u32x4*>(vc + ck * (16 * D));
+    __builtin_nontemporal_store(o0, dst + lane);                                                // written once
+    __builtin_nontemporal_store(o1, dst + 64 + lane);
+    wave_lds_fence();                               // read before the next chunk's words are written
   }
 }
 
@@ -922,6 +1180,69 @@ extern "C" int kvq_kivi_quant(const void* x, int x_dtype, int64_t B, int64_t H, 
                                                    scale, meta_bh, xhat, (int)T));
   }
   KVQ_LAUNCH_CHECK("kvq_kivi_quant");
+  return KVQ_OK;
+}
+
+extern "C" int kvq_kivi_compress(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb,
+                                 int64_t v_sh, int64_t v_st, int dtype, int64_t B, int64_t H, int64_t T, int64_t d,
+                                 int64_t window, int group_k, int group_v, int64_t cap_t, uint8_t* kc, uint16_t* k_lo,
+                                 uint16_t* k_sc, uint8_t* vc, uint16_t* vmeta, void* k_exact, void* v_exact,
+                                 int64_t cap_e, int ring, void* stream) {
+  KVQ_REQUIRE(k && v && kc && k_lo && k_sc && vc && vmeta && k_exact && v_exact, "kvq_kivi_compress: null pointer");
+  KVQ_REQUIRE(valid_dtype(dtype) && d == 128, "kvq_kivi_compress: need d = 128 and fp32, fp16 or bf16 rows");
+  KVQ_REQUIRE((group_k == 32 || group_k == 64 || group_k == 128) && (group_v == 32 || group_v == 64 || group_v == 128),
+              "kvq_kivi_compress: groups must be 32, 64 or 128");
+  KVQ_REQUIRE(B >= 0 && H > 0 && B * H < (1LL << 24) && T >= 0 && T < (1LL << 31) && window >= 0 && window <= T,
+              "kvq_kivi_compress: bad sizes");
+  const int64_t n_q = T - window;
+  KVQ_REQUIRE(cap_t > 0 && cap_t < (1LL << 31) && cap_t % 32 == 0 && cap_t % group_k == 0 && cap_t >= n_q,
+              "kvq_kivi_compress: the capacity must hold the packed rows in whole groups and tiles");
+  KVQ_REQUIRE(cap_e > 0 && (ring ? cap_e == window : cap_e >= window) && cap_e < (1LL << 31),
+              "kvq_kivi_compress: the exact rows do not fit");
+  const int es = dtype == KVQ_F32 ? 4 : 2;
+  for (const int64_t st : {k_st, v_st})             // a row item is addressed with 32-bit byte offsets
+    KVQ_REQUIRE(st >= d && st * es * 128 < (1LL << 31), "kvq_kivi_compress: bad token stride");
+  for (const int64_t st : {k_sb, k_sh, k_st, v_sb, v_sh, v_st})
+    KVQ_REQUIRE(st * es % 16 == 0, "kvq_kivi_compress: strides must be multiples of 16 bytes");
+  for (const void* p : {k, v, static_cast<const void*>(kc), static_cast<const void*>(k_lo), static_cast<const void*>(k_sc),
+                        static_cast<const void*>(vc), static_cast<const void*>(vmeta),
+                        static_cast<const void*>(k_exact), static_cast<const void*>(v_exact)})
+    KVQ_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "kvq_kivi_compress: pointers must be 16-byte aligned");
+  if (B == 0) return KVQ_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int cap_g = static_cast<int>(cap_t / group_k), n_gq = static_cast<int>((n_q + group_k - 1) / group_k);
+  const int64_t k_items = B * H * cap_g;
+  // a lane holds RPL rows of 8 channels: 8 of fp32 or 16 of 16 bits are 64 registers
+#define KVQ_COMPRESS_KEYS(RPL_, WPI_)                                                                                \
+  hipLaunchKernelGGL((kivi_compress_keys<DT_, RPL_, WPI_>), dim3(static_cast<unsigned>((k_items * WPI_ + 3) / 4)), dim3(256), 0, \
+                     s, k, (int)H, k_sb, k_sh, k_st, (int)T, n_gq, cap_g, kc, k_lo, k_sc, k_items)
+  KVQ_REQUIRE(k_items < (1LL << 31), "kvq_kivi_compress: too many key groups");
+  KVQ_DISPATCH_DTYPE(dtype, if constexpr (DT_ == KVQ_F32) {
+    if (group_k == 32) KVQ_COMPRESS_KEYS(8, 1);
+    else if (group_k == 64) KVQ_COMPRESS_KEYS(8, 2);
+    else KVQ_COMPRESS_KEYS(8, 4);
+  } else {
+    if (group_k == 32) KVQ_COMPRESS_KEYS(8, 1);
+    else if (group_k == 64) KVQ_COMPRESS_KEYS(16, 1);
+    else KVQ_COMPRESS_KEYS(16, 2);
+  });
+#undef KVQ_COMPRESS_KEYS
+  KVQ_LAUNCH_CHECK("kvq_kivi_compress(keys)");
+  const int64_t n_chunks = cap_t / 32, exact_units = B * H * cap_e * (d * es / 16);
+#define KVQ_COMPRESS_VALUES(L_)                                                                                      \
+  KVQ_DISPATCH_DTYPE(dtype, constexpr int CH_ = DT_ == KVQ_F32 ? 1 : 2;                                              \
+    const int64_t items_bh = (n_chunks + CH_ - 1) / CH_; const int64_t items = B * H * items_bh;                     \
+    const int64_t ib = (items + 3) / 4; const int64_t eb = (2 * exact_units + 255) / 256;                            \
+    KVQ_REQUIRE(ib + eb < (1LL << 31), "kvq_kivi_compress: too many value rows");                                    \
+    hipLaunchKernelGGL((kivi_compress_values<DT_, L_, CH_>), dim3(static_cast<unsigned>(ib + eb)), dim3(256), 0, s,  \
+                       v, k, (int)H, v_sb, v_sh, v_st, k_sb, k_sh, k_st, n_q, (int)window, n_chunks, vc, vmeta, items_bh, \
+                       items, static_cast<unsigned>(ib), static_cast<u32x4*>(k_exact), static_cast<u32x4*>(v_exact), cap_e, \
+                       ring, exact_units))
+  if (group_v == 32) { KVQ_COMPRESS_VALUES(4); }
+  else if (group_v == 64) { KVQ_COMPRESS_VALUES(8); }
+  else { KVQ_COMPRESS_VALUES(16); }
+#undef KVQ_COMPRESS_VALUES
+  KVQ_LAUNCH_CHECK("kvq_kivi_compress(values)");
   return KVQ_OK;
 }
 

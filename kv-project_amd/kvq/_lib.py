@@ -28,6 +28,8 @@ SIGNATURES = {
     "kvq_abi_version": (i32, []),
     "kvq_kivi_quant": (i32, [vp, i32, i64, i64, i64, i64, i64, i64, i64, i32, i32, i32, i32,
                              vp, i64, vp, i64, vp, vp, i64, vp, vp]),
+    "kvq_kivi_compress": (i32, [vp, i64, i64, i64, vp, i64, i64, i64, i32, i64, i64, i64, i64, i64, i32, i32, i64,
+                                vp, vp, vp, vp, vp, vp, vp, i64, i32, vp]),
     "kvq_pack_codes": (i32, [vp, i64, i32, vp, vp]),
     "kvq_unpack_codes": (i32, [vp, i64, i32, vp, vp]),
     "kvq_unpack_rows_lut": (i32, [vp, i64, i32, vp, vp, vp]),

@@ -24,6 +24,23 @@ def _round_up(x: int, m: int) -> int:
     return -(-x // m) * m
 
 
+def _compress_takes(K: torch.Tensor, V: torch.Tensor, group_k: int, group_v: int, cap_t: int) -> bool:
+    """Whether kvq_kivi_compress takes this context: head_dim 128, groups of 32, 64 or 128, K and V alike, rows
+    of 16-byte pieces that do not overlap.  Every other form is quantised, packed and tiled in separate steps."""
+    if (K.shape != V.shape or K.dtype != V.dtype or K.dtype not in _lib.DTYPE_CODE or K.shape[3] != 128 or K.numel() == 0
+            or group_k not in (32, 64, 128) or group_v not in (32, 64, 128)):
+        return False
+    B, H, T, d = K.shape
+    if B * H >= 1 << 24 or cap_t >= 1 << 31 or B * H * (cap_t // 32) >= 1 << 30:
+        return False
+    es = K.element_size()
+    for x in (K, V):
+        if (x.stride(3) != 1 or x.data_ptr() % 16 or any(s * es % 16 for s in x.stride()[:3])
+                or not d <= x.stride(2) < (1 << 31) // (128 * es)):
+            return False
+    return True
+
+
 @dataclass
 class PackedKIVICache:
     kc: torch.Tensor            # (B, Hkv, cap_t, d/2) uint8
@@ -70,6 +87,19 @@ class PackedKIVICache:
         dtype = dtype or K.dtype
         dev = K.device
         cap_t = max(_round_up(max(n_q + extra_tokens, 1), math.lcm(group_k, 32)), math.lcm(group_k, 32))
+        if ring and (window < group_k or window == 0):
+            raise ValueError("the streaming window must hold at least one key group")
+        cap_e = window if ring else max(window + extra_exact, 1)
+        if dtype == K.dtype and _compress_takes(K, V, group_k, group_v, cap_t):
+            new = lambda *s, dt=torch.float16: torch.empty((B, H, *s), dtype=dt, device=dev)
+            kc, k_lo = new(cap_t, d // 2, dt=torch.uint8), new(cap_t // group_k, d)
+            vc, vmeta = new(cap_t // 32, 16 * d, dt=torch.uint8), new(cap_t // 32, d // group_v, 32, 2)
+            k_sc, k_ex, v_ex = torch.empty_like(k_lo), new(cap_e, d, dt=dtype), new(cap_e, d, dt=dtype)
+            _lib.call("kvq_kivi_compress", K.data_ptr(), *K.stride()[:3], V.data_ptr(), *V.stride()[:3],
+                      _lib.DTYPE_CODE[dtype], B, H, T, d, window, group_k, group_v, cap_t, kc.data_ptr(), k_lo.data_ptr(),
+                      k_sc.data_ptr(), vc.data_ptr(), vmeta.data_ptr(), k_ex.data_ptr(), v_ex.data_ptr(), cap_e,
+                      int(ring), _lib.stream_of(K))
+            return cls(kc, k_lo, k_sc, vc, vmeta, n_q, group_k, group_v, k_ex, v_ex, window, ring=ring, next_pos=T)
         kq = kivi_quant_stored(K, bits, group_k, True, 0)
         vq = kivi_quant_stored(V, bits, group_v, False, 0)
         kc = torch.zeros((B, H, cap_t, d // 2), dtype=torch.uint8, device=dev)
@@ -85,9 +115,6 @@ class PackedKIVICache:
         k_sc[:, :, :n_gq] = kq["scale"][:, :, :n_gq]
         vc = v_tile(vq["packed"][:, :, :n_q].contiguous(), cap_t)
         vmeta = vmeta_tile(vq["lo"][:, :, :n_q].contiguous(), vq["scale"][:, :, :n_q].contiguous(), cap_t)
-        cap_e = window if ring else max(window + extra_exact, 1)
-        if ring and (window < group_k or window == 0):
-            raise ValueError("the streaming window must hold at least one key group")
         k_ex = torch.zeros((B, H, cap_e, d), dtype=dtype, device=dev)
         v_ex = torch.zeros_like(k_ex)
         slots = (torch.arange(n_q, T, device=dev) % cap_e) if ring else torch.arange(window, device=dev)
