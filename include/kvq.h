@@ -433,6 +433,15 @@ int kvq_mixed_decode(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int
 int kvq_dct_encode(const void* x, int x_dtype, int64_t BH, int64_t T, int64_t d, int64_t x_bh,
                    const float* ctab, int for_values, uint8_t* codes, uint16_t* scales, void* stream);
 
+/* A whole context into the DCT cache: k, v (B, H, T, 128) of one dtype with element strides, channels
+ * contiguous.  Rows [0, n_coded) (n_coded % 64 == 0) are coded as kvq_dct_encode codes them (kc, ks keys,
+ * vc, vs values); rows [n_coded, T) go to slots 0 .. of k_exact / v_exact (BH, cap_e, 128), the other
+ * slots are zeroed.  Pointers and strides (in bytes) multiples of 16. */
+int kvq_dct_compress(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb,
+                     int64_t v_sh, int64_t v_st, int dtype, int64_t B, int64_t H, int64_t T, int64_t d,
+                     int64_t n_coded, const float* ctab, uint8_t* kc, uint16_t* ks, uint8_t* vc, uint16_t* vs,
+                     void* k_exact, void* v_exact, int64_t cap_e, void* stream);
+
 /* Decode over a DCT-coded context of T tokens (T % 64 == 0, kc/ks key blocks, vc/vs value blocks,
  * each (B*Hkv, T/64, ...)) plus n_exact exact rows (as kvq_kivi_decode's exact rows, dtype =
  * q_dtype): attention over the reconstructions x_n = sum_k C[k][n] s_k (code_k - 7), computed in

@@ -121,6 +121,37 @@ __device__ __forceinline__ float sqrt_rn(float x) {
   return small ? y * 0x1p-16f : y;
 }
 
+// Exact rows of a compressed context, copied by the workgroups a compression kernel does not need for
+// its codes: slot i of a (b, h) takes row first + i, or with a ring the row first + j at slot
+// (first + j) % cap; slots past `count` rows are zeros.  A thread moves 16 bytes; strides in bytes.
+struct ExactSide {
+  const char* src;
+  int64_t sb, sh, st;
+  uint4* dst;                       // (BH, cap, row)
+};
+struct ExactRows {
+  ExactSide k, v;
+  int H, row_units, ring;           // 16-byte units per row
+  int64_t first, count, cap, units; // units per side = BH cap row_units
+};
+
+__device__ __forceinline__ void copy_exact_unit(const ExactRows& p, int64_t u) {
+  const bool keys = u < p.units;
+  u -= keys ? 0 : p.units;
+  if (u >= p.units) return;
+  const int64_t row = u / p.row_units, bh = row / p.cap, slot = row - bh * p.cap, b = bh / p.H, h = bh - b * p.H;
+  int64_t i = slot;
+  if (p.ring) {
+    i = slot - p.first % p.cap;
+    i += i < 0 ? p.cap : 0;
+  }
+  const char* src = keys ? p.k.src + b * p.k.sb + h * p.k.sh + (p.first + i) * p.k.st
+                         : p.v.src + b * p.v.sb + h * p.v.sh + (p.first + i) * p.v.st;
+  uint4 w = {0, 0, 0, 0};
+  if (i < p.count) w = *reinterpret_cast<const uint4*>(src + 16 * (u - row * p.row_units));
+  (keys ? p.k.dst : p.v.dst)[u] = w;
+}
+
 inline bool valid_dtype(int dt) { return dt == KVQ_F32 || dt == KVQ_F16 || dt == KVQ_BF16; }
 
 }  // namespace kvq

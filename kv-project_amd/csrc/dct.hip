@@ -46,10 +46,11 @@ __device__ __forceinline__ float as_stored_h(float x) {
 
 __device__ __constant__ int kNibOfElem[8] = {0, 4, 1, 5, 2, 6, 3, 7};
 
-// one thread per (b, h, block, channel)
+// one thread per (b, h, block, channel): fp32 rows, and 16-bit rows that are not 16-byte aligned.  Bound by
+// its 32 instructions an element (a product and a sum for each of the 16 coefficients, in the fixed order).
 template <int DT>
-__global__ __launch_bounds__(256) void dct_encode_kernel(const void* __restrict__ x, int64_t T, int64_t x_bh,
-                                                         const float* __restrict__ ctab, int for_values,
+__global__ __launch_bounds__(256) void dct_encode_kernel(const void* __restrict__ x, int64_t T, int H, int64_t sb,
+                                                         int64_t sh, int64_t st, const float* __restrict__ ctab, int for_values,
                                                          uint8_t* __restrict__ codes, uint16_t* __restrict__ scales,
                                                          int64_t total) {
   const int64_t id = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -58,12 +59,12 @@ __global__ __launch_bounds__(256) void dct_encode_kernel(const void* __restrict_
   const int64_t blk_all = id / kDD;                // (bh, block)
   const int64_t nb = T / kDB;
   const int64_t bh = blk_all / nb, blk = blk_all % nb;
-  const int64_t base = bh * x_bh + blk * kDB * kDD + c;
+  const int64_t base = bh / H * sb + bh % H * sh + blk * kDB * st + c;
   float X[kDK];
 #pragma unroll
   for (int k = 0; k < kDK; ++k) X[k] = 0.0f;
   for (int n = 0; n < kDB; ++n) {
-    const float xv = load_as_f32<DT>(x, base + static_cast<int64_t>(n) * kDD);
+    const float xv = load_as_f32<DT>(x, base + static_cast<int64_t>(n) * st);
 #pragma unroll
     for (int k = 0; k < kDK; ++k) X[k] = __fadd_rn(X[k], __fmul_rn(ctab[k * kDB + n], xv));
   }
@@ -98,6 +99,303 @@ __global__ __launch_bounds__(256) void dct_encode_kernel(const void* __restrict_
 #pragma unroll
       for (int e = 0; e < 8; ++e) w |= static_cast<uint32_t>(q[8 * gp + e]) << (4 * kNibOfElem[e]);
       words[(gp * 16 + n) * 8 + b8] = w;
+    }
+  }
+}
+
+
+// 16-bit rows, both sides and the exact rows in one launch.  Bound by memory where the kernel above is bound
+// by its vector instructions: the coefficients come from the matrix cores, and the codes and scales still
+// are those of the fixed order, because what a rounding there could change is found and recomputed in it.
+//
+// A wavefront walks (b, h, block) items, the next item's rows loaded while the current one is coded.  Lane
+// (g, n) loads channels 8n .. 8n+7 of tokens 32 ks + 4 j + g (a load instruction reads four whole rows);
+// byte permutes turn each channel's eight tokens into the B operand of its product, whose column n is
+// channel 8n + e: F[e] = C x[8n + e], eight products a k-step.  C is the sum of three 16-bit parts (24 bits:
+// exact; fp16 parts of 2^12 C), so every product is exact in fp32.  The small parts are summed first.
+//   |F - X| <= err = 8.05e-6 max|C| sum|x|:  the fixed order rounds 64 products and 63 sums, each by at most
+// 2^-24 sum|C x|; the matrix core's 32 additions of the leading part to either half's sum are taken to lose
+// at most 2^-23 of that half's sum|C x| each (truncation included), those of the small parts 2^-8 of
+// that, and the halves' addition 2^-24: 3.9e-6 + 3.9e-6 + 0.1e-6 + 0.1e-6.  sum|x| is one more product,
+// of ones with |x|.
+// The scale fp16(max|X| / 7) is settled where both ends of max|F| -+ err give it; else the coefficients
+// within 2 err of the maximum are summed again in the fixed order.  A code is settled where F / s is
+// further than err / s from a half-integer; else its coefficient is summed again, from the rows in LDS.  On
+// AR(1) rows (rho 0.95) about 4% of the channels repeat one coefficient's sum.
+// 2 x 8 x 131072 bf16 rows (0.58 GB) with 64 exact rows behind them: 137 us, 4.2 TB/s; 108 us without the
+// repeats.  The kernel above took 222 us, with the copies of the sliced rows and the fills 403 us.
+struct DctSide {
+  const uint16_t* src;
+  int64_t sb, sh, st;               // element strides
+  uint8_t* codes;
+  uint16_t* scales;
+};
+struct DctEncode {
+  DctSide k, v;
+  int H, nb, n_keys, n_items;       // blocks per (b, h), items of the keys, items of both sides
+  const float* ctab;
+  unsigned copy_blocks;             // leading workgroups that copy the exact rows
+};
+
+constexpr int kCtabStride = 68;     // LDS row stride of the table: rows start in different banks
+
+// x / 7 rounded to nearest even, x >= 0: the quotient by the rounded reciprocal, corrected once by its exact
+// remainder (Markstein, "IA-64 and Elementary Functions", 2000, theorem 8.5); tiny quotients, whose
+// remainder would be subnormal, only ever meet the scale's floor.
+__device__ __forceinline__ float div7(float x) {
+  const float q = x * 0x1.24924ap-3f;
+  const float c = __builtin_fmaf(__builtin_fmaf(-7.0f, q, x), 0x1.24924ap-3f, q);
+  return x < INFINITY ? c : x;
+}
+
+template <int DT>
+__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (DT == KVQ_F16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(a), as_half8(b), c, 0, 0, 0);
+  } else {
+    typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256, 2) void dct_encode_mfma(DctEncode p, ExactRows exact) {
+  if (blockIdx.x < p.copy_blocks) {
+    copy_exact_unit(exact, static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x);
+    return;
+  }
+  __shared__ float tab[kDK * kCtabStride];
+  __shared__ u32x4 all_rows[4][kDB][16];                          // each wavefront's current item
+  u32x4 (*rows)[16] = all_rows[threadIdx.x >> 6];
+  for (int i = threadIdx.x; i < kDK * kDB; i += 256) tab[(i / kDB) * kCtabStride + i % kDB] = p.ctab[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+  const int stride = static_cast<int>(gridDim.x - p.copy_blocks) * 4;
+  int item = static_cast<int>(blockIdx.x - p.copy_blocks) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr float kUp = DT == KVQ_F16 ? 4096.0f : 1.0f;         // fp16 parts of C are taken of 2^12 C
+  // A operands: row n of part `part` of C at tokens 32 ks + 4 j + g, j = 0 .. 7
+  u32x4 ca[3][2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      uint32_t w[3] = {0, 0, 0};
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        float c = tab[n * kCtabStride + 32 * ks + 4 * (2 * d + o) + g] * kUp;
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+          const uint16_t h = DT == KVQ_F16 ? f32_to_f16(c) : f32_to_bf16(c);
+          c -= DT == KVQ_F16 ? f16_to_f32(h) : bf16_to_f32(h);
+          w[part] |= static_cast<uint32_t>(h) << (16 * o);
+        }
+      }
+#pragma unroll
+      for (int part = 0; part < 3; ++part) ca[part][ks][d] = w[part];
+    }
+  }
+  const uint32_t one = DT == KVQ_F16 ? 0x3c003c00u : 0x3f803f80u;
+  const u32x4 ones = {one, one, one, one};
+
+  u32x4 raw[16];
+  auto load = [&](int item) {                                   // the item's rows, through one buffer resource
+    const bool keys = item < p.n_keys;
+    const DctSide& x = keys ? p.k : p.v;
+    const int i = keys ? item : item - p.n_keys, bh = i / p.nb, blk = i - bh * p.nb, b = bh / p.H;
+    const uint32_t rstride = static_cast<uint32_t>(x.st * 2), at = g * rstride + 16 * n;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(x.src + b * x.sb + (bh - b * p.H) * x.sh + static_cast<int64_t>(blk) * kDB * x.st,
+                                                (kDB - 1) * rstride + kDD * 2);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) raw[r] = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 4 * r * rstride, 2);   // read once
+  };
+  if (item < p.n_items) load(item);
+  for (; item < p.n_items; item += stride) {
+    float F[8][4], err[8];                                       // coefficients 4g + i of channels 8n + e
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        const uint32_t sel = o ? 0x07060302u : 0x05040100u;
+        u32x4 xb[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            xb[ks][j] = __builtin_amdgcn_perm(raw[8 * ks + 2 * j + 1][d], raw[8 * ks + 2 * j][d], sel);
+        f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}}, tot = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int part = 2; part >= 0; --part)
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) acc[ks] = mfma16<DT>(ca[part][ks], xb[ks], acc[ks]);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          u32x4 ab;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) ab[j] = xb[ks][j] & 0x7fff7fffu;
+          tot = mfma16<DT>(ones, ab, tot);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) F[2 * d + o][i] = (acc[0][i] + acc[1][i]) * (1.0f / kUp);
+        err[2 * d + o] = tot[0] * 1.43e-6f;                      // 8.05e-6 sqrt(2) / 8, rounded up
+      }
+    }
+    // the rows stay in LDS for the sums that are repeated (their latency there is what a repeat costs: read again
+    // from memory behind the next item's rows, the repeats took 210 us)
+    wave_lds_fence();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) rows[4 * r + g][n] = raw[r];
+    wave_lds_fence();
+    if (item + stride < p.n_items) load(item + stride);
+
+    // use(bit, X) with X the coefficient 4g + i of channel 8n + e in the fixed order, for every set bit 4e + i
+    auto resum = [&](uint32_t need, auto use) {
+      while (__any(need != 0)) {
+        const int bit = need ? __builtin_ctz(need) : 0;
+        const uint16_t* col = reinterpret_cast<const uint16_t*>(&rows[0][n]) + (bit >> 2);
+        const float* crow = tab + (4 * g + (bit & 3)) * kCtabStride;
+        float X = 0.0f;
+#pragma unroll 2
+        for (int t0 = 0; t0 < kDB; t0 += 16) {
+          uint32_t xw[16];
+#pragma unroll
+          for (int t = 0; t < 16; ++t) xw[t] = col[(t0 + t) * kDD];
+#pragma unroll
+          for (int t = 0; t < 16; ++t)
+            X = __fadd_rn(X, __fmul_rn(crow[t0 + t], DT == KVQ_F16 ? f16_to_f32(xw[t]) : __uint_as_float(xw[t] << 16)));
+        }
+        if (need != 0) use(bit, X);
+        need &= need - 1;
+      }
+    };
+    float amax[8], s[8];
+    uint32_t open = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float m = fmaxf(fmaxf(fmaxf(fabsf(F[e][0]), fabsf(F[e][1])), fabsf(F[e][2])), fabsf(F[e][3]));
+      amax[e] = xmax32(xmax16(fmaxf(m, 0.0f)));
+      // both ends of max|X| / 7 as fp16, the factors 2^-21 to either side of 1 / 7; values that the clamps of
+      // the scale or the codes could touch, infinities and NaN count as open
+      const uint16_t lo = f32_to_f16((amax[e] - err[e]) * 0x1.249240p-3f), hi = f32_to_f16((amax[e] + err[e]) * 0x1.249252p-3f);
+      s[e] = fmaxf(f16_to_f32(lo), 0x1p-24f);
+      if (lo != hi || !(amax[e] + err[e] < 4e5f)) open |= 1u << e;
+    }
+    if (__any(open != 0)) {
+      uint32_t need = 0;
+      float top[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        top[e] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (((open >> e) & 1) && !(fabsf(F[e][i]) < amax[e] - 2.0f * err[e])) need |= 1u << (4 * e + i);
+      }
+      resum(need, [&](int bit, float X) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) top[e] = fmaxf(top[e], bit >> 2 == e ? fabsf(X) : 0.0f);
+      });
+      bool wild = false;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float exact = fmaxf(as_stored_h(div7(xmax32(xmax16(top[e])))), 0x1p-24f);
+        s[e] = ((open >> e) & 1) ? exact : s[e];
+        wild |= !(amax[e] + err[e] < 4e5f);
+      }
+      if (__any(wild)) {                                          // such a channel's codes all come from the fixed order
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bool w = !(amax[e] + err[e] < 4e5f);
+          err[e] = w ? INFINITY : err[e];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) F[e][i] = w ? 0.0f : F[e][i];
+        }
+      }
+    }
+    // Codes: |F / s| <= 7.01 where s is a normal fp16 value, at most 10.5 below (the clamp acts only there),
+    // so F r is within 4e-6 of F / s.  t + 7 is a nibble; four of them sum exactly to the halves of a word.
+    float most[8], r[8], t[8][4];
+    bool unsettled = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      r[e] = __builtin_amdgcn_rcpf(s[e]);
+      most[e] = __builtin_fmaf(-1.01f * err[e], r[e], 0.499996f);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float q = F[e][i] * r[e];
+        t[e][i] = rintf(q);
+        unsettled |= !(fabsf(q - t[e][i]) < most[e]);
+      }
+    }
+    float least = amax[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) least = fminf(least, amax[e]);
+    if (__any(!(least > 7.1f * 0x1p-14f))) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t[e][i] = fminf(fmaxf(t[e][i], -7.0f), 7.0f);
+    }
+    const bool keys = item < p.n_keys;
+    uint32_t word[8];
+    auto halves = [](float lo, float hi) {
+      return static_cast<uint32_t>(static_cast<int>(lo)) | (static_cast<uint32_t>(static_cast<int>(hi)) << 16);
+    };
+    if (keys) {                                                   // word i: coefficient 4g + i of channels 8n ..
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        word[i] = halves(fmaf(t[6][i], 4096.0f, fmaf(t[4][i], 256.0f, fmaf(t[2][i], 16.0f, t[0][i] + 30583.0f))),
+                         fmaf(t[7][i], 4096.0f, fmaf(t[5][i], 256.0f, fmaf(t[3][i], 16.0f, t[1][i] + 30583.0f))));
+    } else {                                                      // word e: channel 8n + e, half of its coefficients
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        word[e] = halves(fmaf(t[e][2], 16.0f, t[e][0] + 119.0f), fmaf(t[e][3], 16.0f, t[e][1] + 119.0f)) << (8 * (g & 1));
+    }
+    if (__any(unsettled)) {
+      uint32_t need = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float q = F[e][i] * r[e];
+          if (!(fabsf(q - rintf(q)) < most[e])) need |= 1u << (4 * e + i);
+        }
+      resum(need, [&](int bit, float X) {
+        const int e = bit >> 2, i = bit & 3;
+        uint32_t sc = 0;                                          // s[e]
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sc |= e == k ? __float_as_uint(s[k]) : 0u;
+        const uint32_t c = static_cast<uint32_t>(static_cast<int>(fminf(fmaxf(rintf(__fdiv_rn(X, __uint_as_float(sc))), -7.0f), 7.0f)) + 7);
+        const int w = keys ? i : e, sh = keys ? 16 * (e & 1) + 4 * (e >> 1) : 16 * (i & 1) + 4 * (i >> 1) + 8 * (g & 1);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (w == k) word[k] = (word[k] & ~(15u << sh)) | (c << sh);
+      });
+    }
+    const int64_t blk = keys ? item : item - p.n_keys;
+    uint32_t* words = reinterpret_cast<uint32_t*>((keys ? p.k.codes : p.v.codes) + blk * 1024);
+    uint16_t* sc = (keys ? p.k.scales : p.v.scales) + blk * kDD;
+    if (keys) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) words[(4 * g + i) * 16 + n] = word[i];
+      if (g == 0) {
+        u32x4 w;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) w[d] = f32_to_f16(s[2 * d]) | (static_cast<uint32_t>(f32_to_f16(s[2 * d + 1])) << 16);
+        *reinterpret_cast<u32x4*>(sc + 8 * n) = w;
+      }
+    } else {
+      // lane groups 2 gp and 2 gp + 1 hold the two halves of a word's coefficients; each stores four of the words
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const auto x = __builtin_amdgcn_permlane16_swap(word[e], word[e], false, false);
+        word[e] = x[0] | x[1];
+      }
+      const uint32_t odd = (g & 1) ? ~0u : 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        words[((g >> 1) * 16 + 8 * (n & 1) + 4 * (g & 1) + e) * 8 + (n >> 1)] = (word[e] & ~odd) | (word[4 + e] & odd);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e >> 1 == g) sc[(8 * (n & 1) + e) * 8 + (n >> 1)] = f32_to_f16(s[e]);
     }
   }
 }
@@ -886,19 +1184,99 @@ constexpr size_t kPairSmem = (kDWaves * 8 * kDD + kDWaves * 8 * 2 + kDWaves * kP
 
 using namespace kvq;
 
+namespace {
+// rows the matrix-core encoder takes: 16 bits, 16-byte pieces that do not overlap, 32-bit offsets in a block
+bool dct_rows_fast(const void* x, int dt, int64_t sb, int64_t sh, int64_t st) {
+  return dt != KVQ_F32 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && sb % 8 == 0 && sh % 8 == 0 && st % 8 == 0 &&
+         st >= kDD && st < (1LL << 23);
+}
+// a persistent grid: two workgroups (eight wavefronts) a CU
+constexpr int64_t kDctEncodeGrid = 512;
+
+int dct_encode_fast(kvq::DctEncode p, const kvq::ExactRows& exact, int dt, hipStream_t s) {
+  const int64_t copy = (2 * exact.units + 255) / 256;
+  const int64_t work = std::min<int64_t>((p.n_items + 3) / 4, kDctEncodeGrid);
+  KVQ_REQUIRE(copy + work < (1LL << 31), "kvq_dct_encode: too large");
+  p.copy_blocks = static_cast<unsigned>(copy);
+  if (copy + work == 0) return KVQ_OK;
+  KVQ_DISPATCH_DTYPE(dt, if constexpr (DT_ != KVQ_F32) hipLaunchKernelGGL(
+      (dct_encode_mfma<DT_>), dim3(static_cast<unsigned>(copy + work)), dim3(256), 0, s, p, exact));
+  KVQ_LAUNCH_CHECK("kvq_dct_encode");
+  return KVQ_OK;
+}
+
+int dct_encode_side(const void* x, int dt, int64_t BH, int64_t nb, int64_t H, int64_t sb, int64_t sh, int64_t st,
+                    const float* ctab, int for_values, uint8_t* codes, uint16_t* scales, hipStream_t s) {
+  const int64_t total = BH * nb * kDD;
+  if (total == 0) return KVQ_OK;
+  KVQ_REQUIRE(x && ctab && codes && scales, "kvq_dct_encode: null pointer");
+  KVQ_REQUIRE(total / 256 < (1LL << 31), "kvq_dct_encode: too large");
+  if (dct_rows_fast(x, dt, sb, sh, st) && BH * nb < (1LL << 29) && (for_values || reinterpret_cast<uintptr_t>(scales) % 16 == 0)) {
+    kvq::DctEncode p = {};
+    (for_values ? p.v : p.k) = {static_cast<const uint16_t*>(x), sb, sh, st, codes, scales};
+    p.H = static_cast<int>(H);
+    p.nb = static_cast<int>(nb);
+    p.n_keys = for_values ? 0 : static_cast<int>(BH * nb);
+    p.n_items = static_cast<int>(BH * nb);
+    p.ctab = ctab;
+    return dct_encode_fast(p, kvq::ExactRows{}, dt, s);
+  }
+  KVQ_DISPATCH_DTYPE(dt, hipLaunchKernelGGL((dct_encode_kernel<DT_>), dim3(static_cast<unsigned>((total + 255) / 256)),
+                                           dim3(256), 0, s, x, nb * kDB, (int)H, sb, sh, st, ctab, for_values, codes,
+                                           scales, total));
+  KVQ_LAUNCH_CHECK("kvq_dct_encode");
+  return KVQ_OK;
+}
+
+__global__ __launch_bounds__(256) void dct_exact_rows(kvq::ExactRows exact) {
+  kvq::copy_exact_unit(exact, static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x);
+}
+}  // namespace
+
 extern "C" int kvq_dct_encode(const void* x, int x_dtype, int64_t BH, int64_t T, int64_t d, int64_t x_bh,
                               const float* ctab, int for_values, uint8_t* codes, uint16_t* scales, void* stream) {
   KVQ_REQUIRE(valid_dtype(x_dtype), "kvq_dct_encode: bad dtype");
   KVQ_REQUIRE(d == kDD, "kvq_dct_encode: head_dim must be 128");
   KVQ_REQUIRE(BH >= 0 && T >= 0 && T % kDB == 0 && x_bh >= T * d, "kvq_dct_encode: T must be a multiple of 64");
-  const int64_t total = BH * (T / kDB) * kDD;
-  if (total == 0) return KVQ_OK;
-  KVQ_REQUIRE(x && ctab && codes && scales, "kvq_dct_encode: null pointer");
-  KVQ_REQUIRE(total / 256 < (1LL << 31), "kvq_dct_encode: too large");
+  return dct_encode_side(x, x_dtype, BH, T / kDB, 1, x_bh, 0, kDD, ctab, for_values, codes, scales,
+                         static_cast<hipStream_t>(stream));
+}
+
+extern "C" int kvq_dct_compress(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb,
+                                int64_t v_sh, int64_t v_st, int dtype, int64_t B, int64_t H, int64_t T, int64_t d,
+                                int64_t n_coded, const float* ctab, uint8_t* kc, uint16_t* ks, uint8_t* vc, uint16_t* vs,
+                                void* k_exact, void* v_exact, int64_t cap_e, void* stream) {
+  KVQ_REQUIRE(valid_dtype(dtype) && d == kDD, "kvq_dct_compress: need d = 128 and fp32, fp16 or bf16 rows");
+  KVQ_REQUIRE(B >= 0 && H > 0 && B * H < (1LL << 24) && T >= 0 && T < (1LL << 31) && n_coded >= 0 && n_coded <= T &&
+                  n_coded % kDB == 0 && cap_e >= T - n_coded && cap_e > 0 && cap_e < (1LL << 31),
+              "kvq_dct_compress: bad sizes");
+  if (B == 0) return KVQ_OK;
+  KVQ_REQUIRE(k && v && ctab && k_exact && v_exact && (n_coded == 0 || (kc && ks && vc && vs)), "kvq_dct_compress: null pointer");
+  const int es = dtype == KVQ_F32 ? 4 : 2;
+  for (const int64_t st : {k_sb, k_sh, k_st, v_sb, v_sh, v_st})
+    KVQ_REQUIRE(st >= 0 && st * es % 16 == 0, "kvq_dct_compress: strides must be multiples of 16 bytes");
+  for (const void* p : {k, v, static_cast<const void*>(k_exact), static_cast<const void*>(v_exact),
+                        static_cast<const void*>(kc), static_cast<const void*>(ks), static_cast<const void*>(vc),
+                        static_cast<const void*>(vs)})
+    KVQ_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "kvq_dct_compress: pointers must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  KVQ_DISPATCH_DTYPE(x_dtype, hipLaunchKernelGGL((dct_encode_kernel<DT_>), dim3(static_cast<unsigned>((total + 255) / 256)),
-                                                dim3(256), 0, s, x, T, x_bh, ctab, for_values, codes, scales, total));
-  KVQ_LAUNCH_CHECK("kvq_dct_encode");
+  const int row_units = static_cast<int>(d * es / 16);
+  const kvq::ExactRows exact = {{static_cast<const char*>(k), k_sb * es, k_sh * es, k_st * es, static_cast<uint4*>(k_exact)},
+      {static_cast<const char*>(v), v_sb * es, v_sh * es, v_st * es, static_cast<uint4*>(v_exact)}, static_cast<int>(H), row_units,
+      0, n_coded, T - n_coded, cap_e, B * H * cap_e * row_units};
+  const int64_t nb = n_coded / kDB;
+  if (dct_rows_fast(k, dtype, k_sb, k_sh, k_st) && dct_rows_fast(v, dtype, v_sb, v_sh, v_st) && B * H * nb < (1LL << 29)) {
+    const kvq::DctEncode p = {{static_cast<const uint16_t*>(k), k_sb, k_sh, k_st, kc, ks},
+                              {static_cast<const uint16_t*>(v), v_sb, v_sh, v_st, vc, vs},
+                              static_cast<int>(H), static_cast<int>(nb), static_cast<int>(B * H * nb),
+                              static_cast<int>(2 * B * H * nb), ctab, 0};
+    return dct_encode_fast(p, exact, dtype, s);
+  }
+  if (int rc = dct_encode_side(k, dtype, B * H, nb, H, k_sb, k_sh, k_st, ctab, 0, kc, ks, s)) return rc;
+  if (int rc = dct_encode_side(v, dtype, B * H, nb, H, v_sb, v_sh, v_st, ctab, 1, vc, vs, s)) return rc;
+  KVQ_REQUIRE((2 * exact.units + 255) / 256 < (1LL << 31), "kvq_dct_compress: too many exact rows");
+  hipLaunchKernelGGL(dct_exact_rows, dim3(static_cast<unsigned>((2 * exact.units + 255) / 256)), dim3(256), 0, s, exact);
+  KVQ_LAUNCH_CHECK("kvq_dct_compress(exact)");
   return KVQ_OK;
 }
 

@@ -824,35 +824,16 @@ constexpr int kVImage = 512 + 4 * 8;
 // four whole rows), so the eight codes of a channel that share a word of the value tile meet in one lane
 // and only the words cross lanes (through LDS, to leave in 16-byte stores); a group of 8 L channels is
 // L lanes.  Tokens past n_q and chunks past the context are zeros.  The other workgroups copy the
-// exact rows, 16 bytes a thread: slot i holds token n_q + i, or with a ring the token n_q + j at
-// (n_q + j) % cap_e; slots without one are zeros.
+// exact rows.
 template <int DT, int L, int CH>
 __global__ __launch_bounds__(256) void kivi_compress_values(
-    const void* __restrict__ x, const void* __restrict__ kx, int H, int64_t sb, int64_t sh, int64_t st, int64_t k_sb,
-    int64_t k_sh, int64_t k_st, int64_t n_q, int window, int64_t n_chunks, uint8_t* __restrict__ vc,
-    uint16_t* __restrict__ vmeta, int64_t items_bh, int64_t n_items, unsigned item_blocks, u32x4* __restrict__ k_exact,
-    u32x4* __restrict__ v_exact, int64_t cap_e, int ring, int64_t exact_units) {
-  constexpr int D = 128, ES = DT == KVQ_F32 ? 4 : 2, NL = ES / 2, NG = D / (8 * L), UR = D * ES / 16;
+    const void* __restrict__ x, int H, int64_t sb, int64_t sh, int64_t st, int64_t n_q, int64_t n_chunks,
+    uint8_t* __restrict__ vc, uint16_t* __restrict__ vmeta, int64_t items_bh, int64_t n_items, unsigned item_blocks,
+    ExactRows exact) {
+  constexpr int D = 128, ES = DT == KVQ_F32 ? 4 : 2, NL = ES / 2, NG = D / (8 * L);
   __shared__ uint32_t image[4][kVImage];
   if (blockIdx.x >= item_blocks) {
-    int64_t u = static_cast<int64_t>(blockIdx.x - item_blocks) * 256 + threadIdx.x;
-    if (u >= 2 * exact_units) return;
-    const bool val = u >= exact_units;
-    u -= val ? exact_units : 0;
-    const int64_t row = u / UR, bh = row / cap_e, slot = row - bh * cap_e, b = bh / H, h = bh - b * H;
-    const int c = static_cast<int>(u - row * UR);
-    int64_t i = slot;
-    if (ring) {
-      i = slot - n_q % cap_e;
-      i += i < 0 ? cap_e : 0;
-    }
-    u32x4 w = {0, 0, 0, 0};
-    if (i < window) {
-      const char* src = static_cast<const char*>(val ? x : kx);
-      const int64_t e = val ? b * sb + h * sh + (n_q + i) * st : b * k_sb + h * k_sh + (n_q + i) * k_st;
-      w = *reinterpret_cast<const u32x4*>(src + e * ES + 16 * c);
-    }
-    (val ? v_exact : k_exact)[u] = w;
+    copy_exact_unit(exact, static_cast<int64_t>(blockIdx.x - item_blocks) * 256 + threadIdx.x);
     return;
   }
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1086,7 +1067,7 @@ extern "C" int kvq_kivi_quant(const void* x, int x_dtype, int64_t B, int64_t H, 
                    al(scale, 16) && meta_bh % 8 == 0;
   // packed-only 4-bit output of 16-bit input: one wavefront per item (the decode cache's prefill)
   const bool p4 = vec && bits == 4 && packed != nullptr && codes == nullptr && xhat == nullptr &&
-                  x_dtype != KVQ_F32 && st < (1LL << 25);
+                  x_dtype != KVQ_F32 && st >= d && st < (1LL << 25);   // one buffer resource spans an item's rows
   if (p4 && along_tokens && group <= 64) {
     const int n_g = (n + group - 1) / group;
     const int64_t n_items = static_cast<int64_t>(n_g) * B * H;
@@ -1228,16 +1209,19 @@ extern "C" int kvq_kivi_compress(const void* k, int64_t k_sb, int64_t k_sh, int6
   });
 #undef KVQ_COMPRESS_KEYS
   KVQ_LAUNCH_CHECK("kvq_kivi_compress(keys)");
-  const int64_t n_chunks = cap_t / 32, exact_units = B * H * cap_e * (d * es / 16);
+  const int64_t n_chunks = cap_t / 32;
+  const int row_units = static_cast<int>(d * es / 16);
+  const ExactRows exact = {{static_cast<const char*>(k), k_sb * es, k_sh * es, k_st * es, static_cast<uint4*>(k_exact)},
+      {static_cast<const char*>(v), v_sb * es, v_sh * es, v_st * es, static_cast<uint4*>(v_exact)}, static_cast<int>(H), row_units,
+      ring, n_q, window, cap_e, B * H * cap_e * row_units};
 #define KVQ_COMPRESS_VALUES(L_)                                                                                      \
   KVQ_DISPATCH_DTYPE(dtype, constexpr int CH_ = DT_ == KVQ_F32 ? 1 : 2;                                              \
     const int64_t items_bh = (n_chunks + CH_ - 1) / CH_; const int64_t items = B * H * items_bh;                     \
-    const int64_t ib = (items + 3) / 4; const int64_t eb = (2 * exact_units + 255) / 256;                            \
+    const int64_t ib = (items + 3) / 4; const int64_t eb = (2 * exact.units + 255) / 256;                            \
     KVQ_REQUIRE(ib + eb < (1LL << 31), "kvq_kivi_compress: too many value rows");                                    \
     hipLaunchKernelGGL((kivi_compress_values<DT_, L_, CH_>), dim3(static_cast<unsigned>(ib + eb)), dim3(256), 0, s,  \
-                       v, k, (int)H, v_sb, v_sh, v_st, k_sb, k_sh, k_st, n_q, (int)window, n_chunks, vc, vmeta, items_bh, \
-                       items, static_cast<unsigned>(ib), static_cast<u32x4*>(k_exact), static_cast<u32x4*>(v_exact), cap_e, \
-                       ring, exact_units))
+                       v, (int)H, v_sb, v_sh, v_st, n_q, n_chunks, vc, vmeta, items_bh, items,                       \
+                       static_cast<unsigned>(ib), exact))
   if (group_v == 32) { KVQ_COMPRESS_VALUES(4); }
   else if (group_v == 64) { KVQ_COMPRESS_VALUES(8); }
   else { KVQ_COMPRESS_VALUES(16); }

@@ -67,6 +67,17 @@ def dct_encode(x: torch.Tensor, for_values: bool = False):
     return codes, scales
 
 
+def _compress_takes(K: torch.Tensor, V: torch.Tensor) -> bool:
+    """Whether kvq_dct_compress takes this context as it lies: head_dim 128, K and V alike, rows of 16-byte
+    pieces.  Every other form is copied to contiguous blocks and coded a side at a time (dct_encode)."""
+    if (K.shape != V.shape or K.dtype != V.dtype or K.dtype not in _lib.DTYPE_CODE or K.shape[3] != 128
+            or K.numel() == 0 or K.shape[0] * K.shape[1] >= 1 << 24 or K.shape[2] >= 1 << 31
+            or K.numel() // 64 >= 1 << 38):
+        return False
+    es = K.element_size()
+    return all(x.stride(3) == 1 and x.data_ptr() % 16 == 0 and not any(s * es % 16 for s in x.stride()[:3]) for x in (K, V))
+
+
 @dataclass
 class DctCache:
     """DCT-coded context of one layer: T coded tokens (whole 64-token blocks) and exact rows (the
@@ -89,10 +100,18 @@ class DctCache:
         _lib.require_gpu(K, V)
         B, H, T, d = K.shape
         nc = max(0, (T - window) // BLOCK * BLOCK)
+        cap_e = max(T - nc + extra_exact, 1)
+        if _compress_takes(K, V):
+            new = lambda *s, dt: torch.empty((B, H, *s), dtype=dt, device=K.device)
+            kc, ks = new(nc // BLOCK, 1024, dt=torch.uint8), new(nc // BLOCK, 128, dt=torch.float16)
+            vc, vs, ke, ve = torch.empty_like(kc), torch.empty_like(ks), new(cap_e, d, dt=K.dtype), new(cap_e, d, dt=K.dtype)
+            _lib.call("kvq_dct_compress", K.data_ptr(), *K.stride()[:3], V.data_ptr(), *V.stride()[:3],
+                      _lib.DTYPE_CODE[K.dtype], B, H, T, d, nc, dct_table(K.device).data_ptr(), kc.data_ptr(), ks.data_ptr(),
+                      vc.data_ptr(), vs.data_ptr(), ke.data_ptr(), ve.data_ptr(), cap_e, _lib.stream_of(K))
+            return cls(nc, kc, ks, vc, vs, ke, ve, T - nc)
         kc, ks = dct_encode(K[:, :, :nc])
         vc, vs = dct_encode(V[:, :, :nc], for_values=True)
         ne = T - nc
-        cap_e = max(ne + extra_exact, 1)
         ke = torch.zeros((B, H, cap_e, d), dtype=K.dtype, device=K.device)
         ve = torch.zeros_like(ke)
         ke[:, :, :ne] = K[:, :, nc:]

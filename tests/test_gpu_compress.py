@@ -82,3 +82,77 @@ def test_other_forms_take_the_general_path():
     assert takes(x, x, 64, 64, 64)
     assert not takes(x, x, 16, 64, 64) and not takes(x, x, 64, 16, 64) and not takes(x, x.float(), 64, 64, 64)
     assert not takes(off, x, 64, 64, 64) and not takes(x, x[:, :, :1].expand(1, 2, 96, 128), 64, 64, 64)
+
+
+# ---- DctCache: the matrix-core encoder, and kvq_dct_compress over views ------------------------------
+
+DCT_FIELDS = ("kc", "ks", "vc", "vs", "k_exact", "v_exact")
+
+
+def _plain(x, for_values):
+    """dct_encode of x through the kernel with one thread per channel, which sums in the fixed order: the rows
+    widened to float32 (exact) are the same sums."""
+    import kvq
+    return kvq.dct_encode(x.float(), for_values)
+
+
+def _same(a, b, what):
+    assert a.shape == b.shape and a.dtype == b.dtype, what
+    assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)), what
+
+
+def _dct_rows(kind, dtype, shape, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(shape, generator=g, device="cuda")
+    if kind == "walk":                                   # slow channels: one large coefficient, the rest near zero
+        x = x.cumsum(2) * 0.05 + 3.0
+    elif kind == "wide":                                 # magnitudes over decades, zeros among them
+        x = x * 10.0 ** torch.randint(-6, 4, (*shape[:3], 1), generator=g, device="cuda")
+        x = x * (torch.rand(shape, generator=g, device="cuda") > 0.3)
+    elif kind == "grid":                                 # few values: coefficients and quotients that tie
+        x = torch.randint(-2, 3, shape, generator=g, device="cuda").float() * 0.5
+    elif kind == "tiny":                                 # subnormals of both types, scales at the floor
+        x = x * 1e-6
+    elif kind == "huge":
+        x = x * (3e4 if dtype == torch.float16 else 1e36)
+    return x.to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["noise", "walk", "wide", "grid", "tiny", "huge"])
+def test_dct_encode_matrix_cores_equal_fixed_order(dtype, kind):
+    import kvq
+    x = _dct_rows(kind, dtype, (2, 3, 4096, 128), 7)
+    for for_values in (False, True):
+        for a, b, f in zip(kvq.dct_encode(x, for_values), _plain(x, for_values), ("codes", "scales")):
+            _same(a, b, f)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_dct_encode_non_finite(dtype):
+    import kvq
+    x = _dct_rows("noise", dtype, (1, 2, 192, 128), 8)
+    x[0, 0, 5, 3], x[0, 0, 70, 4], x[0, 1, 130, 9], x[0, 1, 60, 127] = float("inf"), float("-inf"), float("nan"), float("nan")
+    x[0, 0, 128:192, 20] = 0
+    for for_values in (False, True):
+        for a, b, f in zip(kvq.dct_encode(x, for_values), _plain(x, for_values), ("codes", "scales")):
+            _same(a, b, f)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,window,extra", [(1, 0, 0), (63, 0, 2), (64, 0, 0), (200, 9, 5), (4133, 64, 0)])
+def test_dct_compress_equals_general_path(dtype, T, window, extra, monkeypatch):
+    import kvq
+    from kvq import dct
+    base = _dct_rows("walk", dtype, (2, T + 3, 3, 128), T)
+    for K, V in ((base[:, :T].transpose(1, 2), base[:, 3:].transpose(1, 2)),            # token-major views
+                 (base.transpose(1, 2).contiguous()[:, :, 1:T + 1], base[:, :T].transpose(1, 2).contiguous())):
+        assert T == 1 or dct._compress_takes(K, V)
+        got = kvq.DctCache.from_context(K, V, window=window, extra_exact=extra)
+        monkeypatch.setattr(dct, "_compress_takes", lambda *a: False)
+        want = kvq.DctCache.from_context(K.float(), V.float(), window=window, extra_exact=extra)
+        monkeypatch.undo()
+        assert (got.T, got.n_exact) == (want.T, want.n_exact)
+        for f in DCT_FIELDS:
+            w = getattr(want, f)
+            _same(getattr(got, f), w.to(dtype) if f.endswith("exact") else w, f)

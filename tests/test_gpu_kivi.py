@@ -133,3 +133,14 @@ def test_pack_rows_and_lut_decode(bits):
     got = kvq.unpack_rows(packed, bits, torch.from_numpy(levels).cuda())
     np.testing.assert_array_equal(got.cpu().numpy(), levels[c])
     np.testing.assert_array_equal(got.cpu().numpy(), ok.unpack_rows_lut(ok.pack_rows(c, bits), bits, levels))
+
+
+@pytest.mark.parametrize("along_tokens", [True, False])
+def test_repeated_rows(along_tokens):
+    """Rows repeated by a zero token stride (an expanded view) are coded like their copy."""
+    import kvq
+    x = torch.randn((1, 2, 1, 128), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).cuda().expand(1, 2, 70, 128)
+    a = kvq.kivi_quant_stored(x, 4, 32, along_tokens, 0)
+    b = kvq.kivi_quant_stored(x.contiguous(), 4, 32, along_tokens, 0)
+    for f in ("packed", "lo", "scale"):
+        assert torch.equal(a[f], b[f]), f
