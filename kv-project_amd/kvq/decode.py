@@ -290,7 +290,7 @@ def kivi_decode(q: torch.Tensor, scaling: float, cache: PackedKIVICache, *,
         size = workspace_floats if scores is None else score_workspace_floats
         need = size(B, Hq, Hkv, Tq, d, cache.n_q, cache.n_exact, cache.group_k, cache.group_v,
                                 split_tokens)
-        workspace = torch.zeros((need,), dtype=torch.float32, device=q.device)
+        workspace = torch.empty((need,), dtype=torch.float32, device=q.device)
     if phases is None:
         phases = 7 if scores is not None else 3
     if scores is not None:

@@ -141,7 +141,7 @@ def mixed_decode(q: torch.Tensor, scaling: float, cache: MixedKIVICache, *, q_po
     if cache.k_exact.dtype != q.dtype:
         raise TypeError("q and the exact rows must share a dtype")
     if workspace is None:                      # a caller's workspace is size-checked by the library
-        workspace = torch.zeros((mixed_workspace_floats(B, Hq, Hkv, Tq, d, cache.nb, cache.n_exact),), dtype=torch.float32, device=q.device)
+        workspace = torch.empty((mixed_workspace_floats(B, Hq, Hkv, Tq, d, cache.nb, cache.n_exact),), dtype=torch.float32, device=q.device)
     out = _lib.out_or_new(out, (B, Tq, Hq, d), q.dtype, q.device, "mixed_decode")
     ep = cache.exact_pos if q_pos is not None else None
     qp = q_pos if ep is not None else None

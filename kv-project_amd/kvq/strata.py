@@ -258,7 +258,7 @@ def strata_decode(q: torch.Tensor, scaling: float, cache: StrataCache, *, q_pos:
     nt = len(tiers)
     if workspace is None:                      # a caller's workspace is size-checked by the library
         need = strata_workspace_floats(B, Hq, Hkv, Tq, d, cache.n_exact, [t.n for t in tiers], [t.bits for t in tiers])
-        workspace = torch.zeros((need,), dtype=torch.float32, device=q.device)
+        workspace = torch.empty((need,), dtype=torch.float32, device=q.device)
     out = _lib.out_or_new(out, (B, Tq, Hq, d), q.dtype, q.device, "strata_decode")
     P = ctypes.c_void_p
     bits = (ctypes.c_int * max(1, nt))(*[t.bits for t in tiers])
