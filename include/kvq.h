@@ -175,6 +175,27 @@ int kvq_kivi_decode(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int6
                     int64_t workspace_floats, float* scores, int64_t scores_bh, float score_weight,
                     int64_t split_tokens, int phases, void* stream);
 
+/* kvq_kivi_decode with the query tokens' positions by value: q_at is HOST memory, Tq int64 (read before
+ * the call returns), in the place of the device array q_pos; exact_pos must be set. */
+int kvq_kivi_decode_at(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                       int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t d, float scaling,
+                       const uint8_t* kc, const uint16_t* k_lo, const uint16_t* k_sc,
+                       const uint8_t* vc, const uint16_t* vmeta, int64_t cap_t, int64_t n_q,
+                       int group_k, int group_v, const void* k_exact, const void* v_exact,
+                       int exact_dtype, int64_t cap_e, int64_t n_exact, const int64_t* exact_pos,
+                       const int64_t* q_at, void* out, int out_dtype, float* workspace,
+                       int64_t workspace_floats, float* scores, int64_t scores_bh, float score_weight,
+                       int64_t split_tokens, int phases, void* stream);
+
+/* Rows of t appended tokens k, v (B, H, t, d) of `dtype` (element strides, channels contiguous) copied
+ * behind the exact rows of a decode state: slots n_exact .. of k_exact / v_exact (BH, cap_e, d) of the same
+ * dtype (LayerState.append, STRATA_KV.py:707-714).  positions (HOST memory, t <= 8 values, or NULL with
+ * exact_pos NULL) go to exact_pos[n_exact ..].  Rows, strides and pointers in whole 16-byte units. */
+int kvq_exact_append(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb,
+                     int64_t v_sh, int64_t v_st, int dtype, int64_t B, int64_t H, int64_t t, int64_t d,
+                     const int64_t* positions, void* k_exact, void* v_exact, int64_t cap_e, int64_t n_exact,
+                     int64_t* exact_pos, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * A4  kvq_kivi_decode without a workspace: the allocation-free variant.
  * No counterpart in the reference.  It is for callers that cannot allocate device memory (code

@@ -127,6 +127,35 @@ __global__ void kivi_append_kernel(const void* __restrict__ k_new, const void* _
   store_from_f32<DT>(v_ring, ring_bh + slot * d + c, vv);
 }
 
+// Rows of appended tokens copied behind the exact rows of a decode state, keys and values and the
+// positions in one launch (a token step is bound by its launches: three uploads and two copies took
+// 45 us of host time a layer).  A thread moves 16 bytes; strides in bytes; the positions come by value.
+struct ExactAppend {
+  const char* src[2];
+  int64_t sb[2], sh[2], st[2];
+  uint4* dst[2];                    // (BH, cap_e, row)
+  int H, t, row_units;
+  int64_t cap_e, n_exact, units;    // units per side
+  int64_t* exact_pos;               // null: left alone
+  int64_t pos[8];
+};
+
+__global__ __launch_bounds__(256) void exact_append_kernel(ExactAppend p) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (p.exact_pos != nullptr && i == 0) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k < p.t) p.exact_pos[p.n_exact + k] = p.pos[k];
+  }
+  const bool keys = i < p.units;
+  const int64_t u = keys ? i : i - p.units;
+  if (u >= p.units) return;
+  const int64_t row = u / p.row_units, bh = row / p.t, b = bh / p.H, h = bh - b * p.H;
+  const int64_t r = row - bh * p.t, c = u - row * p.row_units;
+  const char* src = keys ? p.src[0] + b * p.sb[0] + h * p.sh[0] + r * p.st[0] : p.src[1] + b * p.sb[1] + h * p.sh[1] + r * p.st[1];
+  (keys ? p.dst[0] : p.dst[1])[(bh * p.cap_e + p.n_exact + r) * p.row_units + c] = *reinterpret_cast<const uint4*>(src + 16 * c);
+}
+
 }  // namespace
 }  // namespace kvq
 
@@ -155,5 +184,32 @@ extern "C" int kvq_kivi_append(const void* k_new, const void* v_new, int dtype, 
                                               (int)Hkv, (int)d, pos, k_ring, v_ring, W, kc, k_lo, k_sc, vc,
                                               vmeta, cap_t, group_k, group_v));
   KVQ_LAUNCH_CHECK("kvq_kivi_append");
+  return KVQ_OK;
+}
+
+extern "C" int kvq_exact_append(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb,
+                                int64_t v_sh, int64_t v_st, int dtype, int64_t B, int64_t H, int64_t t, int64_t d,
+                                const int64_t* positions, void* k_exact, void* v_exact, int64_t cap_e, int64_t n_exact,
+                                int64_t* exact_pos, void* stream) {
+  KVQ_REQUIRE(k && v && k_exact && v_exact, "kvq_exact_append: null pointer");
+  KVQ_REQUIRE(valid_dtype(dtype) && B >= 0 && H > 0 && B * H < (1LL << 24) && d > 0 && t > 0, "kvq_exact_append: bad sizes");
+  KVQ_REQUIRE(n_exact >= 0 && n_exact + t <= cap_e && cap_e < (1LL << 31), "kvq_exact_append: the rows do not fit");
+  KVQ_REQUIRE((positions == nullptr) == (exact_pos == nullptr) && (positions == nullptr || t <= 8),
+              "kvq_exact_append: at most 8 positions, with exact_pos");
+  const int es = dtype == KVQ_F32 ? 4 : 2;
+  KVQ_REQUIRE(d * es % 16 == 0, "kvq_exact_append: rows must be whole 16-byte units");
+  for (const int64_t x : {k_sb, k_sh, k_st, v_sb, v_sh, v_st})
+    KVQ_REQUIRE(x * es % 16 == 0, "kvq_exact_append: strides must be multiples of 16 bytes");
+  for (const void* x : {k, v, static_cast<const void*>(k_exact), static_cast<const void*>(v_exact)})
+    KVQ_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0, "kvq_exact_append: pointers must be 16-byte aligned");
+  if (B == 0) return KVQ_OK;
+  ExactAppend p{{static_cast<const char*>(k), static_cast<const char*>(v)}, {k_sb * es, v_sb * es}, {k_sh * es, v_sh * es},
+                {k_st * es, v_st * es}, {static_cast<uint4*>(k_exact), static_cast<uint4*>(v_exact)}, static_cast<int>(H),
+                static_cast<int>(t), static_cast<int>(d * es / 16), cap_e, n_exact, B * H * t * (d * es / 16), exact_pos, {}};
+  for (int64_t i = 0; positions != nullptr && i < t; ++i) p.pos[i] = positions[i];
+  const int64_t blocks = (2 * p.units + 255) / 256;
+  KVQ_REQUIRE(blocks < (1LL << 31), "kvq_exact_append: too large");
+  hipLaunchKernelGGL(exact_append_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+  KVQ_LAUNCH_CHECK("kvq_exact_append");
   return KVQ_OK;
 }

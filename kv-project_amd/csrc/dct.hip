@@ -1415,7 +1415,8 @@ extern "C" int kvq_dct_decode(const void* q, int q_dtype, int64_t q_sb, int64_t 
     MergeArgs ma{p.ws_o, p.ws_m, p.ws_l, p.S_all, p.ex_o, p.ex_m, p.ex_l, p.S_ex,
                  p.Hq, p.Hkv, p.Tq, p.rep, p.R_real, p.out, nullptr, ExactArgs{}};
     if (ex_merge)
-      ma.ex = ExactArgs{q, q_sb, q_sh, q_st, p.qscale, k_exact, v_exact, cap_e, static_cast<int>(n_exact), exact_pos, q_pos};
+      ma.ex = ExactArgs{q, q_sb, q_sh, q_st, p.qscale, k_exact, v_exact, cap_e, static_cast<int>(n_exact), exact_pos, q_pos,
+                        exact_pos != nullptr && q_pos != nullptr, {}};
     const int rc = launch_merge_rows(ma, R, p.BH, q_dtype, s);
     if (rc != KVQ_OK) return rc;
   }

@@ -106,7 +106,9 @@ struct DecodeParams {
   int64_t cap_e;
   int n_exact;
   const int64_t* exact_pos;
-  const int64_t* q_pos;
+  const int64_t* q_pos;               // device positions of the query tokens, or null: q_at holds row r's
+  bool masked;                        // exact rows visible by position (else all are)
+  int64_t q_at[8];
   float* ws_m;
   float* ws_l;
   float* row_ml;                      // per (b, h, row): global max (log2 units) and sum of exp2
@@ -136,6 +138,11 @@ __device__ __forceinline__ int64_t q_offset(const DecodeParams& p, int b, int h,
   const int t = r % p.Tq;
   return static_cast<int64_t>(b) * p.q_sb + static_cast<int64_t>(hq) * p.q_sh +
          static_cast<int64_t>(t) * p.q_st;
+}
+
+// Position of query row r's token (0 where nothing is masked).
+__device__ __forceinline__ int64_t q_pos_of_row(const DecodeParams& p, int r) {
+  return !p.masked ? 0 : p.q_pos != nullptr ? p.q_pos[r % p.Tq] : p.q_at[r];
 }
 
 template <int R, int DT>
@@ -244,7 +251,7 @@ __device__ void exact_block(const DecodeParams& p, int bh, int sidx, float* smem
   const int j = lane >> 4, part = lane & 15;       // row slot of 4, 8-channel slice of 16
   const int w0 = e0 + (e1 - e0) * wave / kWaves, w1 = e0 + (e1 - e0) * (wave + 1) / kWaves;
   const int64_t kbase = static_cast<int64_t>(bh) * p.cap_e * kD;
-  const bool masked = p.exact_pos != nullptr && p.q_pos != nullptr;
+  const bool masked = p.masked;
   float qv[R][8];                                   // scaled query rows (set once they are staged)
   int64_t qp[R];
   float m[R], l[R], o[R][8];
@@ -311,7 +318,7 @@ __device__ void exact_block(const DecodeParams& p, int bh, int sidx, float* smem
 #pragma unroll
     for (int k = 0; k < 8; ++k) qv[r][k] = qs[r][8 * part + k];
 #pragma unroll
-  for (int r = 0; r < R; ++r) qp[r] = masked ? p.q_pos[r % p.Tq] : 0;
+  for (int r = 0; r < R; ++r) qp[r] = q_pos_of_row(p, r);
   if (w0 < w1) {
     for (int i0 = w0;; i0 += 16) {
       if (i0 != w0) load_rows(i0 + 12 + j, x3);
@@ -844,11 +851,11 @@ __device__ void packed_block(const DecodeParams& p, int bh, int sidx, float* sme
     }
     if (threadIdx.x < 64) {
       const int i = threadIdx.x;
-      const bool masked = p.exact_pos != nullptr && p.q_pos != nullptr;
+      const bool masked = p.masked;
       const int64_t ep = (masked && i < fne) ? p.exact_pos[fe0 + i] : 0;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const bool vis = i < fne && (!masked || ep <= p.q_pos[r % p.Tq]);
+        const bool vis = i < fne && (!masked || ep <= q_pos_of_row(p, r));
         const uint64_t bal = __ballot(vis);
         if (i == 0) emask[r] = static_cast<uint32_t>(bal);
       }
@@ -874,6 +881,7 @@ __device__ void packed_block(const DecodeParams& p, int bh, int sidx, float* sme
     const void* ek_lds = ek4;
 #pragma unroll
     for (int u = 0; u < kFusedExact / 16; ++u) {
+      if (16 * u >= fne) break;
       const int i = 16 * u + 4 * wave + g;
       float kx[8];
       load8<DT>(ek_lds, static_cast<int64_t>(i) * kD + 8 * n, kx);
@@ -890,25 +898,29 @@ __device__ void packed_block(const DecodeParams& p, int bh, int sidx, float* sme
     const void* ev_lds = ev4;
     for (int idx = threadIdx.x; idx < p.R_real * kD; idx += kThreads) {
       const int r = idx / kD, c = idx % kD;
-      // every logit of the row and every value of channel c read before any use (rows past fne
-      // hold stale data: masked by selects)
-      float sl[kFusedExact], vv[kFusedExact];
-#pragma unroll
-      for (int i = 0; i < kFusedExact; i += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(&esl[r * kFusedExact + i]);
-        sl[i] = x.x; sl[i + 1] = x.y; sl[i + 2] = x.z; sl[i + 3] = x.w;
-      }
-#pragma unroll
-      for (int i = 0; i < kFusedExact; ++i) vv[i] = load_as_f32<DT>(ev_lds, static_cast<int64_t>(i) * kD + c);
+      // rows in eights, only as many as the block holds (rows past fne hold stale data: masked by selects)
       float me = -INFINITY, le = 0.0f, oe = 0.0f;
+      for (int i0 = 0; i0 < fne; i0 += 8) {
+        const float4 x = *reinterpret_cast<const float4*>(&esl[r * kFusedExact + i0]);
+        const float4 y = *reinterpret_cast<const float4*>(&esl[r * kFusedExact + i0 + 4]);
+        const float sl[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
 #pragma unroll
-      for (int i = 0; i < kFusedExact; ++i) me = fmaxf(me, i < fne ? sl[i] : -INFINITY);
+        for (int i = 0; i < 8; ++i) me = fmaxf(me, i0 + i < fne ? sl[i] : -INFINITY);
+      }
       if (me != -INFINITY) {
+        for (int i0 = 0; i0 < fne; i0 += 8) {
+          const float4 x = *reinterpret_cast<const float4*>(&esl[r * kFusedExact + i0]);
+          const float4 y = *reinterpret_cast<const float4*>(&esl[r * kFusedExact + i0 + 4]);
+          const float sl[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+          float vv[8];
 #pragma unroll
-        for (int i = 0; i < kFusedExact; ++i) {
-          const float pr = i < fne ? __builtin_amdgcn_exp2f(sl[i] - me) : 0.0f;
-          le += pr;
-          oe = __builtin_fmaf(pr, i < fne ? vv[i] : 0.0f, oe);
+          for (int i = 0; i < 8; ++i) vv[i] = load_as_f32<DT>(ev_lds, static_cast<int64_t>(i0 + i) * kD + c);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float pr = i0 + i < fne ? __builtin_amdgcn_exp2f(sl[i] - me) : 0.0f;
+            le += pr;
+            oe = __builtin_fmaf(pr, i0 + i < fne ? vv[i] : 0.0f, oe);
+          }
         }
       }
       eo[idx] = oe;
@@ -1157,7 +1169,8 @@ int launch(DecodeParams& p, int phases, hipStream_t stream) {
     ma.out = p.out; ma.row_ml = p.row_ml;
     if (p.fused_per == 0 && p.n_exact_wg == 0 && p.n_exact > 0)
       ma.ex = ExactArgs{p.q, p.q_sb, p.q_sh, p.q_st, p.qscale, p.k_exact, p.v_exact, p.cap_e, p.n_exact,
-                        p.exact_pos, p.q_pos};
+                        p.exact_pos, p.q_pos, p.masked,
+                        {p.q_at[0], p.q_at[1], p.q_at[2], p.q_at[3], p.q_at[4], p.q_at[5], p.q_at[6], p.q_at[7]}};
     const int rc = launch_merge_rows(ma, R, p.BH, DT, stream);
     if (rc != KVQ_OK) return rc;
   }
@@ -1326,14 +1339,16 @@ extern "C" int64_t kvq_kivi_score_workspace(int64_t B, int64_t Hq, int64_t Hkv, 
   return (base + 3) / 4 * 4 + B * Hkv * ((n_q + 31) / 32) * 32 * R;    // logits 16-byte aligned
 }
 
-extern "C" int kvq_kivi_decode(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_st,
+namespace {
+// q_at (host memory): the Tq query positions by value, instead of q_pos on the device
+int kivi_decode_at(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_st,
                                int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int64_t d,
                                float scaling, const uint8_t* kc, const uint16_t* k_lo,
                                const uint16_t* k_sc, const uint8_t* vc, const uint16_t* vmeta,
                                int64_t cap_t, int64_t n_q, int group_k, int group_v,
                                const void* k_exact, const void* v_exact, int exact_dtype,
                                int64_t cap_e, int64_t n_exact, const int64_t* exact_pos,
-                               const int64_t* q_pos, void* out, int out_dtype, float* workspace,
+                               const int64_t* q_pos, const int64_t* q_at, void* out, int out_dtype, float* workspace,
                                int64_t workspace_floats, float* scores, int64_t scores_bh,
                                float score_weight, int64_t split_tokens, int phases,
                                void* stream) {
@@ -1358,7 +1373,9 @@ extern "C" int kvq_kivi_decode(const void* q, int q_dtype, int64_t q_sb, int64_t
                                reinterpret_cast<uintptr_t>(v_exact) % 16 == 0),
               "kvq_kivi_decode: exact rows must be 16-byte aligned");
   KVQ_REQUIRE(q && out && workspace, "kvq_kivi_decode: null q/out/workspace");
-  KVQ_REQUIRE((exact_pos == nullptr) == (q_pos == nullptr), "kvq_kivi_decode: exact_pos and q_pos go together");
+  KVQ_REQUIRE(q_pos == nullptr || q_at == nullptr, "kvq_kivi_decode: positions on the device or by value, not both");
+  KVQ_REQUIRE((exact_pos == nullptr) == (q_pos == nullptr && q_at == nullptr),
+              "kvq_kivi_decode: exact_pos and q_pos go together");
   KVQ_REQUIRE(n_q < (1LL << 31) && B * Hkv < 65536, "kvq_kivi_decode: sizes out of range");
   const SplitPlan sp = plan_split(B, Hq, Hkv, Tq, n_q, n_exact, split_tokens, group_k, group_v);
   const int64_t need = B * Hkv * (static_cast<int64_t>(sp.S1) * sp.R * (kD + 2) + 2 * sp.R);
@@ -1374,6 +1391,8 @@ extern "C" int kvq_kivi_decode(const void* q, int q_dtype, int64_t q_sb, int64_t
   p.cap_t = cap_t; p.n_q = (int)n_q; p.group_k = group_k; p.group_v = group_v; p.ngv = (int)(kD / group_v);
   p.k_exact = k_exact; p.v_exact = v_exact; p.cap_e = cap_e; p.n_exact = (int)n_exact;
   p.exact_pos = exact_pos; p.q_pos = q_pos;
+  p.masked = exact_pos != nullptr;
+  for (int r = 0; r < R_real && q_at != nullptr; ++r) p.q_at[r] = q_at[r % Tq];
   const int64_t nrow = B * Hkv * static_cast<int64_t>(sp.S1) * sp.R;
   p.ws_o = workspace;
   p.ws_m = workspace + nrow * kD;
@@ -1417,6 +1436,36 @@ extern "C" int kvq_kivi_decode(const void* q, int q_dtype, int64_t q_sb, int64_t
   }
 #undef KVQ_R
 #undef KVQ_GV
+}
+}  // namespace
+
+extern "C" int kvq_kivi_decode(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_st, int64_t B,
+                               int64_t Hq, int64_t Hkv, int64_t Tq, int64_t d, float scaling, const uint8_t* kc, const
+                               uint16_t* k_lo, const uint16_t* k_sc, const uint8_t* vc, const uint16_t* vmeta, int64_t
+                               cap_t, int64_t n_q, int group_k, int group_v, const void* k_exact, const void* v_exact,
+                               int exact_dtype, int64_t cap_e, int64_t n_exact, const int64_t* exact_pos, const
+                               int64_t* q_pos, void* out, int out_dtype, float* workspace, int64_t workspace_floats,
+                               float* scores, int64_t scores_bh, float score_weight, int64_t split_tokens, int phases,
+                               void* stream) {
+  return kivi_decode_at(q, q_dtype, q_sb, q_sh, q_st, B, Hq, Hkv, Tq, d, scaling, kc, k_lo, k_sc, vc, vmeta, cap_t, n_q,
+                        group_k, group_v, k_exact, v_exact, exact_dtype, cap_e, n_exact, exact_pos, q_pos, nullptr,
+                        out, out_dtype, workspace, workspace_floats, scores, scores_bh, score_weight, split_tokens,
+                        phases, stream);
+}
+
+extern "C" int kvq_kivi_decode_at(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_st, int64_t B,
+                                  int64_t Hq, int64_t Hkv, int64_t Tq, int64_t d, float scaling, const uint8_t* kc,
+                                  const uint16_t* k_lo, const uint16_t* k_sc, const uint8_t* vc, const uint16_t*
+                                  vmeta, int64_t cap_t, int64_t n_q, int group_k, int group_v, const void* k_exact,
+                                  const void* v_exact, int exact_dtype, int64_t cap_e, int64_t n_exact, const int64_t*
+                                  exact_pos, const int64_t* q_at, void* out, int out_dtype, float* workspace, int64_t
+                                  workspace_floats, float* scores, int64_t scores_bh, float score_weight, int64_t
+                                  split_tokens, int phases, void* stream) {
+  KVQ_REQUIRE(exact_pos != nullptr && q_at != nullptr, "kvq_kivi_decode_at: needs exact_pos and the query positions");
+  return kivi_decode_at(q, q_dtype, q_sb, q_sh, q_st, B, Hq, Hkv, Tq, d, scaling, kc, k_lo, k_sc, vc, vmeta, cap_t, n_q,
+                        group_k, group_v, k_exact, v_exact, exact_dtype, cap_e, n_exact, exact_pos, nullptr, q_at,
+                        out, out_dtype, workspace, workspace_floats, scores, scores_bh, score_weight, split_tokens,
+                        phases, stream);
 }
 
 namespace kvq {
@@ -1494,6 +1543,7 @@ extern "C" int kvq_kivi_decode_retained(const void* q, int q_dtype, int64_t q_sb
   p.cap_t = cap_t; p.n_q = (int)n_q; p.group_k = group_k; p.group_v = group_v; p.ngv = (int)(kD / group_v);
   p.k_exact = k_exact; p.v_exact = v_exact; p.cap_e = cap_e; p.n_exact = (int)n_exact;
   p.exact_pos = exact_pos; p.q_pos = q_pos;
+  p.masked = exact_pos != nullptr;
   const int64_t nrow = B * Hkv * static_cast<int64_t>(S1) * rp.R;
   p.ws_o = workspace;
   p.ws_m = workspace + nrow * kD;

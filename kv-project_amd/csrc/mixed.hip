@@ -626,7 +626,8 @@ extern "C" int kvq_mixed_decode(const void* q, int q_dtype, int64_t q_sb, int64_
   ma.out = out;
   if (exact_in_merge(n_exact)) {
     ma.ex = ExactArgs{q, q_sb, q_sh, q_st, scaling * 1.4426950408889634f, k_exact, v_exact, cap_e,
-                      static_cast<int>(n_exact), exact_pos, q_pos};
+                      static_cast<int>(n_exact), exact_pos, q_pos,
+                        exact_pos != nullptr && q_pos != nullptr, {}};
   } else if (n_exact > 0) {
     if (phases & 1) {
       const int rc = kvq_kivi_decode(q, q_dtype, q_sb, q_sh, q_st, B, Hq, Hkv, Tq, d, scaling, nullptr, nullptr, nullptr,

@@ -32,7 +32,9 @@ struct ExactArgs {
   int64_t cap_e;
   int n;                          // 0: no exact rows in the merge
   const int64_t* exact_pos;
-  const int64_t* q_pos;
+  const int64_t* q_pos;           // device positions of the query tokens, or null: q_at holds them
+  bool masked;                    // visibility by position (else every row is visible)
+  int64_t q_at[8];
 };
 
 // Exact windows up to this many rows are attended inside the merge (one pass over them per query
@@ -91,8 +93,14 @@ __device__ void exact_partial(const ExactArgs& e, int b, int hq, int t, int bh, 
 #pragma unroll
   for (int k = 0; k < 8; ++k) qv[k] = load_as_f32<DT>(e.q, qo + k) * e.qscale;
   const int64_t base = static_cast<int64_t>(bh) * e.cap_e * D;
-  const bool masked = e.exact_pos != nullptr && e.q_pos != nullptr;
-  const int64_t qp = masked ? e.q_pos[t] : 0;
+  const bool masked = e.masked;
+  int64_t qp = 0;
+  if (masked && e.q_pos != nullptr) {
+    qp = e.q_pos[t];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qp = t == k ? e.q_at[k] : qp;
+  }
   for (int i0 = 0; i0 < n; i0 += kRowsPerPass * kKeyBatch) {
     float kx[kKeyBatch][8];
     bool vis[kKeyBatch];

@@ -714,7 +714,8 @@ extern "C" int kvq_quasar_decode(const void* q, int q_dtype, int64_t q_sh, int64
   p.ws_o = ws_o;
   p.tvt = T_v;
   p.muv = mu_v;
-  p.ex = ExactArgs{q, 0, q_sh, q_st, qscale, k_exact, v_exact, cap_e, static_cast<int>(n_exact), exact_pos, q_pos};
+  p.ex = ExactArgs{q, 0, q_sh, q_st, qscale, k_exact, v_exact, cap_e, static_cast<int>(n_exact), exact_pos, q_pos,
+                        exact_pos != nullptr && q_pos != nullptr, {}};
   p.S_ex = static_cast<int>(S_ex);
   p.ex_m = ex_m;
   p.ex_l = ex_l;

@@ -41,6 +41,10 @@ SIGNATURES = {
     "kvq_kivi_decode": (i32, [vp, i32, i64, i64, i64, i64, i64, i64, i64, i64, f32,
                               vp, vp, vp, vp, vp, i64, i64, i32, i32, vp, vp, i32, i64, i64,
                               vp, vp, vp, i32, vp, i64, vp, i64, f32, i64, i32, vp]),
+    "kvq_kivi_decode_at": (i32, [vp, i32, i64, i64, i64, i64, i64, i64, i64, i64, f32,
+                              vp, vp, vp, vp, vp, i64, i64, i32, i32, vp, vp, i32, i64, i64,
+                              vp, vp, vp, i32, vp, i64, vp, i64, f32, i64, i32, vp]),
+    "kvq_exact_append": (i32, [vp, i64, i64, i64, vp, i64, i64, i64, i32, i64, i64, i64, i64, vp, vp, vp, i64, i64, vp, vp]),
     "kvq_kivi_decode_noalloc": (i32, [vp, i32, i64, i64, i64, i64, i64, i64, i64, i64, f32,
                                       vp, vp, vp, vp, vp, i64, i64, i32, i32, vp, vp, i32, i64, i64,
                                       vp, vp, vp, i32, vp, i64, f32, i64, i32, vp]),

@@ -9,6 +9,7 @@ decode step of attention over it; it replaces chunked_attention over KIVI token 
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 from typing import Optional
@@ -253,7 +254,7 @@ def kivi_decode(q: torch.Tensor, scaling: float, cache: PackedKIVICache, *,
 
     With ``q_pos`` (Tq,) int64 and ``cache.exact_pos`` set, exact row i is visible to query t iff
     exact_pos[i] <= q_pos[t] (the causal rule of chunked_attention among appended rows); every
-    packed row is visible.  ``phases`` 1/2 run only the split / merge kernel (timing).
+    packed row is visible.  A ``q_pos`` in host memory goes with the launch by value (no upload).  ``phases`` 1/2 run only the split / merge kernel (timing).
 
     ``scores`` (B, Hkv, >= n_q) float32 on the GPU: the step also adds ``score_weight`` times the
     probability mass each packed token received from the query heads of its KV group (the
@@ -301,22 +302,32 @@ def kivi_decode(q: torch.Tensor, scaling: float, cache: PackedKIVICache, *,
     ep = cache.exact_pos if q_pos is not None else None
     qp = q_pos if ep is not None else None
     dt = _lib.DTYPE_CODE[q.dtype]
+    entry, qp_arg = "kvq_kivi_decode", _lib.ptr(qp)
+    if qp is not None and not qp.is_cuda:
+        if static_scratch:
+            qp = qp.to(device=q.device, dtype=torch.int64)
+            qp_arg = qp.data_ptr()
+        else:
+            at = qp.reshape(-1).tolist()
+            if len(at) != Tq:
+                raise ValueError("q_pos must hold one position per query token")
+            entry, qp_arg = "kvq_kivi_decode_at", ctypes.addressof(held := (ctypes.c_int64 * Tq)(*at))
     if static_scratch:
         _lib.call("kvq_kivi_decode_noalloc", q.data_ptr(), dt, q.stride(0), q.stride(1), q.stride(2),
                   B, Hq, Hkv, Tq, d, float(scaling),
                   cache.kc.data_ptr(), cache.k_lo.data_ptr(), cache.k_sc.data_ptr(), cache.vc.data_ptr(),
                   cache.vmeta.data_ptr(), cache.cap_t, cache.n_q, cache.group_k, cache.group_v,
                   cache.k_exact.data_ptr(), cache.v_exact.data_ptr(), dt, cache.cap_e, cache.n_exact,
-                  _lib.ptr(ep), _lib.ptr(qp), out.data_ptr(), dt,
+                  _lib.ptr(ep), qp_arg, out.data_ptr(), dt,
                   _lib.ptr(scores), scores.stride(1) if scores is not None else 0, float(score_weight),
                   split_tokens, phases, _lib.stream_of(q))
         return out
-    _lib.call("kvq_kivi_decode", q.data_ptr(), dt, q.stride(0), q.stride(1), q.stride(2),
+    _lib.call(entry, q.data_ptr(), dt, q.stride(0), q.stride(1), q.stride(2),
               B, Hq, Hkv, Tq, d, float(scaling),
               cache.kc.data_ptr(), cache.k_lo.data_ptr(), cache.k_sc.data_ptr(), cache.vc.data_ptr(),
               cache.vmeta.data_ptr(), cache.cap_t, cache.n_q, cache.group_k, cache.group_v,
               cache.k_exact.data_ptr(), cache.v_exact.data_ptr(), dt, cache.cap_e, cache.n_exact,
-              _lib.ptr(ep), _lib.ptr(qp), out.data_ptr(), dt, workspace.data_ptr(), workspace.numel(),
+              _lib.ptr(ep), qp_arg, out.data_ptr(), dt, workspace.data_ptr(), workspace.numel(),
               _lib.ptr(scores), scores.stride(1) if scores is not None else 0, float(score_weight),
               split_tokens, phases, _lib.stream_of(q))
     return out

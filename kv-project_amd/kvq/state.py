@@ -21,6 +21,7 @@ switching paths.
 """
 from __future__ import annotations
 
+import ctypes
 from contextlib import contextmanager
 from typing import Dict, Optional
 
@@ -100,6 +101,20 @@ class DecodeCtl:
         return src.attend(q, scaling, self.pos, self.chunk), None
 
 
+def _append_takes(c: PackedKIVICache, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether kvq_exact_append takes these rows: on the cache's device, of its dtype and sizes, in 16-byte pieces
+    (every other form is converted and copied by torch)."""
+    B, H, _, d = c.k_exact.shape
+    es = c.k_exact.element_size()
+    t = k.shape[2]
+    for x, y in ((k, c.k_exact), (v, c.v_exact)):
+        if (x.device != y.device or x.dtype != y.dtype or tuple(x.shape) != (B, H, t, d) or x.stride(3) != 1
+                or x.data_ptr() % 16 or y.data_ptr() % 16 or not y.is_contiguous() or x.requires_grad
+                or any(s * es % 16 for s in x.stride()[:3])):
+            return False
+    return t > 0 and B * H > 0 and d * es % 16 == 0
+
+
 class PackedState:
     """The decode-state protocol (LayerState / StrataState, STRATA_KV.py:682-719, 1710-1818) over one
     ``PackedKIVICache`` ``self.cache`` whose exact rows carry positions (``cache.exact_pos``): append,
@@ -118,10 +133,20 @@ class PackedState:
         t = k.shape[2]
         if c.n_exact + t > c.cap_e:
             raise RuntimeError("decode buffer exhausted")
-        c.k_exact[:, :, c.n_exact:c.n_exact + t] = k.to(c.k_exact.dtype)
-        c.v_exact[:, :, c.n_exact:c.n_exact + t] = v.to(c.v_exact.dtype)
-        p = torch.as_tensor(pos, dtype=torch.int64).reshape(-1).to(c.k_exact.device)
-        c.exact_pos[c.n_exact:c.n_exact + t] = p
+        p = torch.as_tensor(pos, dtype=torch.int64).reshape(-1)
+        if _append_takes(c, k, v):
+            at = None if p.is_cuda or p.numel() != t or t > 8 else (ctypes.c_int64 * t)(*p.tolist())
+            B, H, cap_e, d = c.k_exact.shape
+            _lib.call("kvq_exact_append", k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3],
+                      _lib.DTYPE_CODE[k.dtype], B, H, t, d, None if at is None else ctypes.addressof(at),
+                      c.k_exact.data_ptr(), c.v_exact.data_ptr(), cap_e, c.n_exact,
+                      None if at is None else c.exact_pos.data_ptr(), _lib.stream_of(k))
+        else:
+            at = None
+            c.k_exact[:, :, c.n_exact:c.n_exact + t] = k.to(c.k_exact.dtype)
+            c.v_exact[:, :, c.n_exact:c.n_exact + t] = v.to(c.v_exact.dtype)
+        if at is None:                          # positions on the device, or many, or one for all rows
+            c.exact_pos[c.n_exact:c.n_exact + t] = p.to(c.k_exact.device)
         c.n_exact += t
         self.n += t
 
@@ -134,9 +159,11 @@ class PackedState:
         if not self.use_kernel:
             raise RuntimeError(f"{type(self).__name__}: the HIP decode kernel is disabled (check_kernel failed)")
         c = self.cache
-        qp = torch.as_tensor(qpos, dtype=torch.int64).reshape(-1).to(q.device)
+        qp = torch.as_tensor(qpos, dtype=torch.int64).reshape(-1)
         if qp.numel() != q.shape[2]:
             raise ValueError("qpos must hold one position per query token")
+        if qp.is_cuda:
+            qp = qp.to(q.device).contiguous()
         return kivi_decode(q.to(c.k_exact.dtype), scaling, c, q_pos=qp, chunk=chunk).to(q.dtype)
 
     @torch.no_grad()

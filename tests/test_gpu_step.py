@@ -1,0 +1,93 @@
+"""Token steps whose positions go with the launches by value (kvq_exact_append, kvq_kivi_decode_at) against
+the same steps with positions on the device and rows copied by torch: equal bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(g, *shape, dtype=torch.float16):
+    return torch.randn(shape, generator=g, device="cuda").to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Hkv,rep,T,window,extra,steps", [
+    (1, 2, 4, 700, 64, 40, (1, 2, 1, 9)),             # window in the packed splits; 9 > 8 tokens: pieces, positions uploaded
+    (2, 3, 1, 300, 96, 80, (8, 1, 3)),
+    (1, 1, 8, 2000, 900, 8, (1, 1)),                  # window in the merge
+    (1, 1, 3, 1500, 1300, 8, (2, 2)),                 # window in exact-row blocks of their own
+])
+def test_positions_by_value(dtype, B, Hkv, rep, T, window, extra, steps, monkeypatch):
+    import kvq
+    from kvq import state
+    g = torch.Generator(device="cuda").manual_seed(T)
+    K, V = _rows(g, B, Hkv, T, 128, dtype=dtype), _rows(g, B, Hkv, T, 128, dtype=dtype)
+    a, b = (kvq.KIVIState(K, V, window=window, group_k=32, group_v=64, extra=extra) for _ in (0, 1))
+    pos = T
+    for t in steps:
+        # token-major projections, viewed; the appended rows past the query's position must stay hidden
+        k, v = (_rows(g, B, t, Hkv, 128, dtype=dtype).transpose(1, 2) for _ in (0, 1))
+        q = _rows(g, B, Hkv * rep, t, 128, dtype=dtype)
+        at = torch.arange(pos, pos + t)
+        a.append(k, v, at)
+        with monkeypatch.context() as m:
+            m.setattr(state, "_append_takes", lambda *x: False)
+            b.append(k, v, at.cuda())
+        for f in ("k_exact", "v_exact"):
+            x, y = getattr(a.cache, f), getattr(b.cache, f)
+            assert torch.equal(x[:, :, :a.cache.n_exact], y[:, :, :a.cache.n_exact])
+        assert torch.equal(a.cache.exact_pos, b.cache.exact_pos) and (a.n, a.cache.n_exact) == (b.n, b.cache.n_exact)
+        for shift in (0, -1, 1):                      # earlier positions hide appended rows
+            x, y = a.attend(q, 0.1, at + shift), b.attend(q, 0.1, (at + shift).cuda())
+            assert torch.isfinite(x.float()).all() and torch.equal(x, y)
+        pos += t
+    assert torch.equal(a.attend(q, 0.1, list(range(pos - t, pos))), x if t == 0 else a.attend(q, 0.1, at.cuda()))
+
+
+def test_append_other_forms():
+    """Rows of another dtype, one position for several rows, a full buffer."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(1)
+    st = kvq.KIVIState(_rows(g, 1, 2, 100, 128), _rows(g, 1, 2, 100, 128), window=40, group_k=32, group_v=32, extra=6)
+    k, v = _rows(g, 1, 2, 2, 128, dtype=torch.float32), _rows(g, 1, 2, 2, 128, dtype=torch.float32)
+    st.append(k, v, torch.tensor([100, 101]))
+    st.append(k.half(), v.half(), torch.tensor([7]))
+    assert st.cache.exact_pos[40:44].tolist() == [100, 101, 7, 7]
+    assert torch.equal(st.cache.k_exact[:, :, 40:42], k.half()) and torch.equal(st.cache.v_exact[:, :, 42:44], v.half())
+    st.append(k[:, :, :1].half(), v[:, :, :1].half(), 103)
+    assert st.cache.exact_pos[44].item() == 103
+    with pytest.raises(RuntimeError):
+        st.append(k.half(), v.half(), torch.tensor([104, 105]))
+    q = _rows(g, 1, 4, 2, 128)
+    with pytest.raises(ValueError):
+        st.attend(q, 0.1, torch.tensor([1]))
+    strided = torch.tensor([103, 0, 104, 0], device="cuda")[::2]
+    assert torch.equal(st.attend(q, 0.1, strided), st.attend(q, 0.1, torch.tensor([103, 104])))
+
+
+def test_step_in_a_graph():
+    """A token step captured with host positions replays to the eager result."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(2)
+    st = kvq.KIVIState(_rows(g, 2, 2, 500, 128), _rows(g, 2, 2, 500, 128), window=64, group_k=32, group_v=32, extra=4)
+    k, v, q = _rows(g, 2, 2, 1, 128), _rows(g, 2, 2, 1, 128), _rows(g, 2, 8, 1, 128)
+    n, e = st.n, st.cache.n_exact
+
+    def step():
+        st.n, st.cache.n_exact = n, e
+        st.append(k, v, torch.tensor([500]))
+        return st.attend(q, 0.1, torch.tensor([500]))
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        step()
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for i in range(4):
+        for x in (k, v, q):
+            x.copy_(_rows(g, *x.shape))
+        graph.replay()
+        got = out.clone()
+        torch.cuda.synchronize()
+        assert torch.equal(got, step())
