@@ -16,7 +16,8 @@
 //                             contiguous quarter of it per wavefront; every wavefront streams
 //                             32-token chunks.
 //   exact window: with a one-round class plan, exact-row blocks of the same launch dispatched
-//                 after the packed blocks (they run on the slots the first class leaves free);
+//                 after the packed blocks (they run on the slots the first class leaves free), and
+//                 likewise where the packed blocks leave slots empty;
 //                 otherwise up to kFusedExact rows per packed split are attended by the packed
 //                 blocks themselves (fp32 VALU, staged in LDS with the query rows, after the
 //                 stream), longer windows of up to kExactInMerge rows by the merge, longer still
@@ -1255,6 +1256,23 @@ inline SplitPlan plan_split(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int6
   } else {
     sp.n_exact_wg = (n_exact == 0 || sp.fused_per > 0 || exact_in_merge(n_exact))
                         ? 0 : plan_exact_blocks(B * Hkv, n_exact, &sp.exact_rows);
+    // A small step leaves resident slots empty: there the window goes to exact-row blocks of the same launch
+    // (16 to 64 rows each), which run beside the packed blocks, where the fused pass runs after each
+    // block's stream (split of 2905 packed + 96 exact rows, 8 (b, h), group 32: 8 query rows 11.7 -> 9.1 us,
+    // 4 rows 8.1 -> 5.8, 1 row 5.6 -> 4.6; the packed rows alone 7.8, 5.9, 4.6).  Only while the row's partials
+    // stay within the one-wavefront merge.
+    if (sp.fused_per > 0) {
+      const int64_t slots = static_cast<int64_t>(kCUs) * resident_blocks / std::max<int64_t>((bhn + 7) / 8 * 8, 1);
+      const int64_t room = std::min<int64_t>(slots, kWaveMergePartials) - ns;
+      const int64_t nb = std::min<int64_t>(room, (n_exact + 15) / 16);
+      const int64_t rows = nb > 0 ? ((n_exact + nb - 1) / nb + 15) / 16 * 16 : 0;
+      if (rows > 0 && rows <= 64) {
+        sp.fused_per = 0;
+        sp.exact_inline = 1;
+        sp.exact_rows = static_cast<int>(rows);
+        sp.n_exact_wg = static_cast<int>((n_exact + rows - 1) / rows);
+      }
+    }
   }
   sp.S1 = sp.n_exact_wg + sp.n_split;
   return sp;

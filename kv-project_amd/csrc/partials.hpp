@@ -7,7 +7,7 @@
 //
 // One workgroup per (b, h, row): the partials are spread over all 256 threads (max and sum by
 // block reduction; the output columns by 32 channel quads x 8 partial slices), so the merge
-// costs a few dependent loads whatever the split count.  Rows with at most 32 partials and no
+// costs a few dependent loads whatever the split count.  Rows with at most 48 partials and no
 // exact rows to attend take one wavefront each instead (merge_rows_wave_kernel).
 #pragma once
 #include <algorithm>
@@ -19,6 +19,7 @@ namespace kvq {
 namespace {
 
 constexpr int kMergeThreadsEx = 256;              // threads of the merge blocks
+constexpr int kWaveMergePartials = 48;            // the most partials of a row that one wavefront merges
 
 // Exact rows (the residual window, appended tokens) a merge may attend itself instead of reading
 // their partials: rows [0, n) of k_exact / v_exact (BH, cap_e, D) in the output dtype, visible to
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(MergeArgs a) 
   }
 }
 
-// The merge of a step whose rows have at most NS (<= 32) partials and no exact rows left to attend:
+// The merge of a step whose rows have at most NS (<= 48) partials and no exact rows left to attend:
 // one wavefront per query row (four rows a workgroup, rows in the order of merge_rows_kernel's
 // grid), lane s holding partial s's (m, l) and lane l channels 2 l, 2 l + 1 of every partial's o.
 // Every load goes out at once; the row's maximum and sum are wavefront reductions, the weights
@@ -390,7 +391,7 @@ inline int pow2_rows(int64_t r) {
 // launch merge_rows_kernel for a runtime row count R (power of two <= 8) and output dtype
 inline int launch_merge_rows(const MergeArgs& a, int R, int BH, int out_dtype, hipStream_t s) {
   const int S_all = a.S_ex + a.S;
-  if (a.ex.n == 0 && S_all >= 1 && S_all <= 32) {                // one wavefront per row
+  if (a.ex.n == 0 && S_all >= 1 && S_all <= kWaveMergePartials) {   // one wavefront per row
     const int n_rows = BH * a.R_real;
     const dim3 wgrid(static_cast<unsigned>((n_rows + 3) / 4));
 #define KVQ_MW_N(R_, DT_, N_) hipLaunchKernelGGL((merge_rows_wave_kernel<R_, DT_, N_>), wgrid, dim3(256), 0, s, a, n_rows)
@@ -398,7 +399,8 @@ inline int launch_merge_rows(const MergeArgs& a, int R, int BH, int out_dtype, h
   do {                                                         \
     if (S_all <= 8) KVQ_MW_N(R_, DT_, 8);                      \
     else if (S_all <= 16) KVQ_MW_N(R_, DT_, 16);               \
-    else KVQ_MW_N(R_, DT_, 32);                                \
+    else if (S_all <= 32) KVQ_MW_N(R_, DT_, 32);               \
+    else KVQ_MW_N(R_, DT_, 48);                                \
   } while (0)
 #define KVQ_MW_R(DT_)                              \
   switch (R) {                                     \

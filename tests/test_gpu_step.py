@@ -91,3 +91,23 @@ def test_step_in_a_graph():
         got = out.clone()
         torch.cuda.synchronize()
         assert torch.equal(got, step())
+
+
+@pytest.mark.parametrize("B,Hkv,rep,Tq,T,window", [
+    (1, 1, 1, 1, 40, 8), (1, 2, 1, 1, 700, 15), (1, 3, 4, 2, 1200, 17), (2, 4, 4, 2, 3001, 96),    # exact-row blocks beside
+    (1, 8, 1, 1, 4096, 128), (1, 5, 3, 1, 3000, 250),                                             # up to 48 partials a row
+    (12, 8, 4, 1, 4096, 60), (14, 8, 2, 1, 3000, 100),                                            # in the packed blocks
+    (1, 1, 2, 1, 5000, 800),                                                                      # in the merge
+])
+def test_window_placements_match_dense_attention(B, Hkv, rep, Tq, T, window):
+    """fp32 steps over packed and exact rows, appended ones causal, wherever the plan attends the window."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(T + window)
+    f32 = torch.float32
+    st = kvq.KIVIState(_rows(g, B, Hkv, T, 128, dtype=f32), _rows(g, B, Hkv, T, 128, dtype=f32), window=window, group_k=32,
+                       group_v=32, extra=Tq)
+    st.append(_rows(g, B, Hkv, Tq, 128, dtype=f32), _rows(g, B, Hkv, Tq, 128, dtype=f32), torch.arange(T, T + Tq))
+    q = _rows(g, B, Hkv * rep, Tq, 128, dtype=f32)
+    at = torch.arange(T, T + Tq)
+    got, want = st.attend(q, 128 ** -0.5, at), st.reference_attend(q, 128 ** -0.5, at)
+    assert float((got - want).abs().max()) <= 2e-3                   # the fp32 bar of every decode

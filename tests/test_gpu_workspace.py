@@ -22,6 +22,7 @@ def _same(step, need):
 @pytest.mark.parametrize("B,Hkv,rep,Tq,T,window", [
     (1, 1, 1, 1, 33, 1), (1, 3, 3, 1, 200, 40), (2, 4, 3, 2, 1000, 96), (1, 2, 1, 5, 4000, 700),
     (1, 2, 7, 1, 3000, 2000), (16, 8, 4, 1, 2176, 128),       # 16 x 8: one round of packed blocks by class
+    (12, 8, 4, 1, 4096, 60),                                  # every slot taken: the window in the packed blocks
 ])
 def test_kivi_decode_any_workspace(dtype, B, Hkv, rep, Tq, T, window):
     import kvq
