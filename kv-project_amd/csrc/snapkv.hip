@@ -13,7 +13,7 @@
 //      keys on the matrix cores (v_mfma_f32_16x16x32_{bf16,f16}; fp32 inputs as fp16 hi + lo parts,
 //      three products), each lane keeping an online (max, sum) of its rows in base 2; partials out.
 //   2. snap_rows: each row's (max, 1 / sum) from the partials.
-//   3. snap_cols: per (bh, row group, 256-key chunk) the logits again, probabilities normalised by the
+//   3. snap_cols: per (bh, row group, key split) the logits again, probabilities normalised by the
 //      row statistics and summed over the group's rows on the way out of the accumulators.
 //   4. snap_pool: sum of the row groups' column sums / (rep * w), the pooling window through LDS,
 //      and a maximum per block.
@@ -21,6 +21,14 @@
 // Matrix-core mapping (mfma_common.hpp): A = 16 keys x 32 channels (lane l: key l%16, channels
 // 8(l/16)..+7 of the k-step), B = 32 channels x 16 query rows, D lane l register i = logit of key
 // 4(l/16) + i for row l%16.
+//
+// Both logit passes stream their split's keys through LDS (KeyStream): the four wavefronts of a workgroup hold
+// the operands of 64 rows each and share every key.  What bounds them: the exp2 of every (row, key)
+// pair at a quarter of the vector rate and the products themselves (at 4 x 8 x 65536 bf16 keys and 256 rows
+// each, 137 GFLOP and 0.54 GB a pass: statistics 154 us, columns 153, 131 without the exponentials; a large
+// library product reaches 1.26 PFLOP/s here, which is 109 us).  With each wavefront loading its tiles from
+// L2, one ahead, they took 242 and 288.  Eight wavefronts of 32 rows 153 and 157, stages of 128 keys 163
+// and 161.
 #include <algorithm>
 
 #include "common.hpp"
@@ -30,9 +38,11 @@
 namespace kvq {
 namespace {
 
-constexpr int kSnapThreads = 256;
+constexpr int kSnapThreads = 256;     // workgroups of the row, pooling and window passes
 constexpr int kSnapWaves = 4;
-constexpr int kSnapChunk = 256;       // keys of a column-sum workgroup (16 tiles)
+constexpr int kLogitWaves = 4;        // wavefronts of a logit workgroup
+constexpr int kLogitThreads = 64 * kLogitWaves;
+constexpr int kSnapResident = 2;       // workgroups of a logit pass resident on a CU
 constexpr int kSnapPool = 1024;       // keys of a pooling workgroup
 constexpr int kSnapMaxPad = 32;       // largest pooling half-width
 constexpr float kSnapLog2e = 1.4426950408889634f;
@@ -41,8 +51,9 @@ template <int DT>
 struct SnapTraits {
   static constexpr int NH = TileOps<DT>::NH;                // operand parts (fp32: fp16 hi, lo)
   static constexpr int NBW = DT == KVQ_F32 ? 2 : 4;         // row blocks of 16 per wavefront
-  static constexpr int RG = 16 * NBW * kSnapWaves;          // rows per workgroup
+  static constexpr int RG = 16 * NBW * kLogitWaves;         // rows per workgroup
   static constexpr int ESZ = TileOps<DT>::ESZ;
+  static constexpr int KT = 64 / NH;                        // keys of a stage
 };
 
 struct SnapParams {
@@ -50,10 +61,10 @@ struct SnapParams {
   int64_t q_sb, q_sh, q_st;             // window query rows: (b, head, i) at b*q_sb + head*q_sh + i*q_st
   const void* k;
   int64_t k_sb, k_sh, k_st;             // keys: (b, h, j) at b*k_sb + h*k_sh + j*k_st
-  int Hkv, rep, w, H, rows, n_rg, n_split, split_keys, n_chunk, n_pool, kernel;
+  int BH, Hkv, rep, w, H, rows, n_rg, n_split, split_keys, n_pool, kernel;
   float qscale;                         // scaling * log2(e)
   float inv_count;                      // 1 / (rep * w)
-  float* part_m;                        // (BH, n_split, rows)
+  float* part_m;                        // (BH, rows, n_split)
   float* part_l;
   float* row_m;                         // (BH, rows)
   float* row_il;                        // (BH, rows): 1 / row sum
@@ -104,25 +115,97 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t key_rsrc(const SnapParams& p, 
   return make_rsrc(base, static_cast<uint32_t>((static_cast<int64_t>(p.H - 1) * p.k_st + 128) * esz));
 }
 
-// the A/B operand registers of key kj (channels 32 ks + 8 g .. + 7 of each k-step); keys past the
-// resource's range read as zeros
+// The keys of a split in stages of KT, double-buffered in LDS: the loads of a stage go out two stages before
+// it is computed (into registers, so that they wait for nothing else), and each 16-byte piece (8
+// channels of a key, converted to operand parts where the keys are fp32) is written to LDS once for
+// the four wavefronts.  Piece c of key j lies at column c ^ (j % 16) of its row, which puts the 16 keys of
+// an operand read on different banks.  Keys past H repeat the last one (their logits are masked).
 template <int DT>
-__device__ __forceinline__ void load_keys(const __amdgpu_buffer_rsrc_t& rk, const SnapParams& p, int kj, int g,
-                                          u32x4 (&kop)[4][SnapTraits<DT>::NH]) {
+struct KeyStream {
+  using T = SnapTraits<DT>;
+  static constexpr int UNITS = T::KT * 16 / kLogitThreads;   // pieces of a thread and stage
+  u32x4 (*lds)[T::NH][T::KT * 16];                          // [2][NH][KT 16]
+  __amdgpu_buffer_rsrc_t rk;
+  int64_t st;
+  int last;                                                 // H - 1
+  float xs;
+  u32x4 reg[2][UNITS][T::NH];                               // 8 channels: 16 bytes, or 32 of fp32
+
+  __device__ __forceinline__ void load(int k0, u32x4 (&r)[UNITS][T::NH]) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    load_op_buf<DT>(rk, static_cast<int>((static_cast<int64_t>(kj) * p.k_st + 32 * ks + 8 * g) * SnapTraits<DT>::ESZ),
-                    kop[ks], snap_xs<DT>(p, 1));
+    for (int u = 0; u < UNITS; ++u) {
+      const int id = threadIdx.x + kLogitThreads * u;
+      const int off = static_cast<int>((min(k0 + id / 16, last) * st + 8 * (id % 16)) * T::ESZ);
+#pragma unroll
+      for (int e = 0; e < T::NH; ++e) r[u][e] = __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16 * e, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void store(int buf, const u32x4 (&r)[UNITS][T::NH]) {
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int id = threadIdx.x + kLogitThreads * u;
+      const int at = (id / 16) * 16 + ((id % 16) ^ (id / 16 % 16));
+      if constexpr (DT == KVQ_F32) {
+        float x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = __uint_as_float(r[u][k / 4][k % 4]) * xs;
+        u32x4 hi, lo;
+        f32_parts<DT>(x, hi, lo);
+        lds[buf][0][at] = hi;
+        lds[buf][1][at] = lo;
+      } else {
+        lds[buf][0][at] = r[u][0];
+      }
+    }
+  }
+  // the operand of the 16 keys from 16 tt of the stage in buf
+  __device__ __forceinline__ void operand(int buf, int tt, int g, int n, u32x4 (&kop)[4][T::NH]) const {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int hh = 0; hh < T::NH; ++hh) kop[ks][hh] = lds[buf][hh][(16 * tt + n) * 16 + ((4 * ks + g) ^ n)];
+  }
+  // stage(k, buf) for every stage of [k0, k1), its keys in LDS buffer buf; a barrier lies before each call
+  template <class F>
+  __device__ __forceinline__ void run(int k0, int k1, F stage) {
+    load(k0, reg[0]);
+    load(k0 + T::KT, reg[1]);
+    store(0, reg[0]);
+    block_lds_barrier();
+    for (int k = k0; k < k1; k += 2 * T::KT) {
+      load(k + 2 * T::KT, reg[0]);
+      stage(k, 0);
+      store(1, reg[1]);
+      block_lds_barrier();
+      if (k + T::KT >= k1) break;
+      load(k + 3 * T::KT, reg[1]);
+      stage(k + T::KT, 1);
+      store(0, reg[0]);
+      block_lds_barrier();
+    }
+  }
+};
+
+// (bh, row group, split) of a workgroup: the row groups of one split go to one XCD, which reads its keys once
+__device__ __forceinline__ bool snap_unit(const SnapParams& p, int* bh, int* rg, int* s) {
+  const int k = blockIdx.x / 8;
+  const int unit = (k / p.n_rg) * 8 + blockIdx.x % 8;
+  *rg = k % p.n_rg;
+  *bh = unit / p.n_split;
+  *s = unit % p.n_split;
+  return *bh < p.BH;
 }
 
+constexpr float kSnapNone = -3.0e38f;   // no logit yet (finite, so that a first logit of -inf stays a zero term)
+constexpr float kSnapLazy = 8.0f;       // a row's reference is moved when a logit exceeds it by this many octaves
+
 template <int DT>
-__global__ __launch_bounds__(kSnapThreads) void snap_stats(SnapParams p) {
+__global__ __launch_bounds__(kLogitThreads, 2) void snap_stats(SnapParams p) {
   using T = SnapTraits<DT>;
+  __shared__ u32x4 keys[2][T::NH][T::KT * 16];
   const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
-  int id = blockIdx.x;
-  const int s = id % p.n_split;
-  id /= p.n_split;
-  const int rg = id % p.n_rg, bh = id / p.n_rg;
+  int bh, rg, s;
+  if (!snap_unit(p, &bh, &rg, &s)) return;
   const int b = bh / p.Hkv, h = bh % p.Hkv;
   u32x4 qop[T::NBW][4][T::NH];
   int rowpos[T::NBW], row[T::NBW];
@@ -130,86 +213,90 @@ __global__ __launch_bounds__(kSnapThreads) void snap_stats(SnapParams p) {
   float m[T::NBW], ls[T::NBW];
 #pragma unroll
   for (int bw = 0; bw < T::NBW; ++bw) {
-    m[bw] = -INFINITY;
+    m[bw] = kSnapNone;
     ls[bw] = 0.0f;
   }
-  const __amdgpu_buffer_rsrc_t rk = key_rsrc(p, b, h, T::ESZ);
   const int k0 = s * p.split_keys, k1 = min(k0 + p.split_keys, p.H);
+  const int open = min(k1, p.H - p.w + 1);     // keys below it are in the split and visible to every row
   const float qsc = p.qscale / (snap_xs<DT>(p, 0) * snap_xs<DT>(p, 1));   // logit scale of the scaled rows
-  auto stat_tile = [&](int t0, const u32x4 (&kop)[4][T::NH]) {
+  KeyStream<DT> ks{keys, key_rsrc(p, b, h, T::ESZ), p.k_st, p.H - 1, snap_xs<DT>(p, 1)};
+  ks.run(k0, k1, [&](int k, int buf) {
 #pragma unroll
-    for (int bw = 0; bw < T::NBW; ++bw) {
-      const f32x4 acc = tile_dots<DT, SnapTraits<DT>::NH, SnapTraits<DT>::NH>(kop, qop[bw]);
-      float sv[4];
-      float mt = -INFINITY;
+    for (int tt = 0; tt < T::KT / 16; ++tt) {
+      const int t0 = k + 16 * tt;
+      if (t0 >= k1) break;
+      u32x4 kop[4][T::NH];
+      ks.operand(buf, tt, g, n, kop);
+      f32x4 acc[T::NBW];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = t0 + 4 * g + i;
-        sv[i] = (j < k1 && j <= rowpos[bw]) ? acc[i] * qsc : -INFINITY;
-        mt = fmaxf(mt, sv[i]);
+      for (int bw = 0; bw < T::NBW; ++bw) acc[bw] = tile_dots<DT, T::NH, T::NH>(kop, qop[bw]);
+      const bool edge = t0 + 16 > open;        // the split's end, or keys that some rows do not see
+      const float f = edge ? 1.0f : qsc;       // logit = f acc
+      if (edge) {
+#pragma unroll
+        for (int bw = 0; bw < T::NBW; ++bw)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int j = t0 + 4 * g + i;
+            acc[bw][i] = (j < k1 && j <= rowpos[bw]) ? acc[bw][i] * qsc : -INFINITY;
+          }
       }
-      if (mt > m[bw]) {
-        ls[bw] *= __builtin_amdgcn_exp2f(m[bw] - mt);
-        m[bw] = mt;
-      }
-      if (m[bw] != -INFINITY) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ls[bw] += __builtin_amdgcn_exp2f(sv[i] - m[bw]);
+      for (int bw = 0; bw < T::NBW; ++bw) {
+        float a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = __builtin_fmaf(acc[bw][i], f, -m[bw]);
+        const float top = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
+        if (__any(top > kSnapLazy)) {
+          const float mn = fmaxf(m[bw], fmaxf(fmaxf(acc[bw][0] * f, acc[bw][1] * f), fmaxf(acc[bw][2] * f, acc[bw][3] * f)));
+          ls[bw] *= __builtin_amdgcn_exp2f(m[bw] - mn);
+          m[bw] = mn;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) a[i] = __builtin_fmaf(acc[bw][i], f, -mn);
+        }
+        ls[bw] += (__builtin_amdgcn_exp2f(a[0]) + __builtin_amdgcn_exp2f(a[1])) +
+                  (__builtin_amdgcn_exp2f(a[2]) + __builtin_amdgcn_exp2f(a[3]));
       }
     }
-  };
-  // two key tiles in registers used in turn: the next tile's loads are issued before the current
-  // one is computed (tiles past the split are loaded -- keys past H read as zeros -- never used)
-  if (k0 < k1) {
-    u32x4 ka[4][T::NH], kb[4][T::NH];
-    load_keys<DT>(rk, p, k0 + n, g, ka);
-    for (int t0 = k0;; t0 += 32) {
-      load_keys<DT>(rk, p, t0 + 16 + n, g, kb);
-      stat_tile(t0, ka);
-      if (t0 + 16 >= k1) break;
-      load_keys<DT>(rk, p, t0 + 32 + n, g, ka);
-      stat_tile(t0 + 16, kb);
-      if (t0 + 32 >= k1) break;
-    }
-  }
+  });
   // the four lanes of a row (xor 16, xor 32) hold disjoint keys of it
 #pragma unroll
   for (int bw = 0; bw < T::NBW; ++bw) {
     const float M = xmax32(xmax16(m[bw]));
-    const float part = (M == -INFINITY || m[bw] == -INFINITY) ? 0.0f : ls[bw] * __builtin_amdgcn_exp2f(m[bw] - M);
-    const float L = xsum32(xsum16(part));
+    const float L = xsum32(xsum16(ls[bw] * __builtin_amdgcn_exp2f(m[bw] - M)));
     if (g == 0 && row[bw] < p.rows) {
-      const int64_t o = (static_cast<int64_t>(bh) * p.n_split + s) * p.rows + row[bw];
+      const int64_t o = (static_cast<int64_t>(bh) * p.rows + row[bw]) * p.n_split + s;
       p.part_m[o] = M;
       p.part_l[o] = L;
     }
   }
 }
 
+// 16 lanes a row, each over every 16th split
 __global__ __launch_bounds__(kSnapThreads) void snap_rows(SnapParams p, int64_t n_rows_all) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kSnapThreads + threadIdx.x;
-  if (t >= n_rows_all) return;
-  const int64_t bh = t / p.rows, r = t % p.rows;
-  float M = -INFINITY;
-  for (int s = 0; s < p.n_split; ++s) M = fmaxf(M, p.part_m[(bh * p.n_split + s) * p.rows + r]);
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * (kSnapThreads / 16) + threadIdx.x / 16;
+  const int lane = threadIdx.x % 16;
+  const int64_t at = (t < n_rows_all ? t : n_rows_all - 1) * p.n_split;
+  float M = kSnapNone;
+  for (int s = lane; s < p.n_split; s += 16) M = fmaxf(M, p.part_m[at + s]);
+  M = row_max16(M);
   float L = 0.0f;
-  for (int s = 0; s < p.n_split; ++s) {
-    const float ms = p.part_m[(bh * p.n_split + s) * p.rows + r];
-    if (ms != -INFINITY) L += p.part_l[(bh * p.n_split + s) * p.rows + r] * __builtin_amdgcn_exp2f(ms - M);
+  for (int s = lane; s < p.n_split; s += 16) L += p.part_l[at + s] * __builtin_amdgcn_exp2f(p.part_m[at + s] - M);
+  L = row_sum16(L);
+  if (lane == 0 && t < n_rows_all) {
+    p.row_m[t] = M;
+    p.row_il[t] = 1.0f / L;               // key 0 is visible to every row: L > 0
   }
-  p.row_m[t] = M;
-  p.row_il[t] = 1.0f / L;                 // key 0 is visible to every row: L >= 1
 }
 
 template <int DT>
-__global__ __launch_bounds__(kSnapThreads) void snap_cols(SnapParams p) {
+__global__ __launch_bounds__(kLogitThreads, 2) void snap_cols(SnapParams p) {
   using T = SnapTraits<DT>;
-  __shared__ float cols[kSnapWaves][kSnapChunk];
+  __shared__ u32x4 keys[2][T::NH][T::KT * 16];
+  __shared__ float cols[2][kLogitWaves][T::KT];
   const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
-  int id = blockIdx.x;
-  const int c = id % p.n_chunk;
-  id /= p.n_chunk;
-  const int rg = id % p.n_rg, bh = id / p.n_rg;
+  int bh, rg, s;
+  if (!snap_unit(p, &bh, &rg, &s)) return;
   const int b = bh / p.Hkv, h = bh % p.Hkv;
   u32x4 qop[T::NBW][4][T::NH];
   int rowpos[T::NBW], row[T::NBW];
@@ -229,42 +316,44 @@ __global__ __launch_bounds__(kSnapThreads) void snap_cols(SnapParams p) {
       ril[bw][i] = ok ? p.row_il[static_cast<int64_t>(bh) * p.rows + r] : 0.0f;
     }
   }
-  const __amdgpu_buffer_rsrc_t rk = key_rsrc(p, b, h, T::ESZ);
   const int nc = p.H - p.w;                 // scored keys: every window row sees all of them
-  const int c0 = c * kSnapChunk;
+  const int k0 = s * p.split_keys, k1 = min(k0 + p.split_keys, nc);
   const float qsc = p.qscale / (snap_xs<DT>(p, 0) * snap_xs<DT>(p, 1));   // logit scale of the scaled rows
-  auto col_tile = [&](int tt, const u32x4 (&kop)[4][T::NH]) {
-    const int t0 = c0 + 16 * tt;
-    float colv = 0.0f;
-    if (t0 < nc) {
-#pragma unroll
-      for (int bw = 0; bw < T::NBW; ++bw) {
-        const f32x4 acc = tile_dots<DT, SnapTraits<DT>::NH, SnapTraits<DT>::NH>(qop[bw], kop);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) colv += __builtin_amdgcn_exp2f(acc[i] * qsc - rm[bw][i]) * ril[bw][i];
-      }
+  float* const dst = p.colsum + (static_cast<int64_t>(bh) * p.n_rg + rg) * nc;
+  // the wavefronts' sums of a stage meet behind the next barrier
+  auto flush = [&](int k, int buf) {
+    if (threadIdx.x < T::KT && k + static_cast<int>(threadIdx.x) < k1) {
+      const int t = threadIdx.x;
+      dst[k + t] = (cols[buf][0][t] + cols[buf][1][t]) + (cols[buf][2][t] + cols[buf][3][t]);
     }
-    // the four lane groups hold disjoint rows of key t0 + n
-    colv = xsum32(xsum16(colv));
-    if (g == 0) cols[wave][16 * tt + n] = colv;
   };
-  // two key tiles in registers used in turn, the next one's loads issued first
-  {
-    u32x4 ka[4][T::NH], kb[4][T::NH];
-    load_keys<DT>(rk, p, c0 + n, g, ka);
-    for (int tt = 0; tt < kSnapChunk / 16; tt += 2) {
-      load_keys<DT>(rk, p, c0 + 16 * (tt + 1) + n, g, kb);
-      col_tile(tt, ka);
-      if (tt + 2 < kSnapChunk / 16) load_keys<DT>(rk, p, c0 + 16 * (tt + 2) + n, g, ka);
-      col_tile(tt + 1, kb);
+  if (k0 >= k1) return;
+  KeyStream<DT> ks{keys, key_rsrc(p, b, h, T::ESZ), p.k_st, p.H - 1, snap_xs<DT>(p, 1)};
+  int done = -1, done_buf = 0;
+  ks.run(k0, k1, [&](int k, int buf) {
+    if (done >= 0) flush(done, done_buf);
+#pragma unroll
+    for (int tt = 0; tt < T::KT / 16; ++tt) {
+      if (k + 16 * tt >= k1) break;
+      u32x4 kop[4][T::NH];
+      ks.operand(buf, tt, g, n, kop);
+      f32x4 acc[T::NBW];
+#pragma unroll
+      for (int bw = 0; bw < T::NBW; ++bw) acc[bw] = tile_dots<DT, T::NH, T::NH>(qop[bw], kop);
+      float colv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int bw = 0; bw < T::NBW; ++bw)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          colv[i] = __builtin_fmaf(__builtin_amdgcn_exp2f(__builtin_fmaf(acc[bw][i], qsc, -rm[bw][i])), ril[bw][i], colv[i]);
+      // the four lane groups hold disjoint rows of key t0 + n
+      const float v = xsum32(xsum16((colv[0] + colv[1]) + (colv[2] + colv[3])));
+      if (g == 0) cols[buf][wave][16 * tt + n] = v;
     }
-  }
-  __syncthreads();
-  const int j = c0 + threadIdx.x;
-  if (j < nc) {
-    const float v = (cols[0][threadIdx.x] + cols[1][threadIdx.x]) + (cols[2][threadIdx.x] + cols[3][threadIdx.x]);
-    p.colsum[(static_cast<int64_t>(bh) * p.n_rg + rg) * nc + j] = v;
-  }
+    done = k;
+    done_buf = buf;
+  });
+  flush(done, done_buf);                    // run() ends behind a barrier
 }
 
 __global__ __launch_bounds__(kSnapThreads) void snap_pool(SnapParams p) {
@@ -318,20 +407,20 @@ __global__ __launch_bounds__(kSnapThreads) void snap_window(SnapParams p, int n_
 }
 
 struct SnapPlan {
-  int n_rg, n_split, split_keys, n_chunk, n_pool;
+  int n_rg, n_split, split_keys, n_pool;
 };
 
 SnapPlan snap_plan(int64_t BH, int64_t rows, int64_t w, int64_t H, int dtype) {
   SnapPlan sp{};
   const int64_t RG = dtype == KVQ_F32 ? SnapTraits<KVQ_F32>::RG : SnapTraits<KVQ_BF16>::RG;
+  const int64_t KT = dtype == KVQ_F32 ? SnapTraits<KVQ_F32>::KT : SnapTraits<KVQ_BF16>::KT;
   sp.n_rg = static_cast<int>((rows + RG - 1) / RG);
-  // about 1024 workgroups of key splits, whole 16-key tiles
-  const int64_t want = std::max<int64_t>(1, (1024 + BH * sp.n_rg - 1) / (BH * sp.n_rg));
-  const int64_t tiles = (H + 15) / 16;
-  const int64_t ns = std::min<int64_t>(want, tiles);
-  sp.split_keys = static_cast<int>(((tiles + ns - 1) / ns) * 16);
+  // one round of resident workgroups (kSnapResident a CU) of key splits, whole stages
+  const int64_t want = std::max<int64_t>(1, 256 * kSnapResident / (BH * sp.n_rg));
+  const int64_t stages = (H + KT - 1) / KT;
+  const int64_t ns = std::min<int64_t>(want, stages);
+  sp.split_keys = static_cast<int>(((stages + ns - 1) / ns) * KT);
   sp.n_split = static_cast<int>((H + sp.split_keys - 1) / sp.split_keys);
-  sp.n_chunk = static_cast<int>((H - w + kSnapChunk - 1) / kSnapChunk);
   sp.n_pool = static_cast<int>((H - w + kSnapPool - 1) / kSnapPool);
   return sp;
 }
@@ -384,7 +473,7 @@ extern "C" int kvq_snapkv_scores(const void* q, int dtype, int64_t q_sb, int64_t
   p.k = k; p.k_sb = k_sb; p.k_sh = k_sh; p.k_st = k_st;
   p.Hkv = static_cast<int>(Hkv); p.rep = static_cast<int>(Hq / Hkv); p.w = static_cast<int>(window);
   p.H = static_cast<int>(H); p.rows = static_cast<int>(rows);
-  p.n_rg = sp.n_rg; p.n_split = sp.n_split; p.split_keys = sp.split_keys; p.n_chunk = sp.n_chunk;
+  p.BH = static_cast<int>(BH); p.n_rg = sp.n_rg; p.n_split = sp.n_split; p.split_keys = sp.split_keys;
   p.n_pool = sp.n_pool; p.kernel = kernel;
   p.qscale = scaling * kSnapLog2e;
   p.inv_count = 1.0f / static_cast<float>(rows);
@@ -397,7 +486,7 @@ extern "C" int kvq_snapkv_scores(const void* q, int dtype, int64_t q_sb, int64_t
   p.blockmax = ws; ws += BH * sp.n_pool;
   p.out = out;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 blk(kSnapThreads);
+  const dim3 blk(kSnapThreads), logit(kLogitThreads), units(static_cast<unsigned>((BH * sp.n_split + 7) / 8 * 8 * sp.n_rg));
   if (dtype == KVQ_F32) {
     // the powers of two that bring the window's query rows and the keys into the fp16 parts' range
     p.xs = ws + kAmaxViews * kAmaxBlocks;
@@ -409,11 +498,11 @@ extern "C" int kvq_snapkv_scores(const void* q, int dtype, int64_t q_sb, int64_t
     launch_rows_scales(views, 2, ws, const_cast<float*>(p.xs), s);
     KVQ_LAUNCH_CHECK("kvq_snapkv_scores(fp32 scales)");
   }
-  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((snap_stats<DT_>), dim3(BH * sp.n_rg * sp.n_split), blk, 0, s, p));
+  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((snap_stats<DT_>), units, logit, 0, s, p));
   KVQ_LAUNCH_CHECK("kvq_snapkv_scores(stats)");
-  hipLaunchKernelGGL(snap_rows, dim3((BH * rows + kSnapThreads - 1) / kSnapThreads), blk, 0, s, p, BH * rows);
+  hipLaunchKernelGGL(snap_rows, dim3((BH * rows + kSnapThreads / 16 - 1) / (kSnapThreads / 16)), blk, 0, s, p, BH * rows);
   KVQ_LAUNCH_CHECK("kvq_snapkv_scores(rows)");
-  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((snap_cols<DT_>), dim3(BH * sp.n_rg * sp.n_chunk), blk, 0, s, p));
+  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((snap_cols<DT_>), units, logit, 0, s, p));
   KVQ_LAUNCH_CHECK("kvq_snapkv_scores(cols)");
   hipLaunchKernelGGL(snap_pool, dim3(BH * sp.n_pool), blk, 0, s, p);
   KVQ_LAUNCH_CHECK("kvq_snapkv_scores(pool)");

@@ -214,8 +214,8 @@ def exact_rows_cache(k_exact: torch.Tensor, v_exact: torch.Tensor, n_exact: int,
     are minimal placeholders the decode never reads (it reads no packed row when n_q = 0)."""
     B, H, _, d = k_exact.shape
     dev = k_exact.device
-    z8 = lambda *s: torch.zeros(s, dtype=torch.uint8, device=dev)
-    z16 = lambda *s: torch.zeros(s, dtype=torch.float16, device=dev)
+    z8 = lambda *s: torch.empty(s, dtype=torch.uint8, device=dev)
+    z16 = lambda *s: torch.empty(s, dtype=torch.float16, device=dev)
     return PackedKIVICache(z8(B, H, 64, d // 2), z16(B, H, 1, d), z16(B, H, 1, d), z8(B, H, 2, 16 * d),
                            z16(B, H, 2, d // 64, 32, 2), 0, 64, 64, k_exact, v_exact, n_exact, exact_pos)
 

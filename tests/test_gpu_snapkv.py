@@ -48,6 +48,25 @@ def test_snapkv_scores_match_oracle(B, Hq, Hkv, H, w, kern, dtype):
     np.testing.assert_allclose(got[..., H - w:], want[..., H - w:], rtol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,H,w,scaling,ramp", [
+    (1, 1, 1, 65, 64, 0.09, 0.0),                   # one scored key
+    (1, 3, 1, 139, 10, 0.09, 0.0),                  # 30 rows, a split that ends inside a stage and a tile
+    (3, 6, 1, 128 + 64, 64, 0.09, 0.0),             # 384 rows; the window starts a stage
+    (2, 8, 2, 1000, 33, 0.09, 0.02),                # keys that grow: a row's reference moves again and again
+    (1, 4, 4, 3000, 64, -0.09, 0.005),              # negative and zero scalings
+    (1, 4, 2, 400, 64, 0.0, 0.0),
+])
+def test_snapkv_scores_edges(B, Hq, Hkv, H, w, scaling, ramp, dtype):
+    import kvq
+    q, k = _case(B, Hq, Hkv, H, 128, dtype, seed=H)
+    k = (k.float() * (1.0 + ramp * torch.arange(H + 3.0)[:, None])).to(dtype)
+    cfg = SimpleNamespace(SNAPKV_WINDOW=w, SNAPKV_KERNEL=5)
+    got = kvq.snapkv_scores(q.cuda(), k.cuda(), H, scaling, cfg).cpu().numpy()
+    want = oracle_snapkv(q.double().numpy(), k.double().numpy(), H, scaling, w, 5)
+    np.testing.assert_allclose(got[..., :H - w], want[..., :H - w], rtol=1e-4, atol=1e-7 * want[..., :H - w].max())
+
+
 @pytest.mark.parametrize("qs,ks", [(2.0 ** -17, 2.0 ** 17), (2.0 ** 20, 2.0 ** -20), (2.0 ** -122, 1.0)])
 def test_snapkv_scores_fp32_extreme_magnitudes(qs, ks):
     """fp32 keys past fp16's range (~5e5) or far below it (~4e-6), queries scaled the other way so
