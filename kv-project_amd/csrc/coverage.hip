@@ -12,14 +12,16 @@
 // Rows are laid out per KV head as [group][query head r][query, padded to 16] (row_base of a group in
 // the group table); padded rows have position -1 and contribute nothing.  Launches (one stream, no
 // host synchronisation, no atomics: every sum has a fixed order):
-//   cov_attend    per (h, row blocks, range of keys): logits of 16-key tiles on the matrix cores
-//                 (row_tiles.hpp), p = 2^(s - reference) in registers as the A operand of the PV product
-//                 (hi + lo parts; the two 16-key tiles of a 32-key step give every lane 8 keys of its
-//                 row, in an order the B operand follows), B = values of the step from an LDS tile;
-//                 the range's part of o, reference and sum, fp32.
-//   cov_metric    o M and o M o of the row outputs (the key ranges' parts combined in order), 32 rows per
-//                 workgroup with the query head's metric staged in LDS.
-//   cov_vmv       v M v of the coded values on the matrix cores.
+//   cov_rowstats  per (group, 64-row block, h): logits of 16-key tiles on the matrix cores
+//                 (row_tiles.hpp), online max / sum per row -> row max (base 2) and 1 / sum; every
+//                 key tile feeds all the block's rows a wavefront holds, the wavefronts split the keys.
+//   cov_output    per (group, 64-row block, h, key split): the logits again, p = 2^(s - max) / sum in
+//                 registers as the A operand of the PV product (hi + lo parts; the two 16-key tiles
+//                 of a 32-key step give every lane 8 keys of its row, in an order the B operand
+//                 follows), B = values of the step from an LDS tile; the split's part of o, fp32.
+//   cov_metric    x M and x M x for 32 vectors per workgroup with the query head's metric staged in
+//                 LDS: the row outputs (the key splits' parts summed in order; o M) and the coded
+//                 values (v M v).
 //   cov_rowprep   the rows' operands and values as records of 16 rows, in the order cov_terms reads.
 //   cov_terms     per (h, chunk of tokens, piece of the groups reaching it): logits and v.(oM) on the
 //                 matrix cores, then the per-(row, token) terms, once: the group's drop total, every
@@ -31,7 +33,6 @@
 //   cov_smat      S = sum over rows of weight * alpha * (scaling q)(scaling q)^T.
 //   cov_final     live average, S / sum_j A_j, Mbar, floors (one workgroup for the sums, then all).
 #include <algorithm>
-#include <climits>
 
 #include "common.hpp"
 #include "mfma_common.hpp"
@@ -47,7 +48,7 @@ constexpr int kTW = 4;                   // wavefronts of a cov_terms workgroup
 constexpr int kChunkTok = 32 * kTW;      // its tokens: two 16-token tiles per wavefront
 constexpr int kGT = 8;                  // ints per group-table entry
 constexpr int kMetricRows = 32;         // vectors of a cov_metric workgroup
-constexpr int kOSplit = 8;              // key ranges of cov_attend
+constexpr int kOSplit = 4;              // key splits of cov_output (workgroups per 64-row item)
 constexpr int kRowPart = 20;            // its rows' key-term masses, its read mass in four parts
 constexpr int kTermsUnits = 1536;       // workgroups of cov_terms worth cutting the groups of a chunk for
 constexpr int64_t kStoreFloats = int64_t{1} << 28;   // most floats of the stored token sums (1 GiB)
@@ -59,19 +60,18 @@ struct CovParams {
   const void* qr;                        // (Hkv, NR, d) group query rows (unscaled), DT
   const int32_t* rowpos;                 // (NR): position of each row (-1: padding)
   const int32_t* gtab;                   // (G, kGT)
+  const int32_t* items;                  // (n_items, 2): (group, 64-row block)
   const void* k;
   const void* v;
   int64_t k_sh, k_st, v_sh, v_st;        // element strides of the (head, token) axes
   const float* M;                        // (Hq, d, d)
-  int Hkv, rep, NR, G, rs, re, n, n_chunks, T;
+  int Hkv, rep, NR, G, n_items, rs, re, n, n_chunks, T;
   float qscale;                          // scaling * log2(e)
   float scaling, eta;
-  const int32_t* rowgrp;                 // (NR): group of each row
-  float* ml;                             // (kOSplit, Hkv, NR, 2): reference (base 2) and sum of a row over a key range
-  float* row_m;                          // (Hkv, NR) row reference (base 2)
+  float* row_m;                          // (Hkv, NR) row max (base 2)
   float* row_il;                         // (Hkv, NR) 1 / row sum
   float* o;                              // (Hkv, NR, d) o M (cov_metric over the summed outputs)
-  float* o_part;                         // (kOSplit, Hkv, NR, d) unnormalised fp32 outputs of each key range
+  float* o_part;                         // (kOSplit, Hkv, NR, d) fp32 outputs of each key split
   float* oMo;                            // (Hkv, NR)
   uint32_t* rec;                         // (Hkv, NR / 16) records of cov_terms (rec_units<DT> u32x4)
   float* vmv;                            // (Hkv, rep, n)
@@ -151,241 +151,269 @@ __device__ __forceinline__ void load_tile(__amdgpu_buffer_rsrc_t rs, int64_t st,
     load_op_buf<DT>(rs, static_cast<int>((tok * st + 32 * ks + 8 * g) * TileOps<DT>::ESZ), op[ks], sc);
 }
 
-// The rows' attention outputs in one pass over the keys: per (h, eight or four 16-row blocks, range of
-// the keys) a wavefront holds NRB row blocks, the workgroup's 32-key steps of K and V come through LDS
-// (two stages, loads one more step ahead; fp32 rows as their fp16 parts), and every key tile and value
-// operand read from LDS feeds all the wavefront's rows.  A row's reference exponent moves only when a
-// logit exceeds it by 2^8, so the accumulators are rescaled a few times per row and the running
-// maximum costs one vote a step.  Partials (unnormalised outputs, reference and sum) per range, combined
-// by cov_metric.  The ranges are cut at the same keys for every block, so the workgroups of a range,
-// neighbours on one XCD, share its keys in L2.
-// Bound by the matrix cores (P enters as hi + lo parts) and the exponentials and splits beside them, two
-// wavefronts per SIMD (8 heads x 264 row blocks, 32768 bf16 keys: 530 us; one row block per wavefront at
-// three per SIMD, twice the LDS and L2 reads: 534; the two passes before -- row statistics, then
-// outputs with the final maximum, key tiles from L2 per wavefront -- 288 + 1046).
+// Every key tile a wavefront loads feeds several of the item's 16-row blocks (16-bit data: all four,
+// eight wavefronts (two per SIMD) splitting the keys in eighths; fp32 operands take twice the
+// registers: two blocks, four wavefronts in halves), so the workgroup reads its keys once instead of
+// once per row block.  The wavefronts' states of a row meet in LDS, split by split in a fixed order.
+// The items go in reverse plan order: the groups at the end of the context, whose keys reach
+// furthest, start first.
 template <int DT>
-constexpr int attend_rb() { return DT == KVQ_F32 ? 1 : 2; }    // row blocks per wavefront
-constexpr float kRefNone = -3e38f;       // reference of a row before its first key
-constexpr float kRefLazy = 8.0f;         // powers of two a logit may exceed the reference by
-
-// keys of a range: an equal share of the longest reach, whole steps
-__device__ __forceinline__ int key_range(const CovParams& p) {
-  int reach = 1;
-  for (int x = threadIdx.x % 64; x < p.G; x += 64) reach = max(reach, p.gtab[kGT * x + 3]);
+__global__ __launch_bounds__(DT == KVQ_F32 ? kCThreads : 2 * kCThreads) void cov_rowstats(CovParams p) {
+  constexpr int NH = TileOps<DT>::NH;
+  constexpr int NW = DT == KVQ_F32 ? kCWaves : 2 * kCWaves;  // wavefronts (16-bit: two per SIMD)
+  constexpr int NRB = DT == KVQ_F32 ? 2 : 4;                 // row blocks per wavefront
+  constexpr int KS = NW * NRB / 4;                           // key splits (wavefronts sharing blocks)
+  __shared__ float st[NW][NRB][16][2];
+  const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
+  const int unit = xcd_unit(p.Hkv * p.n_items);                // (h, item), h outermost
+  if (unit < 0) return;
+  const int item = p.n_items - 1 - unit % p.n_items, h = unit / p.n_items;
+  const int grp = p.items[2 * item], rb = p.items[2 * item + 1];
+  const int32_t* gt = p.gtab + kGT * grp;
+  const int rows_g = p.rep * gt[2];
+  const int mmax = gt[3];
+  const int ks = wave % KS, rgrp = wave / KS;
+  u32x4 qop[NRB][4][NH];
+  int pos[NRB];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) reach = max(reach, __shfl_xor(reach, o, 64));
-  return __builtin_amdgcn_readfirstlane((reach + 32 * kOSplit - 1) / (32 * kOSplit) * 32);
+  for (int b = 0; b < NRB; ++b) {
+    const int rl = 64 * rb + 16 * (rgrp * NRB + b);           // first row of the block in the group
+    if (rl < rows_g) {
+      pos[b] = load_rows<DT>(p, h, gt[0] + rl, g, n, qop[b]);
+    } else {
+      pos[b] = -1;
+      zero_ops<DT>(qop[b]);
+    }
+  }
+  // this split's keys: whole 16-key tiles
+  const int ntile = (mmax + 15) / 16;
+  const int k0 = 16 * (ntile * ks / KS), k1 = min(mmax, 16 * (ntile * (ks + 1) / KS));
+  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k, p.k_sh, p.k_st, h, p.T, TileOps<DT>::ESZ);
+  const float qsc = p.qscale / (cov_xs<DT>(p, 0) * cov_xs<DT>(p, 1));   // logit scale of the scaled rows
+  float m[NRB], ls[NRB];
+#pragma unroll
+  for (int b = 0; b < NRB; ++b) {
+    m[b] = -INFINITY;
+    ls[b] = 0.0f;
+  }
+  // three key tiles in rotation: two in flight behind the one computed (a tile past the split reads
+  // zeros through the buffer resource or in-range keys, masked or never computed)
+  u32x4 kt[3][4][NH];
+  load_tile<DT>(rk, p.k_st, k0, g, n, kt[0], cov_xs<DT>(p, 1));
+  load_tile<DT>(rk, p.k_st, k0 + 16, g, n, kt[1], cov_xs<DT>(p, 1));
+  auto tile = [&](int t0, const u32x4 (&kop)[4][NH]) {
+#pragma unroll
+    for (int b = 0; b < NRB; ++b) {
+      const f32x4 d = tile_dots<DT, NH, NH>(kop, qop[b]);
+      float sv[4], mt = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = t0 + 4 * g + i;
+        sv[i] = (j <= pos[b] && j < mmax) ? d[i] * qsc : -INFINITY;
+        mt = fmaxf(mt, sv[i]);
+      }
+      if (mt > m[b]) {
+        ls[b] *= __builtin_amdgcn_exp2f(m[b] - mt);
+        m[b] = mt;
+      }
+      if (m[b] != -INFINITY) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ls[b] += __builtin_amdgcn_exp2f(sv[i] - m[b]);
+      }
+    }
+  };
+  for (int t0 = k0; t0 < k1; t0 += 48) {
+    load_tile<DT>(rk, p.k_st, t0 + 32, g, n, kt[2], cov_xs<DT>(p, 1));
+    tile(t0, kt[0]);
+    if (t0 + 16 >= k1) break;
+    load_tile<DT>(rk, p.k_st, t0 + 48, g, n, kt[0], cov_xs<DT>(p, 1));
+    tile(t0 + 16, kt[1]);
+    if (t0 + 32 >= k1) break;
+    load_tile<DT>(rk, p.k_st, t0 + 64, g, n, kt[1], cov_xs<DT>(p, 1));
+    tile(t0 + 32, kt[2]);
+  }
+  // lanes (0..3, n) hold disjoint keys of row n: this split's state of the row
+#pragma unroll
+  for (int b = 0; b < NRB; ++b) {
+    const float M = xmax32(xmax16(m[b]));
+    const float part = (M == -INFINITY || m[b] == -INFINITY) ? 0.0f : ls[b] * __builtin_amdgcn_exp2f(m[b] - M);
+    const float L = xsum32(xsum16(part));
+    if (g == 0) {
+      st[wave][b][n][0] = M;
+      st[wave][b][n][1] = L;
+    }
+  }
+  __syncthreads();
+  // thread t < 64: row t % 16 of the item's block t / 16, its splits combined in order
+  if (threadIdx.x < 64) {
+    const int rbi = threadIdx.x / 16, row = threadIdx.x % 16;
+    const int rg = rbi / NRB, b = rbi % NRB;
+    float M = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) M = fmaxf(M, st[rg * KS + s][b][row][0]);
+    float L = 0.0f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const float ms = st[rg * KS + s][b][row][0];
+      if (ms != -INFINITY) L += st[rg * KS + s][b][row][1] * __builtin_amdgcn_exp2f(ms - M);
+    }
+    const int rl = 64 * rb + 16 * rbi;
+    const int r_abs = gt[0] + rl + row;
+    if (rl < rows_g && r_abs < p.NR) {
+      const int64_t o = static_cast<int64_t>(h) * p.NR + r_abs;
+      p.row_m[o] = M == -INFINITY ? 0.0f : M;                // padding rows: every p is masked to 0 below
+      p.row_il[o] = L > 0.0f ? 1.0f / L : 0.0f;
+    }
+  }
 }
+
+// values of one 32-key step in LDS: [key][channel].  fp32 rows are padded by 8 bytes against bank
+// conflicts; 16-bit rows take 288 bytes (72 words), so that the transposed reads of a channel block
+// (16 lanes reading 8 bytes each of 4 keys x 4 channel quads) fall on distinct banks
+template <int DT>
+constexpr int vrow_words() { return DT == KVQ_F32 ? (kCD * 4 + 8) / 4 : 72; }
 
 typedef short tr16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) tr16x4 lds_tr16x4;
 
 template <int DT>
-__global__ __launch_bounds__(kCThreads, DT == KVQ_F32 ? 2 : 2) void cov_attend(CovParams p) {
-  constexpr int NH = TileOps<DT>::NH, ESZ = TileOps<DT>::ESZ, NRB = attend_rb<DT>();
-  constexpr int kBlocks = kCWaves * NRB;                   // 16-row blocks of a workgroup
-  // value rows of 288 bytes: the transposed reads of a channel block (16 lanes reading 8 bytes each of
-  // 4 keys x 4 channel quads) fall on distinct banks; key row j holds its 16-byte column c at c ^ (j & 15)
-  constexpr int VRW = 72;
-  __shared__ u32x4 kt[2][NH][32 * 16];
-  __shared__ __align__(16) uint32_t vt[2][NH][32 * VRW];
-  const int l = threadIdx.x % 64, g = l >> 4, n = l & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int nb = p.NR / 16, n_items = (nb + kBlocks - 1) / kBlocks;
-  // work units (h, range, item), the items in reverse, so that blocks of far reach start first
-  const int unit = xcd_unit(p.Hkv * kOSplit * n_items);
+__global__ __launch_bounds__(kCThreads) void cov_output(CovParams p) {
+  constexpr int ESZ = TileOps<DT>::ESZ;
+  constexpr int VRW = vrow_words<DT>();
+  constexpr int U16 = kCD * ESZ / 16;                        // 16-byte units of a value row
+  __shared__ __align__(16) uint32_t vt[32 * VRW];
+  const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
+  // work units (h, item, key split), h outermost; the items in reverse plan order, so the groups at
+  // the end of the context, whose keys reach furthest, start first and the short ones fill the tail
+  const int unit = xcd_unit(p.Hkv * kOSplit * p.n_items);
   if (unit < 0) return;
-  const int h = unit / (n_items * kOSplit), w = unit % (n_items * kOSplit);
-  const int sp = w / n_items, item = n_items - 1 - w % n_items;
-  const int kr = key_range(p), k0 = sp * kr;
-  int k1 = 0;                                              // last key any block of the item reads, + 1
-  int reach[NRB];                                          // of this wavefront's blocks
-#pragma unroll
-  for (int b = 0; b < kBlocks; ++b) {
-    const int block = item * kBlocks + b;
-    const int r = block < nb ? __builtin_amdgcn_readfirstlane(p.gtab[kGT * p.rowgrp[16 * block] + 3]) : 0;
-    k1 = max(k1, r);
-    if (b / NRB == wave) reach[b % NRB] = r;
-  }
-  k1 = min(k1, k0 + kr);
-  if (k0 >= k1) return;
-  u32x4 qop[NRB][4][NH];
-  int pos[NRB], first[NRB];                                // this lane's row's position; the block's smallest
-#pragma unroll
-  for (int b = 0; b < NRB; ++b) {
-    const int block = item * kBlocks + NRB * wave + b;
-    pos[b] = block < nb ? load_rows<DT>(p, h, 16 * block, g, n, qop[b]) : -1;
-    if (block >= nb) zero_ops<DT>(qop[b]);
-    int f = pos[b] < 0 ? INT_MAX : pos[b];
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) f = min(f, __shfl_xor(f, o, 64));
-    first[b] = __builtin_amdgcn_readfirstlane(f);
-  }
+  const int h = unit / (p.n_items * kOSplit), w = unit % (p.n_items * kOSplit);
+  const int item = p.n_items - 1 - w / kOSplit, sp = w % kOSplit;
+  const int grp = p.items[2 * item], rb = p.items[2 * item + 1];
+  const int32_t* gt = p.gtab + kGT * grp;
+  const int rows_g = p.rep * gt[2];
+  const int row0 = gt[0] + 64 * rb + 16 * wave;
+  const bool active = 64 * rb + 16 * wave < rows_g;        // inactive wavefronts still join the barriers
+  u32x4 qop[4][TileOps<DT>::NH];
+  int pos = -1;
+  if (active)
+    pos = load_rows<DT>(p, h, row0, g, n, qop);
+  else
+    zero_ops<DT>(qop);
+  const float rm = (active && row0 + n < p.NR) ? p.row_m[static_cast<int64_t>(h) * p.NR + row0 + n] : 0.0f;
+  const int mmax = gt[3];
+  // this workgroup's keys: split sp of the item's 32-key steps (every split writes its partial,
+  // zeros when it holds no keys; the probabilities use the row's global maximum and sum, so the
+  // partials add up to o)
+  const int nstep = (mmax + 31) / 32;
+  const int k0 = 32 * (nstep * sp / kOSplit), k1 = min(mmax, 32 * (nstep * (sp + 1) / kOSplit));
   const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k, p.k_sh, p.k_st, h, p.T, ESZ);
   const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v, p.v_sh, p.v_st, h, p.T, ESZ);
   const float qsc = p.qscale / (cov_xs<DT>(p, 0) * cov_xs<DT>(p, 1));   // logit scale of the scaled rows
-  // thread t moves the 8-channel units t % 16 of keys t / 16 and 16 + t / 16 of a step
-  u32x4 kx[2][NH], vx[2][NH];
-  const int sk = threadIdx.x / 16, sc = threadIdx.x % 16;
+  const float vsc = cov_xs<DT>(p, 2);
+  f32x4 acc[8];
+#pragma unroll
+  for (int cb = 0; cb < 8; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // a step's loads: its 32 value rows (this thread's 16-byte units; rows at or past mmax as zeros:
+  // p = 0 there must not meet a NaN) and this wavefront's two key tiles.  The next step's loads go
+  // out as soon as the current key tiles have entered the logit products.
+  constexpr int KU = (32 * U16 + kCThreads - 1) / kCThreads;
+  u32x4 vr[KU];
+  u32x4 kr[2][4][TileOps<DT>::NH];
   auto load_step = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int64_t key = t0 + 16 * i + sk;
-      const int ko = static_cast<int>((key * p.k_st + 8 * sc) * ESZ), vo = static_cast<int>((key * p.v_st + 8 * sc) * ESZ);
-#pragma unroll
-      for (int x = 0; x < NH; ++x) {
-        kx[i][x] = __builtin_amdgcn_raw_buffer_load_b128(rk, ko + 16 * x, 0, 0);
-        vx[i][x] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + 16 * x, 0, 0);
-      }
+    for (int k = 0; k < KU; ++k) {
+      const int u = threadIdx.x + kCThreads * k;
+      const int key = u / U16, w16 = u % U16;
+      vr[k] = u32x4{0u, 0u, 0u, 0u};
+      if (u < 32 * U16 && t0 + key < k1)
+        vr[k] = __builtin_amdgcn_raw_buffer_load_b128(
+            rv, static_cast<int>((static_cast<int64_t>(t0 + key) * p.v_st) * ESZ + 16 * w16), 0, 0);
     }
+#pragma unroll
+    for (int tau = 0; tau < 2; ++tau) load_tile<DT>(rk, p.k_st, t0 + 16 * tau, g, n, kr[tau], cov_xs<DT>(p, 1));
   };
-  auto store_step = [&](int s) {
+  if (k0 < k1) load_step(k0);
+  for (int t0 = k0; t0 < k1; t0 += 32) {
+    // LDS-only barriers: the key tiles of the step stay in flight while its value rows are stored
+    block_lds_barrier();                                     // the previous step's value rows are read
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int key = 16 * i + sk;
-      u32x4 ko[NH], vo[NH];
-      if constexpr (NH == 2) {
-        float a[8], b[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          a[e] = __uint_as_float(kx[i][e / 4][e % 4]) * cov_xs<DT>(p, 1);
-          b[e] = __uint_as_float(vx[i][e / 4][e % 4]) * cov_xs<DT>(p, 2);
+    for (int k = 0; k < KU; ++k) {
+      const int u = threadIdx.x + kCThreads * k;
+      if (u < 32 * U16) {
+        uint32_t* dst = vt + (u / U16) * VRW + 4 * (u % U16);
+        if constexpr (DT == KVQ_F32) {
+          dst[0] = vr[k][0];
+          dst[1] = vr[k][1];
+          dst[2] = vr[k][2];
+          dst[3] = vr[k][3];
+        } else {
+          *reinterpret_cast<u32x4*>(dst) = vr[k];                // 288-byte rows: 16-byte aligned
         }
-        f32_parts<DT>(a, ko[0], ko[1]);
-        f32_parts<DT>(b, vo[0], vo[1]);
-      } else {
-        ko[0] = kx[i][0];
-        vo[0] = vx[i][0];
-      }
-#pragma unroll
-      for (int x = 0; x < NH; ++x) {
-        kt[s & 1][x][16 * key + (sc ^ (key & 15))] = ko[x];
-        *reinterpret_cast<u32x4*>(&vt[s & 1][x][key * VRW + 4 * sc]) = vo[x];
       }
     }
-  };
-  f32x4 acc[NRB][8];
-  float m[NRB], ls[NRB];
+    block_lds_barrier();
+    // probabilities of the two 16-key tiles: lane (g, n) holds keys t0 + 4g + i and t0 + 16 + 4g + i
+    // of row n
+    f32x4 dd[2];
 #pragma unroll
-  for (int b = 0; b < NRB; ++b) {
-#pragma unroll
-    for (int cb = 0; cb < 8; ++cb) acc[b][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m[b] = kRefNone;
-    ls[b] = 0.0f;
-  }
-  load_step(k0);
-  store_step(0);
-  load_step(k0 + 32);
-  for (int s = 0, t0 = k0; t0 < k1; ++s, t0 += 32) {
-    __syncthreads();                                       // step s is stored, step s - 1 read
-    store_step(s + 1);
-    load_step(t0 + 64);                                    // (past the keys: zeros, or keys not used)
-    // logits of the two 16-key tiles: lane (g, n) holds keys t0 + 4g + i and t0 + 16 + 4g + i of row n
-    f32x4 d[NRB][2];
+    for (int tau = 0; tau < 2; ++tau) dd[tau] = tile_dots<DT, TileOps<DT>::NH, TileOps<DT>::NH>(kr[tau], qop);
+    if (t0 + 32 < k1) load_step(t0 + 32);
+    float pr[8];
 #pragma unroll
     for (int tau = 0; tau < 2; ++tau) {
-      u32x4 kop[4][NH];
+      const f32x4 d = dd[tau];
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int x = 0; x < NH; ++x) kop[ks][x] = kt[s & 1][x][16 * (16 * tau + n) + ((4 * ks + g) ^ n)];
-#pragma unroll
-      for (int b = 0; b < NRB; ++b) d[b][tau] = tile_dots<DT, NH, NH>(kop, qop[b]);
+      for (int i = 0; i < 4; ++i) {
+        const int j = t0 + 16 * tau + 4 * g + i;
+        pr[4 * tau + i] = (j <= pos && j < mmax) ? __builtin_amdgcn_exp2f(d[i] * qsc - rm) : 0.0f;
+      }
     }
-    u32x4 ph[NRB], pl[NRB];
-    bool edge = false;                                     // some block's keys end in the step
+    // A operand: row n, k-index 8g + kk <-> key kk < 4 ? 4g + kk : 16 + 4g + kk - 4 (hi and lo parts)
+    u32x4 ph, pl;
+    f32_parts<DT>(pr, ph, pl);
+    // B operand per 16-channel block cb: lane (g, n) holds the values of those keys at channel 16cb + n
 #pragma unroll
-    for (int b = 0; b < NRB; ++b) {
-      float sv[8];
+    for (int cb = 0; cb < 8; ++cb) {
+      const int c = 16 * cb + n;
+      if constexpr (DT == KVQ_F32) {
+        float x[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sv[i] = d[b][i / 4][i % 4] * qsc;
-      if (t0 + 31 > first[b]) {                            // keys past a row's position
-        edge = edge || t0 + 32 > reach[b];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int j = t0 + 16 * (i / 4) + 4 * g + i % 4;
-          sv[i] = (j <= pos[b] && j < reach[b]) ? sv[i] : -INFINITY;
+        for (int kk = 0; kk < 8; ++kk) {
+          const int key = kk < 4 ? 4 * g + kk : 16 + 4 * g + kk - 4;
+          x[kk] = __uint_as_float(vt[key * VRW + c]) * vsc;
         }
-      }
-      const float mx = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
-      if (__any(mx > m[b] + kRefLazy)) {
-        const float top = xmax32(xmax16(mx));              // the row's largest logit of the step
-        const float to = top > m[b] + kRefLazy ? top : m[b];
-        const float f = __builtin_amdgcn_exp2f(m[b] - to);
-        ls[b] *= f;
-        m[b] = to;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {                      // register i of the outputs is row 4g + i
-          const float fr = __shfl(f, 4 * g + i, 64);
-#pragma unroll
-          for (int cb = 0; cb < 8; ++cb) acc[b][cb][i] *= fr;
-        }
-      }
-      float pr[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) pr[i] = __builtin_amdgcn_exp2f(sv[i] - m[b]);
-      ls[b] += ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
-      // A operand: row n, k-index 8g + kk <-> key kk < 4 ? 4g + kk : 16 + 4g + kk - 4 (hi and lo parts)
-      f32_parts<DT>(pr, ph[b], pl[b]);
-    }
-    // B operand per 16-channel block: LDS transpose reads (ds_read_b64_tr_b16): within each 16-lane
-    // group, lane n receives element n & 3 of the 8-byte loads of lanes (n >> 2) + 4 j, j = 0..3.  Lane
-    // (g, q + 4 j) therefore points at key 4g + j (then 16 + 4g + j), channels 16 cb + 4q .. + 3, and
-    // lane (g, n) receives keys 4g .. 4g + 3 (16 + 4g ..) of channel 16 cb + n
-    const uint32_t* a0 = &vt[s & 1][0][(4 * g + (n >> 2)) * VRW + 2 * (n & 3)];
-    auto value_op = [&](int x, int cb) {
-      const uint32_t* a = a0 + x * 32 * VRW + 8 * cb;
-      const tr16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a));
-      const tr16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a + 16 * VRW));
-      const uint2 lw = __builtin_bit_cast(uint2, lo), hw = __builtin_bit_cast(uint2, hi);
-      return u32x4{lw.x, lw.y, hw.x, hw.y};
-    };
-    auto accumulate = [&](int b, int cb, const u32x4 (&vb)[NH]) {
-      acc[b][cb] = tile_mfma<DT>(ph[b], vb[0], acc[b][cb]);
-      acc[b][cb] = tile_mfma<DT>(pl[b], vb[0], acc[b][cb]);
-      if constexpr (NH == 2) acc[b][cb] = tile_mfma<DT>(ph[b], vb[1], acc[b][cb]);
-    };
-    if (!edge) {
-#pragma unroll
-      for (int cb = 0; cb < 8; ++cb) {
-        u32x4 vb[NH];
-#pragma unroll
-        for (int x = 0; x < NH; ++x) vb[x] = value_op(x, cb);
-#pragma unroll
-        for (int b = 0; b < NRB; ++b) accumulate(b, cb, vb);
-      }
-    } else {
-      // a block's values past its reach are left out: a zero probability must not meet a NaN there
-#pragma unroll
-      for (int b = 0; b < NRB; ++b) {
-        u32x4 keep;                                        // operand word i: keys (0, 1), (2, 3), (16, 17), (18, 19) + 4g
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = t0 + 16 * (i / 2) + 4 * g + 2 * (i % 2);
-          keep[i] = (j < reach[b] ? 0xffffu : 0u) | (j + 1 < reach[b] ? 0xffff0000u : 0u);
-        }
-#pragma unroll
-        for (int cb = 0; cb < 8; ++cb) {
-          u32x4 vb[NH];
-#pragma unroll
-          for (int x = 0; x < NH; ++x) vb[x] = value_op(x, cb) & keep;
-          accumulate(b, cb, vb);
-        }
+        u32x4 vh, vl;
+        f32_parts<DT>(x, vh, vl);
+        acc[cb] = tile_mfma<DT>(ph, vh, acc[cb]);
+        acc[cb] = tile_mfma<DT>(pl, vh, acc[cb]);
+        acc[cb] = tile_mfma<DT>(ph, vl, acc[cb]);
+      } else {
+        // LDS transpose reads (ds_read_b64_tr_b16): within each 16-lane group, lane n receives
+        // element n & 3 of the 8-byte loads of lanes (n >> 2) + 4 j, j = 0..3.  Lane (g, q + 4 j)
+        // therefore points at key 4g + j (then 16 + 4g + j), channels 16 cb + 4q .. + 3, and lane
+        // (g, n) receives keys 4g .. 4g + 3 (16 + 4g ..) of channel 16 cb + n: the B operand
+        const int src_key = 4 * g + (n >> 2), src_ch = 16 * cb + 4 * (n & 3);
+        const uint32_t* a0 = vt + src_key * VRW + src_ch / 2;
+        const tr16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a0));
+        const tr16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a0 + 16 * VRW));
+        const uint2 lw = __builtin_bit_cast(uint2, lo), hw = __builtin_bit_cast(uint2, hi);
+        const u32x4 vb = u32x4{lw.x, lw.y, hw.x, hw.y};
+        acc[cb] = tile_mfma<DT>(ph, vb, acc[cb]);
+        acc[cb] = tile_mfma<DT>(pl, vb, acc[cb]);
       }
     }
   }
-  // D lane (g, n) register i: row 4g + i of the block, channel 16 cb + n
+  if (!active) return;
+  // D lane (g, n) register i: row 4g + i of the block, channel 16cb + n
 #pragma unroll
-  for (int b = 0; b < NRB; ++b) {
-    const int block = item * kBlocks + NRB * wave + b;
-    if (k0 >= reach[b]) continue;                          // (a block past the last: no reach)
-    const int64_t row0 = (static_cast<int64_t>(sp) * p.Hkv + h) * p.NR + 16 * block;
-    const float sum = xsum32(xsum16(ls[b]));
-    if (g == 0) reinterpret_cast<float2*>(p.ml)[row0 + n] = make_float2(m[b], sum);
+  for (int i = 0; i < 4; ++i) {
+    const int row = row0 + 4 * g + i;
+    if (row >= p.NR) continue;
+    const float il = p.row_il[static_cast<int64_t>(h) * p.NR + row] / vsc;   // exact: vsc a power of two
+    float* dst = p.o_part + ((static_cast<int64_t>(sp) * p.Hkv + h) * p.NR + row) * kCD + n;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int cb = 0; cb < 8; ++cb) p.o_part[(row0 + 4 * g + i) * kCD + 16 * cb + n] = acc[b][cb][i];
+    for (int cb = 0; cb < 8; ++cb) dst[16 * cb] = acc[cb][i] * il;
   }
 }
 
@@ -501,73 +529,38 @@ __global__ __launch_bounds__(kCThreads) void cov_vmv(CovParams p) {
   }
 }
 
-// o M and o M o for 32 rows of query head r per workgroup, M = the metric of (h, r) staged in LDS in two
-// halves of 64 rows; the rows' key ranges are combined on the way in.  Grid: (h, r, tile of 32 rows).
-template <int DT>
-__global__ __launch_bounds__(kCThreads) void cov_metric(CovParams p, const int32_t* rlist, int count) {
+// x M and x M x for 32 vectors per workgroup, M = the metric of query head (h, r) staged in LDS in
+// two halves of 64 rows.  ROWS: the row outputs of query head r (o M replaces o, o M o out);
+// otherwise the coded values (v M v out).  Grid: (h, r, tile of 32 vectors).
+template <int DT, bool ROWS>
+__global__ __launch_bounds__(kCThreads) void cov_metric(CovParams p, const int32_t* rlist, int n_rlist) {
   constexpr int XS = kCD + 1;                          // odd stride: the rows' reads hit distinct banks
   __shared__ float Ms[64 * kCD];                       // 32 KiB
   __shared__ float xs[kMetricRows * XS];
   __shared__ float red[kMetricRows][8];
-  __shared__ float wsp[kMetricRows][kOSplit];          // a row's weight of each key range
-  __shared__ int parts[kMetricRows];                   // and the last of its ranges
+  const int count = ROWS ? n_rlist : p.n;
   const int per = (count + kMetricRows - 1) / kMetricRows;
   const int hr = blockIdx.x / per, tile = blockIdx.x % per;
   const int h = hr / p.rep, r = hr % p.rep;
   const float* Mg = p.M + static_cast<int64_t>(h * p.rep + r) * kCD * kCD;
-  const int32_t* rl = rlist + static_cast<int64_t>(r) * count;
-  const int kr = key_range(p);
-  if (threadIdx.x < kMetricRows) {
-    const int at = kMetricRows * tile + static_cast<int>(threadIdx.x), row = at < count ? rl[at] : -1;
-    int last = -1;
-    if (row >= 0) {
-      last = (p.gtab[kGT * p.rowgrp[row] + 3] - 1) / kr;
-      const float2* ml = reinterpret_cast<const float2*>(p.ml) + static_cast<int64_t>(h) * p.NR + row;
-      float2 x[kOSplit];
-      float M = kRefNone, L = 0.0f;
+  const int32_t* rl = ROWS ? rlist + static_cast<int64_t>(r) * n_rlist : nullptr;
+  for (int u = threadIdx.x; u < kMetricRows * kCD; u += kCThreads) {
+    const int k = u / kCD, c = u % kCD;
+    const int idx = kMetricRows * tile + k;
+    float x = 0.0f;
+    if (idx < count) {
+      if constexpr (ROWS) {
+        if (rl[idx] >= 0) {                            // the key splits' outputs, summed in order
+          const int64_t o = (static_cast<int64_t>(h) * p.NR + rl[idx]) * kCD + c;
+          const int64_t split = static_cast<int64_t>(p.Hkv) * p.NR * kCD;
 #pragma unroll
-      for (int sp = 0; sp < kOSplit; ++sp) {
-        x[sp] = sp <= last ? ml[static_cast<int64_t>(sp) * p.Hkv * p.NR] : make_float2(kRefNone, 0.0f);
-        M = fmaxf(M, x[sp].x);
-      }
-#pragma unroll
-      for (int sp = 0; sp < kOSplit; ++sp) L += x[sp].y * __builtin_amdgcn_exp2f(x[sp].x - M);
-      const float il = L > 0.0f ? 1.0f / L : 0.0f;
-#pragma unroll
-      for (int sp = 0; sp < kOSplit; ++sp)             // exact division: a power of two
-        wsp[threadIdx.x][sp] = sp <= last ? __builtin_amdgcn_exp2f(x[sp].x - M) * il / cov_xs<DT>(p, 2) : 0.0f;
-      p.row_m[static_cast<int64_t>(h) * p.NR + row] = M;
-      p.row_il[static_cast<int64_t>(h) * p.NR + row] = il;
-    }
-    parts[threadIdx.x] = last;
-  }
-  __syncthreads();
-  for (int u = threadIdx.x; u < kMetricRows * kCD / 4; u += kCThreads) {
-    const int k = u / (kCD / 4), c = 4 * (u % (kCD / 4));
-    const int last = parts[k];
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (last >= 0) {
-      // the ranges' outputs, weighted and summed in order; past the last its own again, not counted
-      const int64_t o = (static_cast<int64_t>(h) * p.NR + rl[kMetricRows * tile + k]) * kCD + c;
-      const int64_t split = static_cast<int64_t>(p.Hkv) * p.NR * kCD;
-      float4 y[kOSplit];
-#pragma unroll
-      for (int sp = 0; sp < kOSplit; ++sp) y[sp] = *reinterpret_cast<const float4*>(p.o_part + min(sp, last) * split + o);
-#pragma unroll
-      for (int sp = 0; sp < kOSplit; ++sp) {
-        const float w = wsp[k][sp];
-        if (sp <= last) {
-          x.x = __builtin_fmaf(y[sp].x, w, x.x);
-          x.y = __builtin_fmaf(y[sp].y, w, x.y);
-          x.z = __builtin_fmaf(y[sp].z, w, x.z);
-          x.w = __builtin_fmaf(y[sp].w, w, x.w);
+          for (int sp = 0; sp < kOSplit; ++sp) x += p.o_part[sp * split + o];
         }
+      } else {
+        x = load_as_f32<DT>(p.v, static_cast<int64_t>(h) * p.v_sh + static_cast<int64_t>(p.rs + idx) * p.v_st + c);
       }
     }
-    xs[k * XS + c] = x.x;
-    xs[k * XS + c + 1] = x.y;
-    xs[k * XS + c + 2] = x.z;
-    xs[k * XS + c + 3] = x.w;
+    xs[k * XS + c] = x;
   }
   // thread: vector k = t / 8, output channels 16 (t % 8) .. + 15
   const int k = threadIdx.x / 8, c8 = threadIdx.x % 8;
@@ -601,12 +594,16 @@ __global__ __launch_bounds__(kCThreads) void cov_metric(CovParams p, const int32
   if (idx >= count) return;
   const float tot = ((red[k][0] + red[k][1]) + (red[k][2] + red[k][3])) +
                     ((red[k][4] + red[k][5]) + (red[k][6] + red[k][7]));
-  if (rl[idx] < 0) return;
-  const int64_t rid = static_cast<int64_t>(h) * p.NR + rl[idx];
-  float* dst = p.o + rid * kCD + 16 * c8;
+  if constexpr (ROWS) {
+    if (rl[idx] < 0) return;
+    const int64_t rid = static_cast<int64_t>(h) * p.NR + rl[idx];
+    float* dst = p.o + rid * kCD + 16 * c8;             // this workgroup staged its rows before any write
 #pragma unroll
-  for (int e = 0; e < 16; ++e) dst[e] = y[e];
-  if (c8 == 0) p.oMo[rid] = tot;
+    for (int e = 0; e < 16; ++e) dst[e] = y[e];
+    if (c8 == 0) p.oMo[rid] = tot;
+  } else {
+    if (c8 == 0) p.vmv[(static_cast<int64_t>(h) * p.rep + r) * p.n + idx] = tot;
+  }
 }
 
 // Rows of cov_terms in blocks of 16, each one contiguous record: the A operands of its products in lane
@@ -987,10 +984,9 @@ __global__ __launch_bounds__(kCThreads) void cov_roww(CovParams p, const int32_t
   if (qt || !in) return;
   const int x = threadIdx.x;
   a = (part[0][x] + part[1][x]) + (part[2][x] + part[3][x]);
-  const float gw = grp >= 0 ? p.gw[grp] : 0.0f;
-  a = grp >= 0 ? a / static_cast<float>(p.gtab[kGT * grp + 1]) * gw : 0.0f;
+  a = grp >= 0 ? a / static_cast<float>(p.gtab[kGT * grp + 1]) * p.gw[grp] : 0.0f;
   if (i < 16) p.roww[static_cast<int64_t>(h) * p.NR + row] = a;
-  else p.omega[static_cast<int64_t>(hb) * 4 + i - 16] = gw == 0.0f ? 0.0f : a;   // as cov_wsum: no part of the group
+  else p.omega[static_cast<int64_t>(hb) * 4 + i - 16] = a;
 }
 
 // the groups' stored token sums with their weights: A, DD and the read mass of the tokens
@@ -1173,7 +1169,7 @@ static int64_t cov_store_tokens(int64_t Hkv, int64_t n, int64_t G) {
   return std::max<int64_t>(1, std::min(all, fit)) * kChunkTok;
 }
 
-// workspace layout (floats): ml (2 kOSplit Hkv NR); row_m, row_il, oMo, roww (Hkv NR each), omega (Hkv NR / 4); o (Hkv NR d); o_part (kOSplit Hkv
+// workspace layout (floats): row_m, row_il, oMo, roww (Hkv NR each), omega (Hkv NR / 4); o (Hkv NR d); o_part (kOSplit Hkv
 // NR d); vmv (Hkv rep n); ddpart (G Hkv n_chunks kTW); gw (2 G + 1); red (4 + Hkv rep + Hkv); tsum (G Hkv 3
 // store tokens); row_part (Hkv n_chunks NR / 16 kRowPart), rec (Hkv NR / 16 records, fp32's the larger
 // ones), 16-byte aligned; S_part (kSSplit Hkv d d); sums (Hkv (2 + rep));
@@ -1181,7 +1177,7 @@ static int64_t cov_store_tokens(int64_t Hkv, int64_t n, int64_t G) {
 extern "C" int64_t kvq_coverage_stats_workspace(int64_t Hkv, int64_t rep, int64_t n, int64_t NR, int64_t G) {
   if (Hkv <= 0 || rep <= 0 || n <= 0 || NR <= 0 || G <= 0) return -1;
   const int64_t nch = (n + kChunkTok - 1) / kChunkTok;
-  return (4 + 2 * kOSplit) * Hkv * NR + Hkv * (NR / 4) + (1 + kOSplit) * Hkv * NR * kCD + Hkv * rep * n + G * Hkv * nch * kTW + Hkv * nch * (NR / 16) * kRowPart +
+  return 4 * Hkv * NR + Hkv * (NR / 4) + (1 + kOSplit) * Hkv * NR * kCD + Hkv * rep * n + G * Hkv * nch * kTW + Hkv * nch * (NR / 16) * kRowPart +
          (2 * G + 1) + (4 + Hkv * rep + Hkv) + G * Hkv * 3 * cov_store_tokens(Hkv, n, G) +
          Hkv * (NR / 16) * rec_units<KVQ_F32>() * 4 + 4 + kSSplit * Hkv * kCD * kCD + Hkv * (2 + rep) + kAmaxFloats;
 }
@@ -1214,14 +1210,13 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
   KVQ_REQUIRE(workspace_floats >= need, "kvq_coverage_stats: workspace too small (%lld < %lld floats)",
               (long long)workspace_floats, (long long)need);
   CovParams p{};
-  p.qr = qr; p.rowpos = rowpos; p.rowgrp = rowgrp; p.gtab = gtab;
+  p.qr = qr; p.rowpos = rowpos; p.gtab = gtab; p.items = items;
   p.k = k; p.v = v; p.k_sh = k_sh; p.k_st = k_st; p.v_sh = v_sh; p.v_st = v_st;
   p.M = M;
-  p.Hkv = (int)Hkv; p.rep = (int)rep; p.NR = (int)NR; p.G = (int)G;
+  p.Hkv = (int)Hkv; p.rep = (int)rep; p.NR = (int)NR; p.G = (int)G; p.n_items = (int)n_items;
   p.rs = (int)rs; p.re = (int)re; p.n = (int)n; p.n_chunks = (int)((n + kChunkTok - 1) / kChunkTok); p.T = (int)T;
   p.scaling = scaling; p.qscale = scaling * kCLog2e; p.eta = eta;
   float* w = workspace;
-  p.ml = w; w += 2 * kOSplit * Hkv * NR;
   p.row_m = w; w += Hkv * NR;
   p.row_il = w; w += Hkv * NR;
   p.oMo = w; w += Hkv * NR;
@@ -1254,14 +1249,13 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
     launch_rows_scales(views, 3, amax_part, const_cast<float*>(p.xs), s);
     KVQ_LAUNCH_CHECK("kvq_coverage_stats(fp32 scales)");
   }
-  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_attend<DT_>),
-                                               dim3(xcd_grid(Hkv * kOSplit * ((NR / 16 + kCWaves * attend_rb<DT_>() - 1) /
-                                                                              (kCWaves * attend_rb<DT_>())))),
-                                               blk, 0, s, p));
-  KVQ_LAUNCH_CHECK("kvq_coverage_stats(outputs)");
-  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_metric<DT_>),
-                                               dim3(Hkv * rep * ((n_rlist + kMetricRows - 1) / kMetricRows)), blk, 0, s, p,
-                                               rlist, (int)n_rlist));
+  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_rowstats<DT_>), dim3(xcd_grid(n_items * Hkv)),
+                                               dim3(DT_ == KVQ_F32 ? kCThreads : 2 * kCThreads), 0, s, p));
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(rowstats)");
+  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_output<DT_>), dim3(xcd_grid(n_items * Hkv * kOSplit)), blk, 0, s, p));
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(output)");
+  hipLaunchKernelGGL((cov_metric<KVQ_F32, true>), dim3(Hkv * rep * ((n_rlist + kMetricRows - 1) / kMetricRows)), blk,
+                     0, s, p, rlist, (int)n_rlist);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(o M)");
   KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_vmv<DT_>),
                                                dim3(Hkv * rep * ((n + kVmvPer - 1) / kVmvPer)), blk, 0, s, p));

@@ -167,27 +167,3 @@ def test_coverage_token_ranges():
     for n in ("A", "W", "DD", "S"):
         _check(st[n], ref, n, 2e-4)
     _check(st["Mbar"], ref, "Mbar", 1e-5)
-
-
-@pytest.mark.parametrize("dtype,rep", [(torch.bfloat16, 4), (torch.float16, 1), (torch.float32, 2)])
-def test_coverage_nan_past_a_groups_reach(dtype, rep, monkeypatch):
-    """NaN in the first key and value past a group's reach, inside the 32-key step its last keys are in
-    and read by later groups of the same workgroup: the groups that do not attend it keep their
-    statistics, those that do are not live (their drop total is NaN).  Reference: the oracle over the
-    groups that end before it (a closing group that reaches nothing stands for the window group).
-    Row blocks of several groups in one workgroup (rep 1, 2).  Bar as above."""
-    import kvq
-    H, Hkv, rs, re = 1300, 2, 4, 1268
-    q, k, v, M = _inputs(31, Hkv * rep, Hkv, H, H, dtype)
-    groups = oc.coverage_groups(H, oc.CoverageParams())
-    bad = int(groups[0].max()) + 1
-    k[:, :, bad] = float("nan")
-    v[:, :, bad] = float("nan")
-    print(f"coverage NaN at key {bad}: {dtype} rep {rep}", flush=True)
-    st = _run(q, k, v, M, H, rs, re)
-    monkeypatch.setattr(oc, "coverage_groups", lambda H, c: [groups[0], np.array([0])])
-    k, v = k.nan_to_num(0.0), v.nan_to_num(0.0)
-    ref = _oracle(q, k, v, M, H, rs, re)
-    for name in ("A", "W", "DD"):                                     # (S weighs the dead groups' rows by zero: NaN)
-        _check(st[name], ref, name, 2e-4)
-    _check(st["Mbar"], ref, "Mbar", 1e-5)
