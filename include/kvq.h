@@ -284,7 +284,7 @@ int kvq_snapkv_scores(const void* q, int dtype, int64_t q_sb, int64_t q_sh, int6
  *    aligned rows; M (Hq, d, d) float32: the output metric of each query head.  d = 128.
  * Outputs float32: A, W, DD (Hkv, re - rs); S, Mbar (Hkv, d, d) -- the reference's A, W, DD, S and
  *    Mbar with floor eta (STRATA_FLOOR).  workspace: kvq_coverage_stats_workspace(...) floats.
- *    Launches on `stream` only, no host synchronisation, deterministic (no atomics).
+ *    Eleven launches on `stream`, no host synchronisation, deterministic (no atomics).
  * ---------------------------------------------------------------------------------------- */
 int64_t kvq_coverage_stats_workspace(int64_t Hkv, int64_t rep, int64_t n, int64_t NR, int64_t G);
 int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const int32_t* rowpos, const int32_t* rowgrp,

@@ -22,14 +22,14 @@
 //   cov_metric    x M and x M x for 32 vectors per workgroup with the query head's metric staged in
 //                 LDS: the row outputs (the key splits' parts summed in order; o M) and the coded
 //                 values (v M v).
-//   cov_rowprep   the rows' operands and values as records of 16 rows, in the order cov_terms reads.
-//   cov_terms     per (h, chunk of tokens, piece of the groups reaching it): logits and v.(oM) on the
-//                 matrix cores, then the per-(row, token) terms, once: the group's drop total, every
-//                 row's key-term mass and the read mass per 16 rows as partials per chunk, and the
-//                 group's unweighted sums per token.
+//   cov_terms<A>  per (h, 256-token chunk, group split): for every group of the split reaching the
+//                 chunk, logits and v.(oM) of 16-token tiles on the matrix cores (rows as the A side:
+//                 a lane holds four rows of one token), then the per-(row, token) terms: the group's
+//                 drop total and every row's key-term mass, as partials per chunk.
 //   cov_groups    N per group -> weight 1 / N (0 if N = 0), live flag.
-//   cov_roww      per row (block): its group's weight x its key-term (read) mass.
-//   cov_wsum      the groups' token sums with their weights: A, DD and the read mass W.
+//   cov_roww      per row: its group's weight x its key-term mass.
+//   cov_terms<B>  the same tiles with the weights: A, DD and the read mass per query head, one partial
+//                 per group split; cov_split_sums adds the splits in order.
 //   cov_smat      S = sum over rows of weight * alpha * (scaling q)(scaling q)^T.
 //   cov_final     live average, S / sum_j A_j, Mbar, floors (one workgroup for the sums, then all).
 #include <algorithm>
@@ -44,14 +44,12 @@ namespace {
 constexpr int kCD = 128;
 constexpr int kCThreads = 256;
 constexpr int kCWaves = 4;
-constexpr int kTW = 4;                   // wavefronts of a cov_terms workgroup
-constexpr int kChunkTok = 32 * kTW;      // its tokens: two 16-token tiles per wavefront
+constexpr int kChunkTok = 256;          // tokens of a cov_terms workgroup
 constexpr int kGT = 8;                  // ints per group-table entry
 constexpr int kMetricRows = 32;         // vectors of a cov_metric workgroup
 constexpr int kOSplit = 4;              // key splits of cov_output (workgroups per 64-row item)
-constexpr int kRowPart = 20;            // its rows' key-term masses, its read mass in four parts
-constexpr int kTermsUnits = 1536;       // workgroups of cov_terms worth cutting the groups of a chunk for
-constexpr int64_t kStoreFloats = int64_t{1} << 28;   // most floats of the stored token sums (1 GiB)
+constexpr int kTSplit = 4;              // group splits of cov_terms (workgroups per token chunk)
+constexpr int kTermsLdsRep = 8;         // most query heads per KV head of cov_terms' LDS form
 constexpr int kSSplit = 16;             // row splits of cov_smat (workgroups per 16 rows of S)
 constexpr float kCLog2e = 1.4426950408889634f;
 
@@ -73,19 +71,22 @@ struct CovParams {
   float* o;                              // (Hkv, NR, d) o M (cov_metric over the summed outputs)
   float* o_part;                         // (kOSplit, Hkv, NR, d) fp32 outputs of each key split
   float* oMo;                            // (Hkv, NR)
-  uint32_t* rec;                         // (Hkv, NR / 16) records of cov_terms (rec_units<DT> u32x4)
+  uint32_t* mop;                         // (Hkv, NR, 4 ks, 4 g, 2 parts) u32x4: o M operand parts
+  float* rowf;                           // (Hkv, NR) float4: row max, 1 / sum, o M o, o M scale
   float* vmv;                            // (Hkv, rep, n)
-  float* ddpart;                         // (G, Hkv, n_chunks, kTW): drop totals per wavefront
-  float* row_part;                       // (Hkv, n_chunks, NR / 16, kRowPart): a 16-row block over a chunk
-  float* tsum;                           // (G, Hkv, 3, store_n): a group's key term, drop term, read mass per token
+  float* ddpart;                         // (G, Hkv, n_chunks, 4): drop totals per wavefront
+  float* alpha_part;                     // (Hkv, n_chunks, NR)
   float* gw;                             // (2 G + 1): 1 / N or 0 per group; [G + 1 + group]: 1 if live
   float* roww;                           // (Hkv, NR): weight * alpha
-  float* omega;                          // (Hkv, NR / 16, 4): weight * read mass of a block, in parts
   float* red;                            // finalisation sums
   float* sums;                           // (Hkv, 2 + rep): per-head sums of A, DD, read masses
   float* A;                              // (Hkv, n)
   float* W;                              // (Hkv, n)
   float* DD;                             // (Hkv, n)
+  float* WVa;                            // (Hkv, rep, n)
+  float* A_part;                         // (kTSplit, Hkv, n) weighted pass: each group split's sums
+  float* DD_part;                        // (kTSplit, Hkv, n)
+  float* WVa_part;                       // (kTSplit, Hkv, rep, n)
   float* S;                              // (Hkv, d, d)
   float* S_part;                         // (kSSplit, Hkv, d, d): each row split's sum
   float* Mbar;                           // (Hkv, d, d)
@@ -606,43 +607,46 @@ __global__ __launch_bounds__(kCThreads) void cov_metric(CovParams p, const int32
   }
 }
 
-// Rows of cov_terms in blocks of 16, each one contiguous record: the A operands of its products in lane
-// order (part p, k-step ks, lane l at unit (4 p + ks) 64 + l: the row's DT parts, then o M times the power
-// of two that brings its largest entry to [128, 256), inside the range of fp16 parts, as hi and lo
-// parts), then per row the max, 1 / sum, o M o, -2 x the power of two back, and the last key it counts
-// (-1: padding), and the smallest and largest of those keys.  A stage of cov_terms is a plain copy of
-// its records and every operand read is 64 consecutive 16-byte units.
-template <int DT>
-constexpr int rec_ops() { return (TileOps<DT>::NH + 2) * 4 * 64; }            // 16-byte operand units
-constexpr int kRecMeta = 32;                                                   // 16-byte units of row values (22 used)
-template <int DT>
-constexpr int rec_units() { return rec_ops<DT>() + kRecMeta; }
+__global__ __launch_bounds__(kCThreads) void cov_clear(float* x, int64_t count) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kCThreads + threadIdx.x;
+  if (t < count) x[t] = 0.0f;
+}
 
-// Once per row (after cov_metric): thread (row, ks, g) converts channels 32 ks + 8 g .. + 7 of its row
-template <int DT>
-__global__ __launch_bounds__(kCThreads) void cov_rowprep(CovParams p, const int32_t* rowgrp) {
-  constexpr int NH = TileOps<DT>::NH;
-  __shared__ int lims[16];
-  const int nb = p.NR / 16, h = blockIdx.x / nb, block = blockIdx.x % nb;
-  const int n = threadIdx.x / 16, sl = threadIdx.x % 16, ks = sl / 4, g = sl % 4;
-  const int row = 16 * block + n, pos = p.rowpos[row], grp = rowgrp[row];
-  const int64_t rid = static_cast<int64_t>(h) * p.NR + row;
-  u32x4* rec = reinterpret_cast<u32x4*>(p.rec) + (static_cast<int64_t>(h) * nb + block) * rec_units<DT>();
-  const bool live = pos >= 0 && grp >= 0;
-  const float4* src = reinterpret_cast<const float4*>(p.o + rid * kCD + 32 * ks + 8 * g);
-  float x[8];
-  u32x4 qop[NH];
+// the weighted pass's group splits summed in split order: A, DD (Hkv, n) and WVa (Hkv, rep, n)
+__global__ __launch_bounds__(kCThreads) void cov_split_sums(CovParams p) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kCThreads + threadIdx.x;
+  const int64_t nA = static_cast<int64_t>(p.Hkv) * p.n, nW = nA * p.rep;
+  if (t < nA) {
+    float a = 0.0f, dd = 0.0f;
 #pragma unroll
-  for (int hh = 0; hh < NH; ++hh) qop[hh] = u32x4{0u, 0u, 0u, 0u};
-  if (live) {
-    const float4 a = src[0], b = src[1];
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-    x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-    load_op<DT>(p.qr, rid * kCD + 32 * ks + 8 * g, qop, cov_xs<DT>(p, 0));
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = 0.0f;
+    for (int s = 0; s < kTSplit; ++s) {
+      a += p.A_part[s * nA + t];
+      dd += p.DD_part[s * nA + t];
+    }
+    p.A[t] = a;
+    p.DD[t] = dd;
   }
+  if (t < nW) {
+    float w = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kTSplit; ++s) w += p.WVa_part[s * nW + t];
+    p.WVa[t] = w;
+  }
+}
+
+// Once per row (after cov_metric): o M as the A operand of cov_terms' v.(oM) products -- times a
+// power of two that brings its largest entry to [128, 256) (inside the range of fp16 parts), in two
+// parts of the operand type -- and the row's values as one float4 (row max, 1 / sum, o M o, the
+// power of two back).  Thread (row, ks, g) converts channels 32 ks + 8 g .. + 7; a row's 16 threads
+// are one DPP row of a wavefront.
+template <int DT>
+__global__ __launch_bounds__(kCThreads) void cov_rowprep(CovParams p) {
+  const int64_t rid = static_cast<int64_t>(blockIdx.x) * (kCThreads / 16) + threadIdx.x / 16;
+  const int sl = threadIdx.x % 16, ks = sl / 4, g = sl % 4;
+  if (rid >= static_cast<int64_t>(p.Hkv) * p.NR) return;          // whole rows: 16 lanes alike
+  const float4* src = reinterpret_cast<const float4*>(p.o + rid * kCD + 32 * ks + 8 * g);
+  const float4 a = src[0], b = src[1];
+  float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
   float mx = 0.0f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[e]));
@@ -655,283 +659,343 @@ __global__ __launch_bounds__(kCThreads) void cov_rowprep(CovParams p, const int3
   for (int e = 0; e < 8; ++e) x[e] *= up;
   u32x4 hi, lo;
   f32_parts<DT>(x, hi, lo);
-  const int l = 16 * g + n;
-#pragma unroll
-  for (int hh = 0; hh < NH; ++hh) rec[(4 * hh + ks) * 64 + l] = qop[hh];
-  rec[(4 * NH + ks) * 64 + l] = hi;
-  rec[(4 * NH + 4 + ks) * 64 + l] = lo;
-  float* meta = reinterpret_cast<float*>(rec + rec_ops<DT>());
-  int* lim = reinterpret_cast<int*>(meta) + 64;
-  const int last = live ? min(pos - p.gtab[kGT * grp + 5], p.gtab[kGT * grp + 4] - 1) : -1;
-  if (sl == 0) {
-    meta[n] = live ? p.row_m[rid] : 0.0f;
-    meta[16 + n] = live ? p.row_il[rid] : 0.0f;
-    meta[32 + n] = live ? p.oMo[rid] : 0.0f;
-    meta[48 + n] = -2.0f * ldexpf(1.0f, ex - 8) / cov_xs<DT>(p, 2);       // exact: powers of two
-    lim[n] = last;
-    lims[n] = last;
-  }
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    int m = lims[0];
-    for (int i = 1; i < 16; ++i) m = threadIdx.x == 0 ? min(m, lims[i]) : max(m, lims[i]);
-    lim[16 + threadIdx.x] = m;
-  }
+  u32x4* dst = reinterpret_cast<u32x4*>(p.mop) + rid * 32 + (ks * 4 + g) * 2;
+  dst[0] = hi;
+  dst[1] = lo;
+  if (sl == 0)
+    reinterpret_cast<float4*>(p.rowf)[rid] = make_float4(p.row_m[rid], p.row_il[rid], p.oMo[rid], ldexpf(1.0f, ex - 8));
 }
 
-// The per-(row, token) terms, once: per (h, 256-token chunk, piece of the groups reaching it) the chunk's
-// key and value tiles stay in registers, 32 tokens per wavefront, and the groups' rows stream past them
-// through LDS (records of cov_rowprep, a block per stage, two stages, loads one more stage ahead), so
-// a group's sums over its rows (key term, drop term, read mass of a token) stay in the lane until its
-// last block and no wavefront waits for another within a group.  They go out unweighted, one value per
-// (group, h, term, token): a group's weight needs its drop total over every token, and reading them
-// back (cov_wsum) costs far less than the logits, exponentials and quotients a second time.  Per block
-// the wavefronts' row sums (key-term mass) and read mass meet in LDS, added in wavefront order.
-// Bound by the vector ALU and its waits: about 26 issue slots per (row, token) term, the exponential and
-// the reciprocal 4 each; 168 registers (three wavefronts per SIMD) hold two tiles -- four tiles (256
-// registers) spill and take 950 us, eight wavefronts per workgroup at 128 registers spill and take 1200.
-// 8 heads x 4 query heads, 65 groups, 32768 bf16 keys: 705 us and 41 us to read the sums back; the two
-// passes before (terms for the totals, then again with the weights, rows in registers and tokens from
-// LDS) took 893 and 1287 us.
-// R: tokens [store0, store0 + store_n) have their sums stored; `totals`: drop totals, key-term and read
-// masses written (the first launch; later ones only fill further token ranges of the store).
-struct TermsRange {
-  int chunk0, chunks, store0, store_n, pieces;
-  bool totals;
-};
-
-// lanes 0..31: a over the lane pair (l, l + 32); lanes 32..63: b
-__device__ __forceinline__ float add32(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-// rows of 16 lanes 0 and 2: a over the row pairs (0, 1) and (2, 3); rows 1 and 3: b over them
-__device__ __forceinline__ float add16(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-template <int DT>
-__global__ __launch_bounds__(64 * kTW, DT == KVQ_F32 ? 2 : 3) void cov_terms(CovParams p, TermsRange R) {
+// per (h, 256-token chunk, group split): every group reaching the chunk, its rows in 64-row blocks
+// (one 16-row block per wavefront, one query head per block since nq_pad is a multiple of 16),
+// 16-token tiles.  WEIGHTED = false: drop totals (one partial per wavefront, combined in order by
+// cov_groups) and key-term masses; true: the weighted per-token sums.
+// LDS (16-bit keys and values, rep <= kTermsLdsRep): the chunk's 256 key and value rows (128 KiB)
+// and its v M v of every query head are staged in LDS once, and every group and wavefront reads its
+// tiles there (a tile used to come from L2 once per group and wavefront); the weighted pass also
+// keeps its read masses there until the end.  Row t of a tensor holds its 16-byte column c at
+// c ^ (t & 15), so the 16 tokens of a tile read in one instruction fall on distinct banks.  The workgroup is two quads of wavefronts (two per SIMD, so one's products overlap
+// the other's terms): for the drop totals the quads take alternate groups with work; for the weighted
+// sums every group, quad q the tokens [c0 + 128 q, c0 + 128 q + 128), a lane's sums over the groups
+// kept in registers and added across the lane groups once at the end.  LDS = false: tiles and v M v
+// from memory, one tile ahead, one quad, a token's sums over the groups in LDS.
+template <int DT, bool WEIGHTED, bool LDS>
+__global__ __launch_bounds__(LDS ? 2 * kCThreads : kCThreads) void cov_terms(CovParams p) {
   constexpr int NH = TileOps<DT>::NH;
-  constexpr int NT = 64 * kTW;
-  constexpr int RU = rec_units<DT>();
-  constexpr int kPer = rec_ops<DT>() / NT;               // 16-byte operand units per thread and stage
-  static_assert(rec_ops<DT>() % NT == 0 && NT % kRecMeta == 0, "whole loads");
-  __shared__ u32x4 stage[2][RU];
-  __shared__ float vmv_lds[2][kChunkTok];                // v M v of the chunk's tokens with the block's query head
-  __shared__ float red[2][kTW][kRowPart];                // a block's 16 row sums, then its read mass in four parts
-  const int l = threadIdx.x % 64, g = l >> 4, n = l & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  // Work units u = (h, chunk, piece) in order, a contiguous range per XCD: the pieces and chunks of a
-  // head share one L2 for its rows' records.
-  const int u = xcd_unit(p.Hkv * R.chunks * R.pieces);
+  static_assert(!LDS || NH == 1, "LDS tiles hold 16-bit rows");
+  constexpr int NT = LDS ? 2 * kCThreads : kCThreads;
+  __shared__ u32x4 kv_lds[LDS ? 2 * kChunkTok * 16 : 1];         // [K, V][token][16-byte column]
+  __shared__ float vmv_lds[LDS ? kTermsLdsRep * kChunkTok : 1];  // [query head][token]
+  __shared__ float wva_lds[LDS && WEIGHTED ? kTermsLdsRep * kChunkTok : 1];   // read masses [head][token]
+  __shared__ float accA[kCWaves][kChunkTok];
+  __shared__ float accD[kCWaves][kChunkTok];
+  __shared__ float accW[kCWaves][kChunkTok];             // read mass of the wavefront's current block
+  const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
+  const int quad = wave / kCWaves, wq = wave % kCWaves;
+  // groups ts, ts + kTSplit, ... of (h, chunk): the chunks near the start, which every group reaches,
+  // spread over kTSplit workgroups.  Work units u = (h, chunk, ts) in order; block b runs on XCD b % 8
+  // (round-robin dispatch), and each XCD takes a contiguous range of units, so the splits of a chunk
+  // share one L2 and its key and value tiles stay there.
+  const int u = xcd_unit(p.Hkv * p.n_chunks * kTSplit);
   if (u < 0) return;
-  const int ts = u % R.pieces, h = u / R.pieces / R.chunks, chunk = R.chunk0 + u / R.pieces % R.chunks;
+  const int ts = u % kTSplit;
+  const int h = u / kTSplit / p.n_chunks, chunk = u / kTSplit % p.n_chunks;
   const int c0 = p.rs + chunk * kChunkTok;               // first token of the chunk
-  // the groups that reach the chunk lie in [g0, G); this piece of them, and its blocks
-  // the group table is only read here: scalar loads
-  const auto gtab = reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p.gtab));
-  int g0 = p.G;
-  for (int x = 0; x < p.G && g0 == p.G; x += 64) {
-    const uint64_t hit = __ballot(x + l < p.G && p.gtab[kGT * min(x + l, p.G - 1) + 4] > c0);
-    if (hit) g0 = x + __builtin_ctzll(hit);
-  }
-  const int ga = g0 + (p.G - g0) * ts / R.pieces, gb = g0 + (p.G - g0) * (ts + 1) / R.pieces;
-  if (ga == gb) return;
-  auto blocks_of = [&](int grp) { return p.rep * (gtab[kGT * grp + 2] / 16); };
-  auto first_of = [&](int grp) { return gtab[kGT * grp] / 16; };
-  int nb = 0;
-  for (int x = ga; x < gb; ++x) nb += blocks_of(x);
-  const u32x4* rec = reinterpret_cast<const u32x4*>(p.rec) + static_cast<int64_t>(h) * (p.NR / 16) * RU;
-  u32x4 pre[kPer + 1];
-  float pre_vmv;
-  // the next block to load: its group, blocks left in it and in its query head
-  int lg = ga, lleft = blocks_of(ga), lper = gtab[kGT * ga + 2] / 16, lbh = lper;
-  const float* const vmv_h = p.vmv + static_cast<int64_t>(h) * p.rep * p.n;
-  const float* vmv_r = vmv_h;
-  const uint32_t vmv_tok = min(c0 + static_cast<int>(threadIdx.x % kChunkTok), p.re - 1) - p.rs;
-  const u32x4* src = rec + static_cast<int64_t>(first_of(ga)) * RU;
-  auto load_stage = [&]() {
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) pre[i] = src[i * NT + threadIdx.x];
-    pre[kPer] = src[kPer * NT + threadIdx.x % kRecMeta];   // (every group of threads: no branch)
-    pre_vmv = vmv_r[vmv_tok];                              // (a token past the range is masked)
-    if (--lleft > 0) {
-      src += RU;
-      if (--lbh == 0) {
-        lbh = lper;
-        vmv_r += p.n;
-      }
-    } else if (++lg < gb) {                                // past the piece: its last block again, not used
-      src = rec + static_cast<int64_t>(first_of(lg)) * RU;
-      lleft = blocks_of(lg);
-      lbh = lper = gtab[kGT * lg + 2] / 16;
-      vmv_r = vmv_h;
-    }
-  };
-  auto store_stage = [&](int s) {
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) stage[s & 1][i * NT + threadIdx.x] = pre[i];
-    stage[s & 1][kPer * NT + threadIdx.x % kRecMeta] = pre[kPer];
-    vmv_lds[s & 1][threadIdx.x % kChunkTok] = pre_vmv;
-  };
-  load_stage();
-  const int t0 = c0 + 32 * wave;                          // this wavefront's tokens t0 .. t0 + 31
-  u32x4 kop[2][4][NH], vop[2][4][NH];
-  {
-    const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k, p.k_sh, p.k_st, h, p.T, TileOps<DT>::ESZ);
-    const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v, p.v_sh, p.v_st, h, p.T, TileOps<DT>::ESZ);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      load_tile<DT>(rk, p.k_st, t0 + 16 * t, g, n, kop[t], cov_xs<DT>(p, 1));
-      load_tile<DT>(rv, p.v_st, t0 + 16 * t, g, n, vop[t], cov_xs<DT>(p, 2));
-    }
-  }
+  const int c1 = min(c0 + kChunkTok, p.re);
+  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k, p.k_sh, p.k_st, h, p.T, TileOps<DT>::ESZ);
+  const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v, p.v_sh, p.v_st, h, p.T, TileOps<DT>::ESZ);
   const float qsc = p.qscale / (cov_xs<DT>(p, 0) * cov_xs<DT>(p, 1));   // logit scale of the scaled rows
-  store_stage(0);
-  load_stage();
-  // block `block`'s row sums and read mass, the wavefronts' added in order by one of them
-  float* row_part = p.row_part + (static_cast<int64_t>(h) * p.n_chunks + chunk) * (p.NR / 16) * kRowPart;
-  auto combine = [&](int s, int block) {
-    if (wave != (s & (kTW - 1)) || l >= kRowPart) return;
-    float a = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kTW; ++w) a += red[s & 1][w][l];
-    (row_part + static_cast<int64_t>(block) * kRowPart)[static_cast<uint32_t>(l)] = a;
-  };
-  int grp = ga, left = blocks_of(ga), block = first_of(ga), last = -1;
-  int ended = -1;                                          // group whose last block is done, its sums not yet out
-  float rA[2] = {0.0f, 0.0f}, rD[2] = {0.0f, 0.0f}, rW[2] = {0.0f, 0.0f};   // this lane's token sums over its rows
-  // group ga's token sums over the lane groups' rows, out
-  auto flush = [&](int ga) {
-    const int te = gtab[kGT * ga + 4];
-    float* out = p.tsum + (static_cast<int64_t>(ga) * p.Hkv + h) * 3 * R.store_n;
-    float dsum = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      // added over the lane groups and dealt to them at once: group 0 ends with A, 1 with D, 2 with W
-      const float z = add16(add32(rA[t], rW[t]), add32(rD[t], rD[t]));
-      rA[t] = rD[t] = rW[t] = 0.0f;
-      dsum += z;
-      const int j = t0 + 16 * t + n, at = j - R.store0;
-      if (g < 3 && j < te && at >= 0 && at < R.store_n) out[static_cast<uint32_t>(g * R.store_n + at)] = z;
+  if constexpr (WEIGHTED) {
+    for (int u = threadIdx.x; u < kCWaves * kChunkTok; u += NT) {
+      (&accA[0][0])[u] = 0.0f;
+      (&accD[0][0])[u] = 0.0f;
     }
-    if (R.totals) {
-      dsum = row_sum16(dsum);
-      if (l == 16) p.ddpart[((static_cast<int64_t>(ga) * p.Hkv + h) * p.n_chunks + chunk) * kTW + wave] = dsum;
+    if constexpr (LDS)
+      for (int u = threadIdx.x; u < kTermsLdsRep * kChunkTok; u += NT) wva_lds[u] = 0.0f;
+  }
+  // weighted LDS form: every group with work has 16 padded queries, so a wavefront's 16 rows are one
+  // query head and a head's read masses only ever come from one wavefront (no barrier between blocks)
+  bool solo = LDS && WEIGHTED;
+  // a group has work in this chunk if it reaches it (and, weighted, has a nonzero weight)
+  auto has_work = [&](int grp) { return p.gtab[kGT * grp + 4] > c0 && (!WEIGHTED || p.gw[grp] != 0.0f); };
+  if constexpr (LDS) {
+    bool used = false;                                   // some group of this split reaches the chunk
+    for (int grp = ts; grp < p.G; grp += kTSplit) {
+      const bool w = has_work(grp);
+      used = used || w;
+      solo = solo && (!w || p.gtab[kGT * grp + 2] == 16);
     }
-  };
-  for (int s = 0; s < nb; ++s) {
-    __syncthreads();                                       // stage s is stored, stage s - 1 read
-    store_stage(s + 1);
-    load_stage();
-    // the results of block s - 1 go out here, a block's work ahead of the next wait for loads
-    if (R.totals && last >= 0) combine(s - 1, last);
-    if (ended >= 0) flush(ended);
-    ended = -1;
-    const u32x4* ops = stage[s & 1];
-    const float* meta = reinterpret_cast<const float*>(ops + rec_ops<DT>());
-    const int* lim = reinterpret_cast<const int*>(meta) + 64;
-    const int lim_min = __builtin_amdgcn_readfirstlane(lim[16]), lim_max = __builtin_amdgcn_readfirstlane(lim[17]);
-    float alpha[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mass = 0.0f;
-    if (t0 <= lim_max) {
-      f32x4 sd[2], ov[2];
+    if (used) {
+      // 16-byte unit u = (tensor, token, column): all of a thread's loads issued before its stores
+      constexpr int kPer = 2 * kChunkTok * 16 / NT;
+      u32x4 x[kPer];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) sd[t] = ov[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < kPer; ++i) {
+        const int u = i * NT + static_cast<int>(threadIdx.x);
+        const int tok = (u >> 4) & (kChunkTok - 1), col = u & 15;
+        const bool key = u < kChunkTok * 16;
+        const int64_t off = (static_cast<int64_t>(c0 + tok) * (key ? p.k_st : p.v_st) + 8 * col) * 2;
+        x[i] = __builtin_amdgcn_raw_buffer_load_b128(key ? rk : rv, static_cast<int>(off), 0, 0);
+      }
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        u32x4 q[NH];
+      for (int i = 0; i < kPer; ++i) {
+        const int u = i * NT + static_cast<int>(threadIdx.x);
+        const int tok = (u >> 4) & (kChunkTok - 1), col = u & 15;
+        kv_lds[((u < kChunkTok * 16 ? 0 : kChunkTok) + tok) * 16 + (col ^ (tok & 15))] = x[i];
+      }
+      for (int u = threadIdx.x; u < p.rep * kChunkTok; u += NT) {
+        const int r = u / kChunkTok, j = c0 + u % kChunkTok;
+        vmv_lds[u] = j < c1 ? p.vmv[(static_cast<int64_t>(h) * p.rep + r) * p.n + (j - p.rs)] : 0.0f;
+      }
+    }
+    __syncthreads();
+  }
+  int n_work = 0;                                        // groups with work so far (drop totals, LDS)
+  // weighted LDS form: this lane's token sums over the groups, tile by tile of the quad's half
+  float rA[kChunkTok / 32], rD[kChunkTok / 32];
 #pragma unroll
-        for (int hh = 0; hh < NH; ++hh) q[hh] = ops[(4 * hh + ks) * 64 + l];
-        const u32x4 mh = ops[(4 * NH + ks) * 64 + l], ml = ops[(4 * NH + 4 + ks) * 64 + l];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          sd[t] = tile_mfma<DT>(q[0], kop[t][ks][0], sd[t]);
-          ov[t] = tile_mfma<DT>(mh, vop[t][ks][0], ov[t]);
-          if constexpr (NH > 1) {
-            sd[t] = tile_mfma<DT>(q[0], kop[t][ks][1], sd[t]);
-            sd[t] = tile_mfma<DT>(q[1], kop[t][ks][0], sd[t]);
-            ov[t] = tile_mfma<DT>(mh, vop[t][ks][1], ov[t]);
-          }
-          ov[t] = tile_mfma<DT>(ml, vop[t][ks][0], ov[t]);
+  for (int it = 0; it < kChunkTok / 32; ++it) rA[it] = rD[it] = 0.0f;
+  for (int grp = ts; grp < p.G; grp += kTSplit) {
+    const int32_t* gt = p.gtab + kGT * grp;
+    const int row_base = gt[0], nq = gt[1], nq_pad = gt[2], te = gt[4], local = gt[5];
+    const int rows_g = p.rep * nq_pad;
+    const int64_t dd_at = ((static_cast<int64_t>(grp) * p.Hkv + h) * p.n_chunks + chunk) * kCWaves;
+    if (te <= c0) {                                      // the group does not reach this chunk
+      if constexpr (!WEIGHTED) {
+        if (quad == 0) {
+          for (int u = threadIdx.x; u < rows_g; u += kCThreads)
+            p.alpha_part[(static_cast<int64_t>(h) * p.n_chunks + chunk) * p.NR + row_base + u] = 0.0f;
+          if (threadIdx.x < kCWaves) p.ddpart[dd_at + threadIdx.x] = 0.0f;
         }
       }
-      // rows 4g + i: their values; lane (g, n) holds the products of those rows with token t0 + 16 t + n
-      const float4 m4 = *reinterpret_cast<const float4*>(meta + 4 * g);
-      const float4 i4 = *reinterpret_cast<const float4*>(meta + 16 + 4 * g);
-      const float4 o4 = *reinterpret_cast<const float4*>(meta + 32 + 4 * g);
-      const float4 c4 = *reinterpret_cast<const float4*>(meta + 48 + 4 * g);
-      const float rm[4] = {m4.x, m4.y, m4.z, m4.w}, ril[4] = {i4.x, i4.y, i4.z, i4.w};
-      const float omo[4] = {o4.x, o4.y, o4.z, o4.w}, msc[4] = {c4.x, c4.y, c4.z, c4.w};
-      auto terms = [&](auto edge) {
-        int far[4];
-        if constexpr (decltype(edge)::value) {
-          const int4 f4 = *reinterpret_cast<const int4*>(lim + 4 * g);
-          far[0] = f4.x; far[1] = f4.y; far[2] = f4.z; far[3] = f4.w;
+      continue;
+    }
+    if (WEIGHTED && p.gw[grp] == 0.0f) continue;        // N = 0: every term of the group is zero
+    if constexpr (LDS && !WEIGHTED) {
+      if ((n_work++ & 1) != quad) continue;              // the other quad's group
+    }
+    const int t_end = min(c1, te);
+    // the tiles of this quad: weighted LDS form, its half of the chunk
+    const int ta0 = LDS && WEIGHTED ? c0 + (kChunkTok / 2) * quad : c0;
+    const int ta1 = LDS && WEIGHTED ? min(t_end, ta0 + kChunkTok / 2) : t_end;
+    const float wq_w = (WEIGHTED ? p.gw[grp] : 1.0f) / static_cast<float>(nq);
+    float dsum = 0.0f;                                   // drop terms of this wavefront (pass A)
+    for (int rb0 = 0; rb0 < rows_g; rb0 += 64) {
+      const int rbl = rb0 + 16 * wq;                      // this wavefront's first row in the group
+      const bool act = rbl < rows_g;
+      const int r = act ? rbl / nq_pad : 0;
+      const int row0 = row_base + rbl;
+      // operands (lane n: row n of the block, channels 8g + 32 ks ..) as the A side of the products,
+      // the token tiles as the B side: the results hold rows 4g + i of token n in lane (g, n), so a
+      // token's sums over the rows are three in-lane adds and two cross-group steps, and a row's sums
+      // over the tokens stay in the lane until the block's end
+      u32x4 qop[4][NH], mop[4][2];
+      int pos[4];
+      float rm[4], ril[4], omo[4], msc[4];
+      if (act) {
+        // row n's operands and rows 4g + i's values, prepared once per row by cov_rowprep: one
+        // round of independent loads
+        (void)load_rows<DT>(p, h, row0, g, n, qop);
+        const u32x4* mp = reinterpret_cast<const u32x4*>(p.mop) + (static_cast<int64_t>(h) * p.NR + row0 + n) * 32;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          mop[ks][0] = mp[(ks * 4 + g) * 2];
+          mop[ks][1] = mp[(ks * 4 + g) * 2 + 1];
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int tok = 32 * wave + 16 * t + n;
-          const float vmv = vmv_lds[s & 1][tok];
-          float wt = 0.0f;
+        for (int i = 0; i < 4; ++i) {
+          const int row = row0 + 4 * g + i;
+          const float4 f = reinterpret_cast<const float4*>(p.rowf)[static_cast<int64_t>(h) * p.NR + row];
+          pos[i] = p.rowpos[row];
+          rm[i] = f.x;
+          ril[i] = f.y;
+          omo[i] = f.z;
+          msc[i] = f.w / cov_xs<DT>(p, 2);                  // v M o of the scaled values: exact
+        }
+      } else {
+        zero_ops<DT>(qop);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sd[t][i], qsc, -rm[i])) * ril[i];
-            float u2 = fmaxf(__builtin_fmaf(ov[t][i], msc[i], vmv) + omo[i], 0.0f);
-            if constexpr (decltype(edge)::value) {
-              const bool in = c0 + tok <= far[i];
-              pr = in ? pr : 0.0f;
-              u2 = in ? u2 : 0.0f;
-            }
-            // pr / b for b = max(1 - pr, 1e-6) in [1e-6, 1]: the reciprocal's quotient and one
-            // residual correction (no subnormal, infinite or zero operand can occur)
-            const float qb = fmaxf(1.0f - pr, 1e-6f), rb = __builtin_amdgcn_rcpf(qb);
-            const float q0 = pr * rb;
-            const float qd = __builtin_fmaf(__builtin_fmaf(-qb, q0, pr), rb, q0);
-            const float w = pr * pr;
-            rD[t] = __builtin_fmaf(qd * qd, u2, rD[t]);
-            rA[t] = __builtin_fmaf(w, u2, rA[t]);
-            alpha[i] = __builtin_fmaf(w, u2, alpha[i]);
-            wt = i == 0 ? w : wt + w;
+        for (int ks = 0; ks < 4; ++ks) mop[ks][0] = mop[ks][1] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          pos[i] = -1;
+          rm[i] = ril[i] = omo[i] = 0.0f;
+          msc[i] = 1.0f;
+        }
+      }
+      if constexpr (WEIGHTED && !LDS) {
+        for (int u = l; u < kChunkTok; u += 64) accW[wq][u] = 0.0f;
+        wave_lds_fence();
+      }
+      float alpha[4] = {0.0f, 0.0f, 0.0f, 0.0f};          // key-term mass of rows 4g + i (pass A)
+      // a tile's operands (key and value tiles, v M v of this lane's token); the next tile's are
+      // fetched as soon as the current tiles have entered the matrix products
+      const int64_t vmv_base = (static_cast<int64_t>(h) * p.rep + r) * p.n - p.rs;   // + token j
+      u32x4 kop[4][NH], vop[4][NH];
+      float vmv1;
+      auto load_t = [&](int t0) {
+        const int j = t0 + n;
+        if constexpr (LDS) {
+          const int row = t0 - c0 + n;                     // (t0 - c0) % 16 == 0: row & 15 == n
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) {
+            kop[ks][0] = kv_lds[row * 16 + ((4 * ks + g) ^ n)];
+            vop[ks][0] = kv_lds[(kChunkTok + row) * 16 + ((4 * ks + g) ^ n)];
           }
-          rW[t] += wt;
-          mass += wt;
+          vmv1 = (act && j < t_end) ? vmv_lds[r * kChunkTok + row] : 0.0f;
+        } else {
+          load_tile<DT>(rk, p.k_st, t0, g, n, kop, cov_xs<DT>(p, 1));
+          load_tile<DT>(rv, p.v_st, t0, g, n, vop, cov_xs<DT>(p, 2));
+          vmv1 = (act && j < t_end) ? p.vmv[vmv_base + j] : 0.0f;
         }
       };
-      if (t0 + 31 <= lim_min) terms(std::false_type{});
-      else terms(std::true_type{});
+      // the terms of (row 4g + i, token t0 + n) from the tile's products
+      auto terms = [&](int t0, const f32x4& s, const f32x4& ov, float vmv, float (&ta)[4], float (&td)[4],
+                       float (&tw)[4]) {
+        const int j = t0 + n;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool far = act && j < t_end && j <= pos[i] - local;
+          const float pr = far ? __builtin_amdgcn_exp2f(s[i] * qsc - rm[i]) * ril[i] : 0.0f;
+          const float u2 = far ? fmaxf(vmv - 2.0f * (ov[i] * msc[i]) + omo[i], 0.0f) : 0.0f;
+          // pr / b for b = max(1 - pr, 1e-6) in [1e-6, 1]: the reciprocal's quotient and one
+          // residual correction (no subnormal, infinite or zero operand can occur)
+          const float qb = fmaxf(1.0f - pr, 1e-6f), rb = __builtin_amdgcn_rcpf(qb);
+          const float q0 = pr * rb;
+          const float qd = __builtin_fmaf(__builtin_fmaf(-qb, q0, pr), rb, q0);
+          td[i] = qd * qd * u2;
+          ta[i] = pr * pr * u2;
+          tw[i] = pr * pr;
+        }
+      };
+      if constexpr (LDS && WEIGHTED) {
+        // the quad's eight tiles unrolled: token t0 + n's sums over the groups stay in registers, each
+        // lane's four rows apart from the other lane groups' until the workgroup ends (a masked token
+        // adds +0)
+        float wr[kChunkTok / 32];
+        if (ta0 < ta1) load_t(ta0);
+#pragma unroll
+        for (int it = 0; it < kChunkTok / 32; ++it) {
+          const int t0 = ta0 + 16 * it;
+          wr[it] = 0.0f;
+          if (t0 < ta1) {
+            const f32x4 s = tile_dots<DT, NH, NH>(qop, kop);
+            const f32x4 ov = tile_dots<DT, 2, NH>(mop, vop);
+            const float vmv = vmv1;
+            if (t0 + 16 < ta1) load_t(t0 + 16);
+            float ta[4], td[4], tw[4];
+            terms(t0, s, ov, vmv, ta, td, tw);
+            rA[it] += ((ta[0] + ta[1]) + (ta[2] + ta[3])) * wq_w;
+            rD[it] += ((td[0] + td[1]) + (td[2] + td[3])) * wq_w;
+            wr[it] = ((tw[0] + tw[1]) + (tw[2] + tw[3])) * wq_w;
+          }
+        }
+        // the block's read mass of token t0 + n: the four lane groups' rows added
+#pragma unroll
+        for (int it = 0; it < kChunkTok / 32; ++it) wr[it] = xsum32(xsum16(wr[it]));
+        if (solo) {
+          if (g == 0 && act) {
+#pragma unroll
+            for (int it = 0; it < kChunkTok / 32; ++it) wva_lds[r * kChunkTok + ta0 - c0 + 16 * it + n] += wr[it];
+          }
+        } else if (g == 0) {
+#pragma unroll
+          for (int it = 0; it < kChunkTok / 32; ++it) accW[wq][ta0 - c0 + 16 * it + n] = wr[it];
+        }
+      } else {
+        if (ta0 < ta1) load_t(ta0);
+        for (int t0 = ta0; t0 < ta1; t0 += 16) {
+          const f32x4 s = tile_dots<DT, NH, NH>(qop, kop);
+          const f32x4 ov = tile_dots<DT, 2, NH>(mop, vop);
+          const float vmv = vmv1;
+          if (t0 + 16 < ta1) load_t(t0 + 16);
+          const int j = t0 + n;
+          float ta[4], td[4], tw[4];
+          terms(t0, s, ov, vmv, ta, td, tw);
+          if constexpr (!WEIGHTED) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              dsum += td[i];
+              alpha[i] += ta[i];
+            }
+          } else {
+            // token t0 + n: its sums over the block's 16 rows (the lane's four, then the lane groups')
+            float sa = (ta[0] + ta[1]) + (ta[2] + ta[3]);
+            float sd = (td[0] + td[1]) + (td[2] + td[3]);
+            float sw = (tw[0] + tw[1]) + (tw[2] + tw[3]);
+            sa = xsum32(xsum16(sa));
+            sd = xsum32(xsum16(sd));
+            sw = xsum32(xsum16(sw));
+            if (g == 0 && act && j < t_end) {
+              accA[wq][j - c0] += sa * wq_w;
+              accD[wq][j - c0] += sd * wq_w;
+              accW[wq][j - c0] += sw * wq_w;
+            }
+          }
+        }
+      }
+      if constexpr (!WEIGHTED) {
+        // rows 4g + i: their key-term mass over this chunk (the 16 lanes of group g hold its tokens)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float a_row = row_sum16(alpha[i]);
+          if (act && n == 0)
+            p.alpha_part[(static_cast<int64_t>(h) * p.n_chunks + chunk) * p.NR + row0 + 4 * g + i] =
+                a_row / static_cast<float>(nq);
+        }
+      } else if (!solo) {
+        // the wavefronts' read masses into their query heads' rows of WVa, in wavefront order (LDS:
+        // kept in LDS until the workgroup ends, then stored once)
+        __syncthreads();
+        for (int u = threadIdx.x; u < t_end - c0; u += NT) {
+          for (int w = 0; w < kCWaves; ++w) {
+            const int rbw = rb0 + 16 * w;
+            if (rbw >= rows_g) break;
+            if constexpr (LDS)
+              wva_lds[(rbw / nq_pad) * kChunkTok + u] += accW[w][u];
+            else
+              p.WVa_part[((static_cast<int64_t>(ts) * p.Hkv + h) * p.rep + rbw / nq_pad) * p.n + (c0 + u - p.rs)] +=
+                  accW[w][u];
+          }
+        }
+        __syncthreads();
+      }
     }
-    if (R.totals) {
-      // the block's rows over this wavefront's tokens (the 16 lanes of group g hold them): the four rows
-      // are dealt to the lanes of a quad while they are added, lane n ends with row 4g + (n & 3)
-      const float a01 = (n & 1 ? alpha[1] : alpha[0]) + dpp<kQuadSwap1>(n & 1 ? alpha[0] : alpha[1]);
-      const float a23 = (n & 1 ? alpha[3] : alpha[2]) + dpp<kQuadSwap1>(n & 1 ? alpha[2] : alpha[3]);
-      float a = (n & 2 ? a23 : a01) + dpp<kQuadSwap2>(n & 2 ? a01 : a23);
-      a += dpp<kRowRor + 4>(a);
-      a += dpp<kRowRor + 8>(a);
-      mass = row_sum16(mass);
-      if (n < 4) red[s & 1][wave][4 * g + n] = a;
-      if (n == 0) red[s & 1][wave][16 + g] = mass;
-    }
-    last = block++;
-    if (--left > 0) continue;
-    ended = grp;
-    if (++grp < gb) {
-      left = blocks_of(grp);
-      block = first_of(grp);
+    if constexpr (!WEIGHTED) {
+      dsum = wave_sum(dsum);                             // cov_groups adds the four in order
+      if (l == 0) p.ddpart[dd_at + wq] = dsum;
     }
   }
-  flush(ended);
-  if (R.totals) {
+  if constexpr (WEIGHTED) {
+    if constexpr (LDS) {
+#pragma unroll
+      for (int it = 0; it < kChunkTok / 32; ++it) {
+        rA[it] = xsum32(xsum16(rA[it]));
+        rD[it] = xsum32(xsum16(rD[it]));
+      }
+      if (g == 0) {
+        const int tb = (kChunkTok / 2) * quad;
+#pragma unroll
+        for (int it = 0; it < kChunkTok / 32; ++it) {
+          accA[wq][tb + 16 * it + n] = rA[it];
+          accD[wq][tb + 16 * it + n] = rD[it];
+        }
+      }
+    }
     __syncthreads();
-    combine(nb - 1, last);
+    if constexpr (LDS) {
+      // this workgroup is the only writer of its (split, h, heads, chunk) read masses
+      for (int u = threadIdx.x; u < p.rep * kChunkTok; u += NT) {
+        const int r = u / kChunkTok, t = u % kChunkTok;
+        if (c0 + t < c1) p.WVa_part[((static_cast<int64_t>(ts) * p.Hkv + h) * p.rep + r) * p.n + (c0 + t - p.rs)] = wva_lds[u];
+      }
+    }
+    for (int u = threadIdx.x; u < c1 - c0; u += NT) {
+      const int64_t o = (static_cast<int64_t>(ts) * p.Hkv + h) * p.n + (c0 + u - p.rs);
+      p.A_part[o] = (accA[0][u] + accA[1][u]) + (accA[2][u] + accA[3][u]);
+      p.DD_part[o] = (accD[0][u] + accD[1][u]) + (accD[2][u] + accD[3][u]);
+    }
   }
-}
-
-// chunks that a group's keys reach (its partials exist for those)
-__device__ __forceinline__ int reached_chunks(const CovParams& p, int grp) {
-  return max(0, min(p.n_chunks, (p.gtab[kGT * grp + 4] - p.rs + kChunkTok - 1) / kChunkTok));
 }
 
 // N per group (over heads and chunks) -> weight 1 / N (0 if N = 0) in gw[group], and whether the
@@ -939,16 +1003,13 @@ __device__ __forceinline__ int reached_chunks(const CovParams& p, int grp) {
 __global__ __launch_bounds__(kCThreads) void cov_groups(CovParams p) {
   __shared__ float red[kCWaves];
   const int grp = blockIdx.x;
-  const int rc = reached_chunks(p, grp);
-  // the drop total of (group, h, chunk): cov_terms' wavefront partials, in order, over nq
+  const int per = p.Hkv * p.n_chunks;
+  // the drop total of (group, h, chunk): cov_terms' four wavefront partials, in order, over nq
   const float nq = static_cast<float>(p.gtab[kGT * grp + 1]);
   float s = 0.0f;
-  for (int u = threadIdx.x; u < p.Hkv * rc; u += kCThreads) {
-    const float* d = p.ddpart + ((static_cast<int64_t>(grp) * p.Hkv + u / rc) * p.n_chunks + u % rc) * kTW;
-    float t = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kTW; ++w) t += d[w];
-    s += t / nq;
+  for (int u = threadIdx.x; u < per; u += kCThreads) {
+    const float* d = p.ddpart + (static_cast<int64_t>(grp) * per + u) * kCWaves;
+    s += ((d[0] + d[1]) + (d[2] + d[3])) / nq;
   }
   s = wave_sum(s);
   if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = s;
@@ -960,57 +1021,19 @@ __global__ __launch_bounds__(kCThreads) void cov_groups(CovParams p) {
   }
 }
 
-// per row: its group's weight x its key-term mass, per block: its group's weight x its read mass (in the
-// four parts), summed over the chunks, a quarter of them per wavefront: the loads of one entry are a
-// chain of strided reads
+// per row: its group's weight x its key-term mass (summed over the chunks)
 __global__ __launch_bounds__(kCThreads) void cov_roww(CovParams p, const int32_t* rowgrp) {
-  __shared__ float part[4][64];
-  const int nb = p.NR / 16;
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x % 64;    // (h, block, entry)
-  const int qt = threadIdx.x / 64, i = static_cast<int>(t % kRowPart);
-  const bool in = t < static_cast<int64_t>(p.Hkv) * nb * kRowPart;
-  const int hb = in ? static_cast<int>(t / kRowPart) : 0, h = hb / nb, block = hb % nb, row = 16 * block + (i < 16 ? i : 0);
-  const int grp = in && p.rowpos[row] >= 0 ? rowgrp[row] : -1;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * kCThreads + threadIdx.x;
+  if (t >= static_cast<int64_t>(p.Hkv) * p.NR) return;
+  const int h = static_cast<int>(t / p.NR), row = static_cast<int>(t % p.NR);
+  const int grp = rowgrp[row];
+  if (grp < 0 || p.rowpos[row] < 0) {
+    p.roww[t] = 0.0f;
+    return;
+  }
   float a = 0.0f;
-  if (grp >= 0) {
-    const int rc = reached_chunks(p, grp);
-    const int e = rc * (qt + 1) / 4;
-    const float* src = p.row_part + (static_cast<int64_t>(h) * p.n_chunks * nb + block) * kRowPart + i;
-#pragma unroll 8
-    for (int c = rc * qt / 4; c < e; ++c) a += src[static_cast<int64_t>(c) * nb * kRowPart];
-  }
-  part[qt][threadIdx.x % 64] = a;
-  __syncthreads();
-  if (qt || !in) return;
-  const int x = threadIdx.x;
-  a = (part[0][x] + part[1][x]) + (part[2][x] + part[3][x]);
-  a = grp >= 0 ? a / static_cast<float>(p.gtab[kGT * grp + 1]) * p.gw[grp] : 0.0f;
-  if (i < 16) p.roww[static_cast<int64_t>(h) * p.NR + row] = a;
-  else p.omega[static_cast<int64_t>(hb) * 4 + i - 16] = a;
-}
-
-// the groups' stored token sums with their weights: A, DD and the read mass of the tokens
-// [store0, store0 + store_n), one thread per (h, token), groups in order
-__global__ __launch_bounds__(kCThreads) void cov_wsum(CovParams p, int store0, int store_n) {
-  const int per = (store_n + kCThreads - 1) / kCThreads;
-  const int h = blockIdx.x / per, at = blockIdx.x % per * kCThreads + static_cast<int>(threadIdx.x);
-  const int j = store0 + at;
-  if (at >= store_n || j >= p.re) return;
-  float a = 0.0f, dd = 0.0f, w = 0.0f;
-#pragma unroll 4
-  for (int grp = 0; grp < p.G; ++grp) {
-    const float gw = p.gw[grp];
-    if (j >= p.gtab[kGT * grp + 4] || gw == 0.0f) continue;   // N = 0: every term of the group is zero
-    const float wq = gw / static_cast<float>(p.gtab[kGT * grp + 1]);
-    const float* src = p.tsum + (static_cast<int64_t>(grp) * p.Hkv + h) * 3 * store_n + at;
-    a = __builtin_fmaf(src[0], wq, a);
-    dd = __builtin_fmaf(src[store_n], wq, dd);
-    w = __builtin_fmaf(src[2 * static_cast<int64_t>(store_n)], wq, w);
-  }
-  const int64_t o = static_cast<int64_t>(h) * p.n + (j - p.rs);
-  p.A[o] = a;
-  p.DD[o] = dd;
-  p.W[o] = w;
+  for (int c = 0; c < p.n_chunks; ++c) a += p.alpha_part[(static_cast<int64_t>(h) * p.n_chunks + c) * p.NR + row];
+  p.roww[t] = a * p.gw[grp];
 }
 
 // S[h] = sum over rows of roww * (scaling q)(scaling q)^T: per (h, 16 output rows, row split), 64
@@ -1080,21 +1103,16 @@ __global__ __launch_bounds__(kCThreads) void cov_smat_sum(CovParams p) {
 // finalisation sums: red[0..2] the means of the live-averaged A, DD, W; red[3] the live count;
 // red[4 + h rep + r] omega (live-averaged read mass per query head); red[4 + Hkv rep + h] sum_j A
 // (live-averaged).  First every per-head sum over the n tokens, one workgroup each (sums[h][0] A,
-// [1] DD, [2 + r] the read mass of query head r: its blocks' weighted masses), then one thread combines them in a fixed order.
-__global__ __launch_bounds__(1024) void cov_final_sums(CovParams p, const int32_t* rlist, int n_rlist) {
+// [1] DD, [2 + r] the read mass of query head r), then one thread combines them in a fixed order.
+__global__ __launch_bounds__(1024) void cov_final_sums(CovParams p) {
   __shared__ float part[16];
   const int nk = 2 + p.rep;
   const int h = blockIdx.x / nk, kind = blockIdx.x % nk;
+  const float* src = kind == 0 ? p.A + static_cast<int64_t>(h) * p.n
+                   : kind == 1 ? p.DD + static_cast<int64_t>(h) * p.n
+                               : p.WVa + (static_cast<int64_t>(h) * p.rep + (kind - 2)) * p.n;
   float v = 0.0f;
-  if (kind < 2) {
-    const float* src = (kind == 0 ? p.A : p.DD) + static_cast<int64_t>(h) * p.n;
-    for (int j = threadIdx.x; j < p.n; j += 1024) v += src[j];
-  } else {
-    // every 16th row of the head's list starts a block (a block's first row is never padding)
-    const int32_t* rl = rlist + static_cast<int64_t>(kind - 2) * n_rlist;
-    for (int x = threadIdx.x; x < n_rlist / 4; x += 1024)
-      v += p.omega[(static_cast<int64_t>(h) * (p.NR / 16) + rl[x / 4 * 16] / 16) * 4 + x % 4];
-  }
+  for (int j = threadIdx.x; j < p.n; j += 1024) v += src[j];
   v = wave_sum(v);
   if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = v;
   __syncthreads();
@@ -1138,9 +1156,12 @@ __global__ __launch_bounds__(kCThreads) void cov_final(CovParams p) {
   const int64_t nA = static_cast<int64_t>(p.Hkv) * p.n;
   const int64_t nS = static_cast<int64_t>(p.Hkv) * kCD * kCD;
   if (t < nA) {
+    const int h = static_cast<int>(t / p.n), j = static_cast<int>(t % p.n);
+    float w = 0.0f;
+    for (int r = 0; r < p.rep; ++r) w += p.WVa[(static_cast<int64_t>(h) * p.rep + r) * p.n + j];
     p.A[t] = p.A[t] / live + p.eta * p.red[0];
     p.DD[t] = p.DD[t] / live + p.eta * p.red[1];
-    p.W[t] = p.W[t] / live + p.eta * p.red[2];
+    p.W[t] = w / live + p.eta * p.red[2];
   }
   if (t < nS) {
     const int h = static_cast<int>(t / (kCD * kCD)), e = static_cast<int>(t % (kCD * kCD));
@@ -1163,23 +1184,17 @@ __global__ __launch_bounds__(kCThreads) void cov_final(CovParams p) {
 
 using namespace kvq;
 
-// tokens whose per-group sums are stored at once: whole chunks, all of them up to kStoreFloats
-static int64_t cov_store_tokens(int64_t Hkv, int64_t n, int64_t G) {
-  const int64_t all = (n + kChunkTok - 1) / kChunkTok, fit = kStoreFloats / (3 * G * Hkv * kChunkTok);
-  return std::max<int64_t>(1, std::min(all, fit)) * kChunkTok;
-}
-
-// workspace layout (floats): row_m, row_il, oMo, roww (Hkv NR each), omega (Hkv NR / 4); o (Hkv NR d); o_part (kOSplit Hkv
-// NR d); vmv (Hkv rep n); ddpart (G Hkv n_chunks kTW); gw (2 G + 1); red (4 + Hkv rep + Hkv); tsum (G Hkv 3
-// store tokens); row_part (Hkv n_chunks NR / 16 kRowPart), rec (Hkv NR / 16 records, fp32's the larger
-// ones), 16-byte aligned; S_part (kSSplit Hkv d d); sums (Hkv (2 + rep));
+// workspace layout (floats): row_m, row_il, oMo, roww (Hkv NR each); o (Hkv NR d); o_part (kOSplit Hkv
+// NR d); vmv (Hkv rep n); ddpart (G Hkv n_chunks 4); alpha_part (Hkv n_chunks NR); gw (2 G + 1); red (4 +
+// Hkv rep + Hkv); WVa (Hkv rep n); A_part, DD_part (kTSplit Hkv n each); WVa_part (kTSplit Hkv rep n);
+// mop (Hkv NR 128), rowf (Hkv NR 4), 16-byte aligned; S_part (kSSplit Hkv d d); sums (Hkv (2 + rep));
 // fp32 rows: partial maxima and scales (kAmaxFloats)
 extern "C" int64_t kvq_coverage_stats_workspace(int64_t Hkv, int64_t rep, int64_t n, int64_t NR, int64_t G) {
   if (Hkv <= 0 || rep <= 0 || n <= 0 || NR <= 0 || G <= 0) return -1;
   const int64_t nch = (n + kChunkTok - 1) / kChunkTok;
-  return 4 * Hkv * NR + Hkv * (NR / 4) + (1 + kOSplit) * Hkv * NR * kCD + Hkv * rep * n + G * Hkv * nch * kTW + Hkv * nch * (NR / 16) * kRowPart +
-         (2 * G + 1) + (4 + Hkv * rep + Hkv) + G * Hkv * 3 * cov_store_tokens(Hkv, n, G) +
-         Hkv * (NR / 16) * rec_units<KVQ_F32>() * 4 + 4 + kSSplit * Hkv * kCD * kCD + Hkv * (2 + rep) + kAmaxFloats;
+  return 4 * Hkv * NR + (1 + kOSplit) * Hkv * NR * kCD + Hkv * rep * n + G * Hkv * nch * kCWaves + Hkv * nch * NR + (2 * G + 1) +
+         (4 + Hkv * rep + Hkv) + Hkv * rep * n + kTSplit * (2 * Hkv * n + Hkv * rep * n) + 132 * Hkv * NR + 4 + kSSplit * Hkv * kCD * kCD + Hkv * (2 + rep) +
+         kAmaxFloats;
 }
 
 extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const int32_t* rowpos, const int32_t* rowgrp,
@@ -1221,18 +1236,20 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
   p.row_il = w; w += Hkv * NR;
   p.oMo = w; w += Hkv * NR;
   p.roww = w; w += Hkv * NR;
-  p.omega = w; w += Hkv * (NR / 4);
   p.o = w; w += Hkv * NR * kCD;
   p.o_part = w; w += kOSplit * Hkv * NR * kCD;
   p.vmv = w; w += Hkv * rep * n;
-  p.ddpart = w; w += G * Hkv * p.n_chunks * kTW;
+  p.ddpart = w; w += G * Hkv * p.n_chunks * kCWaves;
+  p.alpha_part = w; w += Hkv * p.n_chunks * NR;
   p.gw = w; w += 2 * G + 1;
   p.red = w; w += 4 + Hkv * rep + Hkv;
-  const int64_t store_tokens = cov_store_tokens(Hkv, n, G);
-  p.tsum = w; w += G * Hkv * 3 * store_tokens;
-  w += (4 - (reinterpret_cast<uintptr_t>(w) / 4) % 4) % 4;       // 16-byte alignment
-  p.row_part = w; w += Hkv * p.n_chunks * (NR / 16) * kRowPart;
-  p.rec = reinterpret_cast<uint32_t*>(w); w += Hkv * (NR / 16) * rec_units<KVQ_F32>() * 4;
+  p.WVa = w; w += Hkv * rep * n;
+  p.A_part = w; w += kTSplit * Hkv * n;
+  p.DD_part = w; w += kTSplit * Hkv * n;
+  p.WVa_part = w; w += kTSplit * Hkv * rep * n;
+  w += (4 - (reinterpret_cast<uintptr_t>(w) / 4) % 4) % 4;       // 16-byte alignment of the next two
+  p.mop = reinterpret_cast<uint32_t*>(w); w += 128 * Hkv * NR;
+  p.rowf = w; w += 4 * Hkv * NR;
   p.S_part = w; w += kSSplit * Hkv * kCD * kCD;
   p.sums = w; w += Hkv * (2 + rep);
   float* amax_part = w;                                       // fp32 rows: partial maxima, then scales
@@ -1260,36 +1277,42 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
   KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_vmv<DT_>),
                                                dim3(Hkv * rep * ((n + kVmvPer - 1) / kVmvPer)), blk, 0, s, p));
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(v M v)");
-  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_rowprep<DT_>), dim3(Hkv * (NR / 16)), blk, 0, s, p, rowgrp));
-  KVQ_LAUNCH_CHECK("kvq_coverage_stats(row records)");
-  // the terms of every chunk, the sums of the first store_tokens tokens kept; then, where the store
-  // holds no more, the further ranges' terms again, each read by cov_wsum before the next
-  const int range_chunks = static_cast<int>(store_tokens / kChunkTok);
-  for (int c = 0; c < p.n_chunks; c += range_chunks) {
-    const bool first = c == 0;
-    TermsRange R{c, first ? p.n_chunks : std::min(range_chunks, p.n_chunks - c), p.rs + c * kChunkTok,
-                 static_cast<int>(store_tokens), 1, first};
-    // a workgroup's start (its key and value tiles, the first record) costs about a block's time, so the
-    // groups of a chunk are cut into pieces only while the chip holds more workgroups (three per CU, two
-    // rounds, since the chunks' work differs): 8 heads x 32768 tokens, 4 pieces 763 us, 2 pieces 702, 1 705
-    while (R.pieces < 8 && Hkv * R.chunks * R.pieces < kTermsUnits) R.pieces *= 2;
-    KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_terms<DT_>), dim3(xcd_grid(Hkv * R.chunks * R.pieces)), dim3(64 * kTW),
-                                                 0, s, p, R));
-    KVQ_LAUNCH_CHECK("kvq_coverage_stats(terms)");
-    if (first) {
-      hipLaunchKernelGGL(cov_groups, dim3(static_cast<unsigned>(G)), blk, 0, s, p);
-      KVQ_LAUNCH_CHECK("kvq_coverage_stats(groups)");
-      hipLaunchKernelGGL(cov_roww, dim3((Hkv * (NR / 16) * kRowPart + 63) / 64), blk, 0, s, p, rowgrp);
-      KVQ_LAUNCH_CHECK("kvq_coverage_stats(row weights)");
-    }
-    hipLaunchKernelGGL(cov_wsum, dim3(Hkv * ((store_tokens + kCThreads - 1) / kCThreads)), blk, 0, s, p, R.store0, R.store_n);
-    KVQ_LAUNCH_CHECK("kvq_coverage_stats(weighted sums)");
+  const unsigned terms_blocks = xcd_grid(Hkv * p.n_chunks * kTSplit);
+  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_rowprep<DT_>), dim3((Hkv * NR + 15) / 16), blk, 0, s, p));
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(row operands)");
+  // 16-bit rows and up to kTermsLdsRep query heads per KV head: the chunk's rows staged in LDS, two
+  // quads of wavefronts
+  const bool terms_lds = dtype != KVQ_F32 && rep <= kTermsLdsRep;
+  const dim3 blk2(2 * kCThreads);
+  if (terms_lds) {
+    if (dtype == KVQ_BF16) hipLaunchKernelGGL((cov_terms<KVQ_BF16, false, true>), dim3(terms_blocks), blk2, 0, s, p);
+    else hipLaunchKernelGGL((cov_terms<KVQ_F16, false, true>), dim3(terms_blocks), blk2, 0, s, p);
+  } else {
+    KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_terms<DT_, false, false>), dim3(terms_blocks), blk, 0, s, p));
   }
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(terms)");
+  hipLaunchKernelGGL(cov_groups, dim3(static_cast<unsigned>(G)), blk, 0, s, p);
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(groups)");
+  hipLaunchKernelGGL(cov_roww, dim3((Hkv * NR + kCThreads - 1) / kCThreads), blk, 0, s, p, rowgrp);
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(row weights)");
+  // the read masses are accumulated by the weighted pass: cleared by a fill kernel (graph-capture safe)
+  const int64_t nwp = kTSplit * Hkv * rep * n;
+  hipLaunchKernelGGL(cov_clear, dim3((nwp + kCThreads - 1) / kCThreads), blk, 0, s, p.WVa_part, nwp);
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(clear)");
+  if (terms_lds) {
+    if (dtype == KVQ_BF16) hipLaunchKernelGGL((cov_terms<KVQ_BF16, true, true>), dim3(terms_blocks), blk2, 0, s, p);
+    else hipLaunchKernelGGL((cov_terms<KVQ_F16, true, true>), dim3(terms_blocks), blk2, 0, s, p);
+  } else {
+    KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_terms<DT_, true, false>), dim3(terms_blocks), blk, 0, s, p));
+  }
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(weighted terms)");
+  hipLaunchKernelGGL(cov_split_sums, dim3((Hkv * rep * n + kCThreads - 1) / kCThreads), blk, 0, s, p);
+  KVQ_LAUNCH_CHECK("kvq_coverage_stats(split sums)");
   KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_smat<DT_>), dim3(Hkv * (kCD / 16) * kSSplit), blk, 0, s, p));
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(S parts)");
   hipLaunchKernelGGL(cov_smat_sum, dim3((Hkv * kCD * kCD + kCThreads - 1) / kCThreads), blk, 0, s, p);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(S)");
-  hipLaunchKernelGGL(cov_final_sums, dim3(static_cast<unsigned>(Hkv * (2 + rep))), dim3(1024), 0, s, p, rlist, (int)n_rlist);
+  hipLaunchKernelGGL(cov_final_sums, dim3(static_cast<unsigned>(Hkv * (2 + rep))), dim3(1024), 0, s, p);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(sums)");
   hipLaunchKernelGGL(cov_final_combine, dim3(1), dim3(64), 0, s, p);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(combine)");

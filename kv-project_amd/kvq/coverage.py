@@ -3,7 +3,7 @@
 ``coverage_groups`` draws the observation positions on the host exactly as the reference does
 (numpy's PCG64 seeded by CRC32 keys; the draws are pinned by golden vectors of the reference).
 ``coverage_stats`` builds the row plan of those groups once per shape (int32 tables on the device)
-and runs ``kvq_coverage_stats``: no allocation, no host synchronisation, deterministic sums.
+and runs ``kvq_coverage_stats``: eleven launches, no host synchronisation, deterministic sums.
 """
 from __future__ import annotations
 

@@ -119,51 +119,3 @@ def test_coverage_window_only_and_deterministic():
     b = _run(q, k, v, M, 1200, 4, 1168)
     for name in ("A", "W", "DD", "S", "Mbar"):
         assert torch.equal(a[name], b[name]), name
-
-
-def test_coverage_token_ranges():
-    """More (group, token) sums than the workspace keeps at once (2^28 floats): a group of one query per
-    position, so the last chunks' sums are computed in a second range of tokens, and 15 of every 16 rows
-    are padding.  Reference: the oracle's formulas in float64 with every group a row.  Bar as above."""
-    from types import SimpleNamespace
-    import kvq
-    H, Hkv, rs, re, local = 3420, 8, 4, 3404, 64
-    q, k, v, M = (x.cuda() for x in _inputs(23, Hkv, Hkv, H, H, torch.bfloat16))
-    cfg = SimpleNamespace(STRATA_SEGMENT=1, STRATA_QUERIES=1, W_OBS=1)
-    st = kvq.coverage_stats(q, k, v, D ** -0.5, H, rs, re, M, cfg)
-    torch.cuda.synchronize()
-    pos = torch.tensor([int(g[0]) for g in st["groups"]], device="cuda")
-    print(f"coverage ranges: {len(pos)} groups", flush=True)
-    assert all(len(g) == 1 for g in st["groups"]) and 3 * len(pos) * Hkv * (re - rs) > 2 ** 28
-    ref = {n: [] for n in ("A", "DD", "W", "S")}
-    live = torch.zeros(len(pos), dtype=torch.float64, device="cuda")
-    terms = []
-    for h in range(Hkv):
-        qh, kh, vh, Mh = q[0, h, pos].double() * D ** -0.5, k[0, h].double(), v[0, h].double(), M[h].double()
-        s = qh @ kh.t()
-        p = s.masked_fill(torch.arange(H, device="cuda")[None] > pos[:, None], -torch.inf).softmax(-1)
-        o = p @ vh
-        far = pos - local
-        far[-1] = pos[-1] - 1                                        # the window group
-        j = torch.arange(rs, re, device="cuda")
-        pR = p[:, rs:re] * (j[None] <= far[:, None])
-        vR, oM = vh[rs:re], o @ Mh
-        u = (((vR @ Mh) * vR).sum(-1)[None] - 2 * oM @ vR.t() + (oM * o).sum(-1)[:, None]).clamp_min(0.0)
-        terms.append((qh, pR ** 2 * u, (pR / (1 - pR).clamp_min(1e-6)) ** 2 * u, pR ** 2))
-        live += terms[-1][2].sum(-1)
-    w = torch.where(live > 0, 1 / live.clamp_min(1e-300), 0.0)
-    n_live = float((live > 0).sum().clamp_min(1))
-    for qh, a, dd, r in terms:
-        A = w @ a / n_live
-        ref["A"].append(A)
-        ref["DD"].append(w @ dd / n_live)
-        ref["W"].append(w @ r / n_live)
-        ref["S"].append((qh * (a.sum(-1) * w)[:, None]).t() @ qh / n_live / A.sum().clamp_min(1e-30))
-    ref = {n: torch.stack(x) for n, x in ref.items()}
-    for n in ("A", "DD", "W"):
-        ref[n] = ref[n] + 1e-3 * ref[n].mean()
-    ref = {n: x.cpu().numpy() for n, x in ref.items()}
-    ref["Mbar"] = M.double().cpu().numpy()                            # one query head per KV head
-    for n in ("A", "W", "DD", "S"):
-        _check(st[n], ref, n, 2e-4)
-    _check(st["Mbar"], ref, "Mbar", 1e-5)
