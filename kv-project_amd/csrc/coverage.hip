@@ -268,21 +268,24 @@ __global__ __launch_bounds__(DT == KVQ_F32 ? kCThreads : 2 * kCThreads) void cov
   }
 }
 
-// values of one 32-key step in LDS: [key][channel].  fp32 rows are padded by 8 bytes against bank
-// conflicts; 16-bit rows take 288 bytes (72 words), so that the transposed reads of a channel block
-// (16 lanes reading 8 bytes each of 4 keys x 4 channel quads) fall on distinct banks
-template <int DT>
-constexpr int vrow_words() { return DT == KVQ_F32 ? (kCD * 4 + 8) / 4 : 72; }
-
 typedef short tr16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) tr16x4 lds_tr16x4;
 
+// The rows' attention outputs over one of kOSplit ranges of an item's 32-key steps.  The workgroup's keys and
+// values of a step come through LDS (two stages, the loads one more step ahead; fp32 rows as their fp16
+// parts, split once instead of by every wavefront), so a step is loaded from L2 once for its 64 rows and
+// costs one barrier.
+// Bound by the matrix cores (P enters as hi + lo parts), the exponentials and splits beside them and the LDS
+// reads of 16 rows a wavefront.  8 heads x 66 items, 32768 bf16 keys: 490 us; with every wavefront
+// loading its key tiles from L2 one step ahead and two barriers a step, 1065 (the same bits).
 template <int DT>
-__global__ __launch_bounds__(kCThreads) void cov_output(CovParams p) {
-  constexpr int ESZ = TileOps<DT>::ESZ;
-  constexpr int VRW = vrow_words<DT>();
-  constexpr int U16 = kCD * ESZ / 16;                        // 16-byte units of a value row
-  __shared__ __align__(16) uint32_t vt[32 * VRW];
+__global__ __launch_bounds__(kCThreads, DT == KVQ_F32 ? 2 : 3) void cov_output(CovParams p) {
+  constexpr int NH = TileOps<DT>::NH, ESZ = TileOps<DT>::ESZ;
+  // value rows of 288 bytes: the transposed reads of a channel block (16 lanes reading 8 bytes each of
+  // 4 keys x 4 channel quads) fall on distinct banks; key row j holds its 16-byte column c at c ^ (j & 15)
+  constexpr int VRW = 72;
+  __shared__ u32x4 kt[2][NH][32 * 16];
+  __shared__ __align__(16) uint32_t vt[2][NH][32 * VRW];
   const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
   // work units (h, item, key split), h outermost; the items in reverse plan order, so the groups at
   // the end of the context, whose keys reach furthest, start first and the short ones fill the tail
@@ -295,7 +298,7 @@ __global__ __launch_bounds__(kCThreads) void cov_output(CovParams p) {
   const int rows_g = p.rep * gt[2];
   const int row0 = gt[0] + 64 * rb + 16 * wave;
   const bool active = 64 * rb + 16 * wave < rows_g;        // inactive wavefronts still join the barriers
-  u32x4 qop[4][TileOps<DT>::NH];
+  u32x4 qop[4][NH];
   int pos = -1;
   if (active)
     pos = load_rows<DT>(p, h, row0, g, n, qop);
@@ -315,55 +318,68 @@ __global__ __launch_bounds__(kCThreads) void cov_output(CovParams p) {
   f32x4 acc[8];
 #pragma unroll
   for (int cb = 0; cb < 8; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // a step's loads: its 32 value rows (this thread's 16-byte units; rows at or past mmax as zeros:
-  // p = 0 there must not meet a NaN) and this wavefront's two key tiles.  The next step's loads go
-  // out as soon as the current key tiles have entered the logit products.
-  constexpr int KU = (32 * U16 + kCThreads - 1) / kCThreads;
-  u32x4 vr[KU];
-  u32x4 kr[2][4][TileOps<DT>::NH];
+  // thread t moves the 8-channel units t % 16 of keys t / 16 and 16 + t / 16 of a step (values at or past k1
+  // as zeros: p = 0 there must not meet a NaN)
+  u32x4 kx[2][NH], vx[2][NH];
+  const int sk = threadIdx.x / 16, sc = threadIdx.x % 16;
   auto load_step = [&](int t0) {
 #pragma unroll
-    for (int k = 0; k < KU; ++k) {
-      const int u = threadIdx.x + kCThreads * k;
-      const int key = u / U16, w16 = u % U16;
-      vr[k] = u32x4{0u, 0u, 0u, 0u};
-      if (u < 32 * U16 && t0 + key < k1)
-        vr[k] = __builtin_amdgcn_raw_buffer_load_b128(
-            rv, static_cast<int>((static_cast<int64_t>(t0 + key) * p.v_st) * ESZ + 16 * w16), 0, 0);
-    }
+    for (int i = 0; i < 2; ++i) {
+      const int key = t0 + 16 * i + sk;
+      const int ko = static_cast<int>((key * p.k_st + 8 * sc) * ESZ), vo = static_cast<int>((key * p.v_st + 8 * sc) * ESZ);
 #pragma unroll
-    for (int tau = 0; tau < 2; ++tau) load_tile<DT>(rk, p.k_st, t0 + 16 * tau, g, n, kr[tau], cov_xs<DT>(p, 1));
-  };
-  if (k0 < k1) load_step(k0);
-  for (int t0 = k0; t0 < k1; t0 += 32) {
-    // LDS-only barriers: the key tiles of the step stay in flight while its value rows are stored
-    block_lds_barrier();                                     // the previous step's value rows are read
-#pragma unroll
-    for (int k = 0; k < KU; ++k) {
-      const int u = threadIdx.x + kCThreads * k;
-      if (u < 32 * U16) {
-        uint32_t* dst = vt + (u / U16) * VRW + 4 * (u % U16);
-        if constexpr (DT == KVQ_F32) {
-          dst[0] = vr[k][0];
-          dst[1] = vr[k][1];
-          dst[2] = vr[k][2];
-          dst[3] = vr[k][3];
-        } else {
-          *reinterpret_cast<u32x4*>(dst) = vr[k];                // 288-byte rows: 16-byte aligned
-        }
+      for (int x = 0; x < NH; ++x) {
+        kx[i][x] = __builtin_amdgcn_raw_buffer_load_b128(rk, ko + 16 * x, 0, 0);
+        vx[i][x] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + 16 * x, 0, 0);
       }
     }
-    block_lds_barrier();
+  };
+  auto store_step = [&](int s) {                             // step s: keys k0 + 32 s ..
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int key = 16 * i + sk;
+      const bool in = k0 + 32 * s + key < k1;
+      u32x4 ko[NH], vo[NH];
+      if constexpr (NH == 2) {
+        float a[8], b[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          a[e] = __uint_as_float(kx[i][e / 4][e % 4]) * cov_xs<DT>(p, 1);
+          b[e] = in ? __uint_as_float(vx[i][e / 4][e % 4]) * vsc : 0.0f;
+        }
+        f32_parts<DT>(a, ko[0], ko[1]);
+        f32_parts<DT>(b, vo[0], vo[1]);
+      } else {
+        ko[0] = kx[i][0];
+        vo[0] = in ? vx[i][0] : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int x = 0; x < NH; ++x) {
+        kt[s & 1][x][16 * key + (sc ^ (key & 15))] = ko[x];
+        *reinterpret_cast<u32x4*>(&vt[s & 1][x][key * VRW + 4 * sc]) = vo[x];
+      }
+    }
+  };
+  if (k0 < k1) {
+    load_step(k0);
+    store_step(0);
+    load_step(k0 + 32);
+  }
+  for (int s = 0, t0 = k0; t0 < k1; ++s, t0 += 32) {
+    block_lds_barrier();                                     // step s is stored, step s - 1 read
+    store_step(s + 1);
+    load_step(t0 + 64);                                      // (past the keys: not used)
     // probabilities of the two 16-key tiles: lane (g, n) holds keys t0 + 4g + i and t0 + 16 + 4g + i
     // of row n
-    f32x4 dd[2];
-#pragma unroll
-    for (int tau = 0; tau < 2; ++tau) dd[tau] = tile_dots<DT, TileOps<DT>::NH, TileOps<DT>::NH>(kr[tau], qop);
-    if (t0 + 32 < k1) load_step(t0 + 32);
     float pr[8];
 #pragma unroll
     for (int tau = 0; tau < 2; ++tau) {
-      const f32x4 d = dd[tau];
+      u32x4 kop[4][NH];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int x = 0; x < NH; ++x) kop[ks][x] = kt[s & 1][x][16 * (16 * tau + n) + ((4 * ks + g) ^ n)];
+      const f32x4 d = tile_dots<DT, NH, NH>(kop, qop);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int j = t0 + 16 * tau + 4 * g + i;
@@ -373,36 +389,25 @@ __global__ __launch_bounds__(kCThreads) void cov_output(CovParams p) {
     // A operand: row n, k-index 8g + kk <-> key kk < 4 ? 4g + kk : 16 + 4g + kk - 4 (hi and lo parts)
     u32x4 ph, pl;
     f32_parts<DT>(pr, ph, pl);
-    // B operand per 16-channel block cb: lane (g, n) holds the values of those keys at channel 16cb + n
+    // B operand per 16-channel block cb: lane (g, n) holds the values of those keys at channel 16cb + n, by LDS
+    // transpose reads (ds_read_b64_tr_b16): within each 16-lane group, lane n receives element n & 3 of the
+    // 8-byte loads of lanes (n >> 2) + 4 j, j = 0..3.  Lane (g, q + 4 j) therefore points at key 4g + j (then
+    // 16 + 4g + j), channels 16 cb + 4q .. + 3, and lane (g, n) receives keys 4g .. 4g + 3 (16 + 4g ..)
+    const uint32_t* a0 = &vt[s & 1][0][(4 * g + (n >> 2)) * VRW + 2 * (n & 3)];
 #pragma unroll
     for (int cb = 0; cb < 8; ++cb) {
-      const int c = 16 * cb + n;
-      if constexpr (DT == KVQ_F32) {
-        float x[8];
+      u32x4 vb[NH];
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          const int key = kk < 4 ? 4 * g + kk : 16 + 4 * g + kk - 4;
-          x[kk] = __uint_as_float(vt[key * VRW + c]) * vsc;
-        }
-        u32x4 vh, vl;
-        f32_parts<DT>(x, vh, vl);
-        acc[cb] = tile_mfma<DT>(ph, vh, acc[cb]);
-        acc[cb] = tile_mfma<DT>(pl, vh, acc[cb]);
-        acc[cb] = tile_mfma<DT>(ph, vl, acc[cb]);
-      } else {
-        // LDS transpose reads (ds_read_b64_tr_b16): within each 16-lane group, lane n receives
-        // element n & 3 of the 8-byte loads of lanes (n >> 2) + 4 j, j = 0..3.  Lane (g, q + 4 j)
-        // therefore points at key 4g + j (then 16 + 4g + j), channels 16 cb + 4q .. + 3, and lane
-        // (g, n) receives keys 4g .. 4g + 3 (16 + 4g ..) of channel 16 cb + n: the B operand
-        const int src_key = 4 * g + (n >> 2), src_ch = 16 * cb + 4 * (n & 3);
-        const uint32_t* a0 = vt + src_key * VRW + src_ch / 2;
-        const tr16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a0));
-        const tr16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a0 + 16 * VRW));
+      for (int x = 0; x < NH; ++x) {
+        const uint32_t* a = a0 + x * 32 * VRW + 8 * cb;
+        const tr16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a));
+        const tr16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr16x4*)(a + 16 * VRW));
         const uint2 lw = __builtin_bit_cast(uint2, lo), hw = __builtin_bit_cast(uint2, hi);
-        const u32x4 vb = u32x4{lw.x, lw.y, hw.x, hw.y};
-        acc[cb] = tile_mfma<DT>(ph, vb, acc[cb]);
-        acc[cb] = tile_mfma<DT>(pl, vb, acc[cb]);
+        vb[x] = u32x4{lw.x, lw.y, hw.x, hw.y};
       }
+      acc[cb] = tile_mfma<DT>(ph, vb[0], acc[cb]);
+      acc[cb] = tile_mfma<DT>(pl, vb[0], acc[cb]);
+      if constexpr (NH == 2) acc[cb] = tile_mfma<DT>(ph, vb[1], acc[cb]);
     }
   }
   if (!active) return;

@@ -94,6 +94,17 @@ def test_coverage_stats_matches_oracle(case):
     _compare(st, _oracle(q, k, v, M, H, rs, re))
 
 
+@pytest.mark.parametrize("dtype,H", [(torch.bfloat16, 101), (torch.float16, 129), (torch.float32, 161),
+                                     (torch.bfloat16, 223), (torch.float32, 545)])
+def test_coverage_outputs_at_range_edges(dtype, H):
+    """Contexts whose key ranges hold no, one or two 32-key steps, the last of them partial; the rows behind
+    the context are NaN, which a zero probability must not meet."""
+    q, k, v, M = _inputs(H, 4, 2, H + 40, H, dtype, True)
+    print(f"coverage range edges: H {H} {dtype}", flush=True)
+    st = _run(q, k, v, M, H, 4, H - 32)
+    _compare(st, _oracle(q, k, v, M, H, 4, H - 32))
+
+
 @pytest.mark.parametrize("qs,ks,vs", [(2.0 ** -17, 2.0 ** 17, 2.0 ** 17), (2.0 ** 20, 2.0 ** -20, 2.0 ** -20),
                                       (2.0 ** -122, 1.0, 1.0)])
 def test_coverage_stats_fp32_extreme_magnitudes(qs, ks, vs):
