@@ -430,39 +430,45 @@ __global__ __launch_bounds__(kCThreads, DT == KVQ_F32 ? 2 : 3) void cov_output(C
 // split into parts, y = x M by the products hi*hi + hi*lo + lo*hi (fp32 accumulation, about 2^-22
 // relative), and x . y by a row sum with x exchanged through the wavefront's LDS into the layout
 // of the products' output.
-constexpr int kVmvPer = 512;             // values of a cov_vmv workgroup
+// Bound by the latencies between its steps: the metric's 68 KiB leave room for one workgroup a CU, so it has
+// eight wavefronts, two per SIMD (32 query heads x 32732 values: 139 us; four
+// wavefronts 217, the same bits).
+constexpr int kVmvPer = 512;             // values of a cov_vmv workgroup, or twice as many where that fills the CUs
+constexpr int kVmvWaves = 8;
+constexpr int kVmvThreads = 64 * kVmvWaves;
 constexpr int kMtStride = kCD + 8;       // halves per LDS row of M^T (16-byte aligned rows)
 
 template <int DT>
-__global__ __launch_bounds__(kCThreads) void cov_vmv(CovParams p) {
+__global__ __launch_bounds__(kVmvThreads) void cov_vmv(CovParams p, int per) {
   __shared__ __align__(16) uint16_t mt[2][kCD * kMtStride];   // [part][col][k]
-  __shared__ __align__(16) float xs[kCWaves][16][kCD + 4];
-  __shared__ float red[kCWaves];
-  __shared__ int xex[kCWaves][16];
-  const int tiles = (p.n + kVmvPer - 1) / kVmvPer;
+  __shared__ __align__(16) float xs[kVmvWaves][16][kCD + 4];
+  __shared__ float red[kVmvWaves];
+  __shared__ int xex[kVmvWaves][16];
+  const int tiles = (p.n + per - 1) / per;
   const int hr = blockIdx.x / tiles, tile = blockIdx.x % tiles;
   const int h = hr / p.rep;
   const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, n = l & 15;
   // the metric's largest entry over the workgroup, then its transposed parts
   const float* Mg = p.M + static_cast<int64_t>(hr) * kCD * kCD;
-  constexpr int kPer = kCD * kCD / kCThreads;
+  constexpr int kPer = kCD * kCD / kVmvThreads;
   float mv[kPer];
   float mx = 0.0f;
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
-    mv[e] = Mg[threadIdx.x + kCThreads * e];
+    mv[e] = Mg[threadIdx.x + kVmvThreads * e];
     mx = fmaxf(mx, fabsf(mv[e]));
   }
   mx = wave_max(mx);
   if (l == 0) red[wave] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+  for (int i = 0; i < kVmvWaves; ++i) mx = fmaxf(mx, red[i]);
   int em = 0;
   if (mx > 0.0f) (void)frexpf(mx, &em);
   const float upm = ldexpf(1.0f, 8 - em);
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
-    const int idx = threadIdx.x + kCThreads * e, k = idx / kCD, c = idx % kCD;
+    const int idx = threadIdx.x + kVmvThreads * e, k = idx / kCD, c = idx % kCD;
     const float x = mv[e] * upm;
     const _Float16 hi = static_cast<_Float16>(x);
     const _Float16 lo = static_cast<_Float16>(x - static_cast<float>(hi));
@@ -470,8 +476,8 @@ __global__ __launch_bounds__(kCThreads) void cov_vmv(CovParams p) {
     mt[1][c * kMtStride + k] = __builtin_bit_cast(uint16_t, lo);
   }
   __syncthreads();
-  for (int t0 = 0; t0 < kVmvPer; t0 += 64) {
-    const int j0 = tile * kVmvPer + t0 + 16 * wave;         // this wavefront's 16 values
+  for (int t0 = 0; t0 < per && tile * per + t0 < p.n; t0 += 16 * kVmvWaves) {
+    const int j0 = tile * per + t0 + 16 * wave;         // this wavefront's 16 values
     const int j = j0 + n;                                   // lane (g, n): value n, channels 32 ks + 8 g ..
     float x[4][8];
 #pragma unroll
@@ -1279,8 +1285,9 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
   hipLaunchKernelGGL((cov_metric<KVQ_F32, true>), dim3(Hkv * rep * ((n_rlist + kMetricRows - 1) / kMetricRows)), blk,
                      0, s, p, rlist, (int)n_rlist);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(o M)");
-  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_vmv<DT_>),
-                                               dim3(Hkv * rep * ((n + kVmvPer - 1) / kVmvPer)), blk, 0, s, p));
+  const int64_t vmv_per = Hkv * rep * ((n + 2 * kVmvPer - 1) / (2 * kVmvPer)) >= 256 ? 2 * kVmvPer : kVmvPer;
+  KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_vmv<DT_>), dim3(Hkv * rep * ((n + vmv_per - 1) / vmv_per)),
+                                               dim3(kVmvThreads), 0, s, p, static_cast<int>(vmv_per)));
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(v M v)");
   const unsigned terms_blocks = xcd_grid(Hkv * p.n_chunks * kTSplit);
   KVQ_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((cov_rowprep<DT_>), dim3((Hkv * NR + 15) / 16), blk, 0, s, p));

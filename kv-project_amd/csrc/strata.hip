@@ -221,12 +221,14 @@ using namespace kvq;
 // ---- distortion table of the compression side (STRATA_KV.py:1543-1559) ----
 // Metric in the code basis, written transposed: out[h] = (R (R S[h]^T)^T ... ) computed as
 // rot(rows of (rot(rows of S))^T) = R S^T R^T, whose quadratic form equals that of R S R^T.
-// One block per matrix; both passes through LDS.
-__global__ __launch_bounds__(256) void strata_metric_kernel(const float* __restrict__ S, const float* __restrict__ signs,
-                                                            float* __restrict__ out) {
+// One block per matrix, the keys' and the values' (grid.y) in one launch; both passes through LDS.
+__global__ __launch_bounds__(256) void strata_metric_kernel(const float* __restrict__ S, const float* __restrict__ Mbar,
+                                                            const float* __restrict__ signs, float* __restrict__ out_k,
+                                                            float* __restrict__ out_v) {
   __shared__ float a[kSD][kSD + 1];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const float* src = S + static_cast<int64_t>(blockIdx.x) * kSD * kSD;
+  const float* src = (blockIdx.y == 0 ? S : Mbar) + static_cast<int64_t>(blockIdx.x) * kSD * kSD;
+  float* const out = blockIdx.y == 0 ? out_k : out_v;
   const float inv = 0.08838834764831845f;         // float32(1 / sqrt(128))
   for (int pass = 0; pass < 2; ++pass) {
     float r0[kSD / 4], r1[kSD / 4];
@@ -271,38 +273,55 @@ struct ErrWidths {
 // (largest entry to [128, 256)), and y = e M comes from the products hi*hi + hi*lo + lo*hi in fp32
 // (about 2^-22 relative); e . y is a row sum, e exchanged through the wavefront's LDS into the
 // layout of the products' output.
+// Bound by the codec's arithmetic (96 IEEE quotients a lane and tile) and the latencies around it: the metric's
+// 68 KiB leave room for one workgroup a CU, so it has eight wavefronts, two per SIMD, and both sides go in
+// one launch (8 heads x 32732 tokens a side, three widths: 271 us; two launches of four wavefronts
+// 359, the same bits).  A workgroup stages the metric for kSErrTok tokens, or for twice as many where
+// that still fills the CUs.
 constexpr int kSErrTok = 512;
+constexpr int kSErrWaves = 8;
+constexpr int kSErrThreads = 64 * kSErrWaves;
 constexpr int kSMtStride = kSD + 8;              // halves per LDS row of M^T (16-byte aligned rows)
 
-__global__ __launch_bounds__(256) void strata_err_mfma(const float* __restrict__ y, int64_t n,
-                                                       const float* __restrict__ Mt, ErrWidths w,
-                                                       float* __restrict__ err) {
+struct ErrSide {
+  const float* y;                                // (BH, n, d) rotated rows
+  const float* Mt;                               // (BH, d, d)
+  float* err;                                    // (BH, n, widths)
+};
+
+__global__ __launch_bounds__(kSErrThreads) void strata_err_mfma(ErrSide keys, ErrSide values, int64_t n, int tok,
+                                                                ErrWidths w) {
+  const ErrSide side = blockIdx.z == 0 ? keys : values;
+  const float* __restrict__ y = side.y;
+  const float* __restrict__ Mt = side.Mt;
+  float* __restrict__ err = side.err;
   __shared__ __align__(16) uint16_t mt[2][kSD * kSMtStride];  // [part][col][k]
-  __shared__ __align__(16) float es[4][16][kSD + 4];
-  __shared__ float red[4];
-  __shared__ int eex[4][16];
+  __shared__ __align__(16) float es[kSErrWaves][16][kSD + 4];
+  __shared__ float red[kSErrWaves];
+  __shared__ int eex[kSErrWaves][16];
   const int wave = threadIdx.x / 64, l = threadIdx.x % 64, g = l >> 4, nl = l & 15;
   const int64_t bh = blockIdx.y;
   // M's largest entry over the workgroup, then its transposed parts
   const float* mg = Mt + bh * kSD * kSD;
-  constexpr int kPer = kSD * kSD / 256;
+  constexpr int kPer = kSD * kSD / kSErrThreads;
   float mv[kPer];
   float mx = 0.0f;
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
-    mv[e] = mg[threadIdx.x + 256 * e];
+    mv[e] = mg[threadIdx.x + kSErrThreads * e];
     mx = fmaxf(mx, fabsf(mv[e]));
   }
   mx = wave_max(mx);
   if (l == 0) red[wave] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+  for (int i = 0; i < kSErrWaves; ++i) mx = fmaxf(mx, red[i]);
   int em = 0;
   if (mx > 0.0f) (void)frexpf(mx, &em);
   const float upm = ldexpf(1.0f, 8 - em);
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
-    const int idx = threadIdx.x + 256 * e, k = idx / kSD, c = idx % kSD;
+    const int idx = threadIdx.x + kSErrThreads * e, k = idx / kSD, c = idx % kSD;
     const float x = mv[e] * upm;
     const _Float16 hi = static_cast<_Float16>(x);
     const _Float16 lo = static_cast<_Float16>(x - static_cast<float>(hi));
@@ -310,8 +329,8 @@ __global__ __launch_bounds__(256) void strata_err_mfma(const float* __restrict__
     mt[1][c * kSMtStride + k] = __builtin_bit_cast(uint16_t, lo);
   }
   __syncthreads();
-  const int64_t t_end = min<int64_t>(n, static_cast<int64_t>(blockIdx.x + 1) * kSErrTok);
-  for (int64_t t0 = static_cast<int64_t>(blockIdx.x) * kSErrTok + 16 * wave; t0 < t_end; t0 += 64) {
+  const int64_t t_end = min<int64_t>(n, static_cast<int64_t>(blockIdx.x + 1) * tok);
+  for (int64_t t0 = static_cast<int64_t>(blockIdx.x) * tok + 16 * wave; t0 < t_end; t0 += 16 * kSErrWaves) {
     const int64_t t = t0 + nl;                                  // this lane's token
     float yv[32];
     const bool ok = t < t_end;
@@ -1379,11 +1398,10 @@ extern "C" int kvq_strata_distortion(const float* yk, const float* yv, int64_t H
   float* mv = mk + Hkv * kSD * kSD;
   float* ek = mv + Hkv * kSD * kSD;
   float* ev = ek + Hkv * n * nbits;
-  hipLaunchKernelGGL(strata_metric_kernel, dim3(static_cast<unsigned>(Hkv)), dim3(256), 0, st, S, signs, mk);
-  hipLaunchKernelGGL(strata_metric_kernel, dim3(static_cast<unsigned>(Hkv)), dim3(256), 0, st, Mbar, signs, mv);
-  const dim3 eg(static_cast<unsigned>((n + kSErrTok - 1) / kSErrTok), static_cast<unsigned>(Hkv));
-  hipLaunchKernelGGL(strata_err_mfma, eg, dim3(256), 0, st, yk, n, mk, w, ek);
-  hipLaunchKernelGGL(strata_err_mfma, eg, dim3(256), 0, st, yv, n, mv, w, ev);
+  hipLaunchKernelGGL(strata_metric_kernel, dim3(static_cast<unsigned>(Hkv), 2), dim3(256), 0, st, S, Mbar, signs, mk, mv);
+  const int tok = 2 * Hkv * ((n + 2 * kSErrTok - 1) / (2 * kSErrTok)) >= 256 ? 2 * kSErrTok : kSErrTok;
+  const dim3 eg(static_cast<unsigned>((n + tok - 1) / tok), static_cast<unsigned>(Hkv), 2);
+  hipLaunchKernelGGL(strata_err_mfma, eg, dim3(kSErrThreads), 0, st, ErrSide{yk, mk, ek}, ErrSide{yv, mv, ev}, n, tok, w);
   const int64_t total = Hkv * n;
   hipLaunchKernelGGL(strata_dtable_kernel, dim3(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 4096))),
                      dim3(256), 0, st, ek, ev, A, W, DD, nbits, total, D);

@@ -88,10 +88,13 @@ def strata_center_rotate(x: torch.Tensor, signs: Optional[torch.Tensor] = None):
     _lib.require_gpu(x)
     B, H, n, d = x.shape
     signs = rotation_signs(d, device=x.device) if signs is None else signs
-    x = x.contiguous()
+    # a range of one sequence's tokens is read where it lies: dense rows, a stride of its own from head to head
+    if not (B == 1 and n > 1 and x.stride(3) == 1 and x.stride(2) == d and (H == 1 or x.stride(1) >= n * d)):
+        x = x.contiguous()
+    x_bh = x.stride(1) if H > 1 else n * d
     mu = torch.empty((B, H, d), dtype=torch.float16, device=x.device)
     y = torch.empty((B, H, n, d), dtype=torch.float32, device=x.device)
-    _lib.call("kvq_strata_center_rotate", x.data_ptr(), _lib.DTYPE_CODE[x.dtype], B * H, n, d, n * d,
+    _lib.call("kvq_strata_center_rotate", x.data_ptr(), _lib.DTYPE_CODE[x.dtype], B * H, n, d, x_bh,
               signs.data_ptr(), mu.data_ptr(), y.data_ptr(), _lib.stream_of(x))
     return mu, y
 

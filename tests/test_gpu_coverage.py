@@ -105,6 +105,14 @@ def test_coverage_outputs_at_range_edges(dtype, H):
     _compare(st, _oracle(q, k, v, M, H, 4, H - 32))
 
 
+def test_coverage_many_heads():
+    """Enough (query head, value) work for 1024 values a workgroup of the v M v pass, the last one ragged."""
+    q, k, v, M = _inputs(5, 64, 8, 3150, 3150, torch.bfloat16)
+    print("coverage many heads: Hq 64 Hkv 8 H 3150", flush=True)
+    st = _run(q, k, v, M, 3150, 4, 3118)
+    _compare(st, _oracle(q, k, v, M, 3150, 4, 3118))
+
+
 @pytest.mark.parametrize("qs,ks,vs", [(2.0 ** -17, 2.0 ** 17, 2.0 ** 17), (2.0 ** 20, 2.0 ** -20, 2.0 ** -20),
                                       (2.0 ** -122, 1.0, 1.0)])
 def test_coverage_stats_fp32_extreme_magnitudes(qs, ks, vs):

@@ -219,3 +219,45 @@ def test_strata_decode_class_plan(B, T, fracs):
     out = kvq.strata_decode(q.cuda(), d ** -0.5, cache).float().cpu().numpy()
     ref = _oracle_out(cache, q, K, V, W, d ** -0.5)
     assert float(np.abs(out - ref).max()) <= 1e-2
+
+
+@pytest.mark.parametrize("n", [2, 301, 1500])
+def test_center_rotate_reads_ranges_where_they_lie(n):
+    """A range of tokens (a stride of its own from head to head), a slice of heads, repeated heads and a
+    two-sequence range give what their dense copies give."""
+    import kvq
+    x = (torch.randn((2, 4, n + 9, 128), generator=torch.Generator().manual_seed(n)) * 3).to(torch.bfloat16).cuda()
+    for v in (x[:1, :, 4:4 + n], x[1:, 1:2, :n], x[1:, 1:3, 9:], x[:1, :1, 2:2 + n].expand(1, 3, n, 128), x[:, :, 4:4 + n],
+              x[:1, :, :2 * (n // 2):2]):
+        for a, b in zip(kvq.strata_center_rotate(v), kvq.strata_center_rotate(v.clone(memory_format=torch.contiguous_format))):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,n", [(3, 1), (2, 130), (4, 1025), (8, 15500)])
+def test_distortion_table_is_per_token(H, n):
+    """A token's errors depend on its rows alone, so the table of a range of tokens is that range of the table,
+    wherever the workgroups' and wavefronts' shares end (the largest takes 1024 tokens a workgroup)."""
+    import ctypes
+    import kvq
+    from kvq import _lib
+    from kvq.strata import rotation_signs
+    g = torch.Generator(device="cuda").manual_seed(n)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")
+    yk, yv, A, W, DD = r(H, n, 128), r(H, n, 128), r(H, n).abs(), r(H, n).abs(), r(H, n).abs()
+    S, M = (torch.matmul(x.transpose(1, 2).contiguous(), x).contiguous() for x in (r(H, 128, 128), r(H, 128, 128)))
+    signs, bits = rotation_signs(128, device=yk.device), (2, 4, 8)
+    steps = (ctypes.c_float * 3)(*[kvq.uniform_step(b)[0] for b in bits])
+
+    def table(a, b):
+        m = b - a
+        c = [t[:, a:b].contiguous() for t in (yk, yv, A, W, DD)]
+        D = torch.empty((H, m, 5), device="cuda")
+        ws = torch.empty(int(_lib.load().kvq_strata_distortion_workspace(H, m, 3)) // 4 + 1, device="cuda")
+        _lib.call("kvq_strata_distortion", c[0].data_ptr(), c[1].data_ptr(), H, m, 128, S.data_ptr(), M.data_ptr(),
+                  signs.data_ptr(), c[2].data_ptr(), c[3].data_ptr(), c[4].data_ptr(), 3, (ctypes.c_int * 3)(*bits), steps,
+                  D.data_ptr(), ws.data_ptr(), ws.numel() * 4, _lib.stream_of(yk))
+        return D
+
+    whole = table(0, n)
+    for a, b in {(0, 1), (n - 1, n), (n // 3, n // 3 + min(n - n // 3, 37)), (max(0, n - 700), n)}:
+        assert torch.equal(whole[:, a:b], table(a, b)), (a, b)
