@@ -1032,9 +1032,10 @@ __global__ __launch_bounds__(kCThreads) void cov_groups(CovParams p) {
   }
 }
 
-// per row: its group's weight x its key-term mass (summed over the chunks)
-__global__ __launch_bounds__(kCThreads) void cov_roww(CovParams p, const int32_t* rowgrp) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kCThreads + threadIdx.x;
+// per row: its group's weight x its key-term mass (summed over the chunks in order, sixteen loads in flight: 8 x
+// 4224 rows, 128 chunks 8 us, one at a time 48)
+__global__ __launch_bounds__(64) void cov_roww(CovParams p, const int32_t* rowgrp) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
   if (t >= static_cast<int64_t>(p.Hkv) * p.NR) return;
   const int h = static_cast<int>(t / p.NR), row = static_cast<int>(t % p.NR);
   const int grp = rowgrp[row];
@@ -1042,8 +1043,17 @@ __global__ __launch_bounds__(kCThreads) void cov_roww(CovParams p, const int32_t
     p.roww[t] = 0.0f;
     return;
   }
+  const float* part = p.alpha_part + static_cast<int64_t>(h) * p.n_chunks * p.NR + row;
   float a = 0.0f;
-  for (int c = 0; c < p.n_chunks; ++c) a += p.alpha_part[(static_cast<int64_t>(h) * p.n_chunks + c) * p.NR + row];
+  int c = 0;
+  for (; c + 16 <= p.n_chunks; c += 16) {
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = part[static_cast<int64_t>(c + i) * p.NR];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) a += x[i];
+  }
+  for (; c < p.n_chunks; ++c) a += part[static_cast<int64_t>(c) * p.NR];
   p.roww[t] = a * p.gw[grp];
 }
 
@@ -1305,7 +1315,7 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(terms)");
   hipLaunchKernelGGL(cov_groups, dim3(static_cast<unsigned>(G)), blk, 0, s, p);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(groups)");
-  hipLaunchKernelGGL(cov_roww, dim3((Hkv * NR + kCThreads - 1) / kCThreads), blk, 0, s, p, rowgrp);
+  hipLaunchKernelGGL(cov_roww, dim3((Hkv * NR + 63) / 64), dim3(64), 0, s, p, rowgrp);
   KVQ_LAUNCH_CHECK("kvq_coverage_stats(row weights)");
   // the read masses are accumulated by the weighted pass: cleared by a fill kernel (graph-capture safe)
   const int64_t nwp = kTSplit * Hkv * rep * n;

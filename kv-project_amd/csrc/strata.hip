@@ -100,8 +100,17 @@ __global__ __launch_bounds__(1024) void strata_mean_part_kernel(const void* __re
 __global__ __launch_bounds__(kSD) void strata_mean_combine_kernel(const double* __restrict__ part, int P, int64_t n,
                                                                   uint16_t* __restrict__ mu) {
   const int c = threadIdx.x;
+  const double* x = part + static_cast<int64_t>(blockIdx.x) * P * kSD + c;
   double sum = 0.0;
-  for (int p = 0; p < P; ++p) sum += part[(static_cast<int64_t>(blockIdx.x) * P + p) * kSD + c];
+  int p = 0;
+  for (; p + 16 <= P; p += 16) {                  // in order, sixteen loads in flight (64 partials: 4 us, one at a time 17)
+    double v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = x[(p + i) * kSD];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum += v[i];
+  }
+  for (; p < P; ++p) sum += x[p * kSD];
   mu[static_cast<int64_t>(blockIdx.x) * kSD + c] = f32_to_f16(as_stored16(static_cast<float>(sum / static_cast<double>(n))));
 }
 
