@@ -134,7 +134,11 @@ int kvq_vmeta_tile(const uint16_t* lo, const uint16_t* scale, int64_t BH, int64_
  *    Every packed row is visible to every query.
  * out: (B, Tq, Hq, d) of out_dtype, contiguous (the reference's output layout).
  * workspace: float32 scratch of kvq_kivi_decode_workspace(...) floats (split partials).  Calls
- *    sharing one workspace must not overlap in time (same stream, or ordered streams).
+ *    sharing one workspace must not overlap in time (same stream, or ordered streams).  With packed
+ *    rows (n_q > 0) the size for n_exact rows holds every step over fewer exact rows too (as does
+ *    kvq_kivi_score_workspace's), so a token loop sizes it once, for its last step.  A workspace of at
+ *    least the size for n_exact = 0 serves every n_exact <= 1024, except beside a class plan (one full
+ *    round of packed splits): what it has no room for is attended by another placement of the exact rows.
  * split_tokens: target packed tokens per workgroup (the packed rows of each (b,h) are cut into
  *    ceil(n_q / split_tokens) splits of equal 32-token chunk counts; 0 = automatic: the split
  *    count whose launch fills whole rounds of resident workgroups).
@@ -206,7 +210,7 @@ int kvq_exact_append(const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st, co
  * partials and row statistics live in a static device array of KVQ_NOALLOC_SCRATCH_FLOATS
  * floats (8 MiB), one copy per GPU, held until the process ends; its device address is looked
  * up on the first call on each device.  The stream must belong to the current device.  A step
- * whose kvq_kivi_decode_workspace(...) exceeds KVQ_NOALLOC_SCRATCH_FLOATS is rejected
+ * whose partials exceed KVQ_NOALLOC_SCRATCH_FLOATS is rejected
  * (KVQ_EINVAL) before any launch (C2, the 8B-shape layer at batch 16 and 32k tokens, needs
  * 400,384).  Nothing in the scratch has to start at zero: every partial and statistic the merge
  * and the score pass read is written earlier in the same call.  The scratch keeps the last

@@ -1195,6 +1195,7 @@ int launch(DecodeParams& p, int phases, hipStream_t stream) {
 
 struct SplitPlan {
   int n_exact_wg, n_split, split_tokens, S1, R, fused_per, exact_rows, classes, exact_inline;
+  int room;                        // exact-row blocks per (b, h) that fit beside the packed blocks
 };
 
 constexpr int kCUs = 256;          // MI355X compute units
@@ -1256,26 +1257,45 @@ inline SplitPlan plan_split(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int6
   } else {
     sp.n_exact_wg = (n_exact == 0 || sp.fused_per > 0 || exact_in_merge(n_exact))
                         ? 0 : plan_exact_blocks(B * Hkv, n_exact, &sp.exact_rows);
-    // A small step leaves resident slots empty: there the window goes to exact-row blocks of the same launch
-    // (16 to 64 rows each), which run beside the packed blocks, where the fused pass runs after each
-    // block's stream (split of 2905 packed + 96 exact rows, 8 (b, h), group 32: 8 query rows 11.7 -> 9.1 us,
-    // 4 rows 8.1 -> 5.8, 1 row 5.6 -> 4.6; the packed rows alone 7.8, 5.9, 4.6).  Only while the row's partials
-    // stay within the one-wavefront merge.
-    if (sp.fused_per > 0) {
-      const int64_t slots = static_cast<int64_t>(kCUs) * resident_blocks / std::max<int64_t>((bhn + 7) / 8 * 8, 1);
-      const int64_t room = std::min<int64_t>(slots, kWaveMergePartials) - ns;
-      const int64_t nb = std::min<int64_t>(room, (n_exact + 15) / 16);
-      const int64_t rows = nb > 0 ? ((n_exact + nb - 1) / nb + 15) / 16 * 16 : 0;
-      if (rows > 0 && rows <= 64) {
-        sp.fused_per = 0;
-        sp.exact_inline = 1;
-        sp.exact_rows = static_cast<int>(rows);
-        sp.n_exact_wg = static_cast<int>((n_exact + rows - 1) / rows);
-      }
-    }
+  }
+  sp.room = 0;
+  if (sp.classes == 0 && ns > 0) {
+    const int64_t slots = static_cast<int64_t>(kCUs) * resident_blocks / std::max<int64_t>((bhn + 7) / 8 * 8, 1);
+    sp.room = static_cast<int>(std::max<int64_t>(0, std::min<int64_t>(slots, kWaveMergePartials) - ns));
   }
   sp.S1 = sp.n_exact_wg + sp.n_split;
   return sp;
+}
+
+// A small step leaves resident slots empty: there the window goes to exact-row blocks of the same launch
+// (16 to 64 rows each), which run beside the packed blocks, where the fused pass runs after each
+// block's stream (split of 2905 packed + 96 exact rows, 8 (b, h), group 32: 8 query rows 11.7 -> 9.1 us,
+// 4 rows 8.1 -> 5.8, 1 row 5.6 -> 4.6; the packed rows alone 7.8, 5.9, 4.6).  Only while the row's partials
+// stay within the one-wavefront merge.  Its partials need workspace that the fused pass does not.
+inline bool place_beside(SplitPlan* sp, int64_t n_exact) {
+  if (sp->fused_per == 0) return false;
+  const int64_t nb = std::min<int64_t>(sp->room, (n_exact + 15) / 16);
+  const int64_t rows = nb > 0 ? ((n_exact + nb - 1) / nb + 15) / 16 * 16 : 0;
+  if (rows == 0 || rows > 64) return false;
+  sp->fused_per = 0;
+  sp->exact_inline = 1;
+  sp->exact_rows = static_cast<int>(rows);
+  sp->n_exact_wg = static_cast<int>((n_exact + rows - 1) / rows);
+  sp->S1 = sp->n_exact_wg + sp->n_split;
+  return true;
+}
+
+// Workspace floats of S1 partials per (b, h) and row, and the rows' statistics.
+inline int64_t plan_floats(int64_t BH, int64_t S1, int R) { return BH * (S1 * R * (kD + 2) + 2 * R); }
+
+// The most partials per (b, h) of a step over n_exact rows or fewer, for a packed cache: the blocks beside the
+// packed ones are at most `room`, of 16 rows or more; blocks of a longer window (or of one beside a
+// class plan) at most what plan_exact_blocks takes before it rounds its rows up.
+inline int64_t most_partials(const SplitPlan& sp, int64_t BH, int64_t n_exact) {
+  if (sp.n_split == 0 || n_exact == 0) return sp.S1;
+  int64_t most = std::min<int64_t>(sp.room, (n_exact + 15) / 16);
+  if (sp.n_exact_wg > 0) most = std::max(most, most_exact_blocks(BH, n_exact));
+  return std::max<int64_t>(sp.S1, sp.n_split + most);
 }
 
 // ---- the allocation-free entry point's scratch ------------------------------------------------
@@ -1342,7 +1362,7 @@ extern "C" int64_t kvq_kivi_decode_workspace(int64_t B, int64_t Hq, int64_t Hkv,
   if (d != kD || B <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Tq <= 0 || group_k <= 0) return -1;
   if (group_v != 32 && group_v != 64 && group_v != 128) return -1;
   const SplitPlan sp = plan_split(B, Hq, Hkv, Tq, n_q, n_exact, split_tokens, group_k, group_v);
-  return B * Hkv * (static_cast<int64_t>(sp.S1) * sp.R * (kD + 2) + 2 * sp.R);
+  return plan_floats(B * Hkv, most_partials(sp, B * Hkv, n_exact), sp.R);
 }
 
 // A scored step's workspace: the decode's, then its logits (32 R floats per 32-token chunk and
@@ -1395,8 +1415,15 @@ int kivi_decode_at(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64
   KVQ_REQUIRE((exact_pos == nullptr) == (q_pos == nullptr && q_at == nullptr),
               "kvq_kivi_decode: exact_pos and q_pos go together");
   KVQ_REQUIRE(n_q < (1LL << 31) && B * Hkv < 65536, "kvq_kivi_decode: sizes out of range");
-  const SplitPlan sp = plan_split(B, Hq, Hkv, Tq, n_q, n_exact, split_tokens, group_k, group_v);
-  const int64_t need = B * Hkv * (static_cast<int64_t>(sp.S1) * sp.R * (kD + 2) + 2 * sp.R);
+  SplitPlan sp = plan_split(B, Hq, Hkv, Tq, n_q, n_exact, split_tokens, group_k, group_v);
+  int64_t need = plan_floats(B * Hkv, sp.S1, sp.R);
+  // the window beside the packed blocks where the workspace holds its partials: one that holds the fused
+  // pass's alone is not too small
+  SplitPlan beside = sp;
+  if (place_beside(&beside, n_exact) && workspace_floats >= plan_floats(B * Hkv, beside.S1, beside.R)) {
+    sp = beside;
+    need = plan_floats(B * Hkv, sp.S1, sp.R);
+  }
   KVQ_REQUIRE(static_cast<int64_t>(sp.S1) * R_real <= 16384, "kvq_kivi_decode: too many splits");
   KVQ_REQUIRE(workspace_floats >= need, "kvq_kivi_decode: workspace too small (%lld < %lld floats)",
               (long long)workspace_floats, (long long)need);
@@ -1610,8 +1637,13 @@ extern "C" int kvq_kivi_decode_noalloc(const void* q, int q_dtype, int64_t q_sb,
                                        const int64_t* q_pos, void* out, int out_dtype, float* scores,
                                        int64_t scores_bh, float score_weight, int64_t split_tokens,
                                        int phases, void* stream) {
-  // shapes the planner rejects fall through to kvq_kivi_decode, which names what is wrong
-  const int64_t need = kvq_kivi_decode_workspace(B, Hq, Hkv, Tq, d, n_q, n_exact, group_k, group_v, split_tokens);
+  // shapes the planner rejects fall through to kvq_kivi_decode, which names what is wrong; the others need the
+  // partials of the plan itself (a scratch without room for exact-row blocks beside them still does)
+  int64_t need = kvq_kivi_decode_workspace(B, Hq, Hkv, Tq, d, n_q, n_exact, group_k, group_v, split_tokens);
+  if (need >= 0) {
+    const SplitPlan sp = plan_split(B, Hq, Hkv, Tq, n_q, n_exact, split_tokens, group_k, group_v);
+    need = plan_floats(B * Hkv, sp.S1, sp.R);
+  }
   KVQ_REQUIRE(need <= kScratchFloats,
               "kvq_kivi_decode_noalloc: this step needs %lld scratch floats, more than the static scratch of "
               "%lld (call kvq_kivi_decode with a workspace instead)", (long long)need, (long long)kScratchFloats);

@@ -48,10 +48,13 @@ inline bool exact_in_merge(int64_t n_exact) { return n_exact > 0 && n_exact <= k
 // Exact-row blocks of a window attended neither by packed splits nor by the merge: about one round
 // of 768 workgroups over the BH (b, h) pairs, at least kExactRowsPerBlock rows each, rows per block
 // a multiple of 16.  Returns the blocks per (b, h); *rows receives the rows of each block.
-inline int plan_exact_blocks(int64_t BH, int64_t n_exact, int* rows) {
+inline int64_t most_exact_blocks(int64_t BH, int64_t n_exact) {
   const int64_t per_bh = std::max<int64_t>(1, 768 / std::max<int64_t>(BH, 1));
   const int64_t most = (n_exact + kExactRowsPerBlock - 1) / kExactRowsPerBlock;
-  const int64_t nb = std::max<int64_t>(1, std::min(per_bh, most));
+  return std::max<int64_t>(1, std::min(per_bh, most));
+}
+inline int plan_exact_blocks(int64_t BH, int64_t n_exact, int* rows) {
+  const int64_t nb = most_exact_blocks(BH, n_exact);
   const int64_t r = ((n_exact + nb - 1) / nb + 15) / 16 * 16;
   *rows = static_cast<int>(r);
   return static_cast<int>((n_exact + r - 1) / r);

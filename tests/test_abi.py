@@ -3,6 +3,8 @@ with the ctypes signatures the Python side binds (no compute call: that needs a 
 import re
 from pathlib import Path
 
+import pytest
+
 ROOT = Path(__file__).resolve().parents[1]
 
 
@@ -64,6 +66,18 @@ def test_split_plan_fills_one_round():
     assert lib.kvq_kivi_decode_workspace(1, 8, 8, 1, 128, 0, 100, 32, 32, 0) == 8 * (0 * 1 * (d + 2) + 2)
     assert lib.kvq_kivi_decode_workspace(1, 8, 8, 1, 128, 0, 2304, 32, 32, 0) == 8 * (36 * 1 * (d + 2) + 2)
     assert lib.kvq_kivi_decode_workspace(1, 8, 8, 1, 128, 64, 0, 32, 32, 0) == 8 * (1 * 1 * (d + 2) + 2)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Tq,n_q", [(1, 8, 8, 1, 3968), (1, 32, 8, 1, 1000), (1, 4, 1, 2, 40), (2, 16, 8, 1, 3001),
+                                             (1, 64, 8, 1, 9000), (16, 32, 8, 1, 32640), (4, 32, 8, 2, 2048)])
+def test_decode_workspace_holds_every_shorter_window(B, Hq, Hkv, Tq, n_q):
+    """A token loop sizes its workspace once, for its last step: no smaller n_exact needs more, scored or not."""
+    from kvq import _lib
+    lib = _lib.load()
+    for size in (lib.kvq_kivi_decode_workspace, lib.kvq_kivi_score_workspace):
+        for group_v in (32, 64, 128):
+            need = [size(B, Hq, Hkv, Tq, 128, n_q, n, 64, group_v, 0) for n in range(0, 4200)]
+            assert need[0] > 0 and all(a <= b for a, b in zip(need, need[1:]))
 
 
 def test_noalloc_rejects_steps_beyond_the_static_scratch():

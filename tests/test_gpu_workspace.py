@@ -62,3 +62,32 @@ def test_coded_decodes_any_workspace(dtype, B, Hkv, rep, Tq, T, window):
                                                                   (2, order[..., n // 2:].contiguous())])
     _same(lambda ws: kvq.strata_decode(q, 0.1, s, workspace=ws),
           kvq.strata_workspace_floats(B, Hq, Hkv, Tq, 128, s.n_exact, [t.n for t in s.tiers], [t.bits for t in s.tiers]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Hkv,rep,T,last", [(1, 8, 4, 1384, 384), (1, 8, 1, 4352, 384), (2, 3, 2, 700, 200)])
+def test_kivi_decode_workspace_sized_once(dtype, B, Hkv, rep, T, last):
+    """A workspace of the last step's size serves every step before it, and one that holds the packed splits'
+    partials alone serves them all: the window then goes where it needs no partials of its own.  The
+    placements agree to rounding (fp32 sums, then one rounding to the output type)."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(T)
+    c = kvq.PackedKIVICache.from_context(_rows(g, B, Hkv, T, 128, dtype=dtype), _rows(g, B, Hkv, T, 128, dtype=dtype),
+                                         window=last, group_k=64, group_v=64)
+    q = _rows(g, B, Hkv * rep, 1, 128, dtype=dtype)
+    size = lambda n: (B, Hkv * rep, Hkv, 1, 128, c.n_q, n, 64, 64)
+    end = torch.empty((kvq.workspace_floats(*size(last)),), device="cuda")
+    end_s = torch.empty((kvq.score_workspace_floats(*size(last)),), device="cuda")
+    few = torch.empty((kvq.workspace_floats(*size(0)),), device="cuda")
+    few_s = torch.empty((kvq.score_workspace_floats(*size(0)),), device="cuda")
+    atol = 1e-5 if dtype == torch.float32 else 2 ** -8
+    for n in sorted({1, 16, 17, 40, 128, last - 1, last}):
+        c.n_exact = n
+        want, score = kvq.kivi_decode(q, 0.1, c), torch.zeros((B, Hkv, c.n_q), device="cuda")
+        assert torch.equal(kvq.kivi_decode(q, 0.1, c, workspace=end), want)
+        torch.testing.assert_close(kvq.kivi_decode(q, 0.1, c, workspace=few), want, rtol=0, atol=atol)
+        assert torch.equal(kvq.kivi_decode(q, 0.1, c, scores=score), want)
+        for ws in (end, end_s, few, few_s):
+            s = torch.zeros_like(score)
+            torch.testing.assert_close(kvq.kivi_decode(q, 0.1, c, workspace=ws, scores=s), want, rtol=0, atol=atol)
+            torch.testing.assert_close(s, score, rtol=1e-5, atol=1e-9)
