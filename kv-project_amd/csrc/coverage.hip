@@ -1240,6 +1240,9 @@ extern "C" int kvq_coverage_stats(const void* qr, int dtype, int64_t NR, const i
                   reinterpret_cast<uintptr_t>(qr) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(M) % 16 == 0 && k_st >= kCD && v_st >= kCD,
               "kvq_coverage_stats: rows must be 16-byte aligned and not overlap");
+  // Loads run ahead of the keys, to key T + 94 at most (cov_output's step t0 + 64).  A buffer offset is an unsigned
+  // 32-bit one, and (T + 96) rows span less than twice (T + 48) rows: it stays below 4 GiB without wrapping,
+  // and past the end of the head's rows it reads zeros.
   KVQ_REQUIRE((T + 48) * std::max(k_st, v_st) * esz < (1LL << 31), "kvq_coverage_stats: one head's rows must span < 2 GiB");
   const int64_t n = re - rs;
   const int64_t need = kvq_coverage_stats_workspace(Hkv, rep, n, NR, G);

@@ -105,6 +105,23 @@ def test_coverage_outputs_at_range_edges(dtype, H):
     _compare(st, _oracle(q, k, v, M, H, 4, H - 32))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_coverage_widest_rows(dtype):
+    """Rows as far apart as one head's 2 GiB allow: loads that run ahead of the keys form offsets past 2 GiB, which
+    must read as zeros.  The memory between the rows is NaN."""
+    H, esz = 161, torch.empty((), dtype=dtype).element_size()
+    st = ((1 << 31) // esz // (H + 48) - 1) // 8 * 8
+    q, k, v, M = _inputs(3, 4, 1, H, H, dtype)
+    buf = torch.full((H * st,), float("nan"), dtype=dtype, device="cuda")
+    kd, vd = (buf[o:].as_strided((1, 1, H, D), (H * st, H * st, st, 1)) for o in (0, 256))
+    kd.copy_(k)
+    vd.copy_(v)
+    print(f"coverage widest rows: H {H} stride {st} {dtype}", flush=True)
+    import kvq
+    st_ = kvq.coverage_stats(q.cuda(), kd, vd, D ** -0.5, H, 4, H - 32, M.cuda())
+    _compare(st_, _oracle(q, k, v, M, H, 4, H - 32))
+
+
 def test_coverage_many_heads():
     """Enough (query head, value) work for 1024 values a workgroup of the v M v pass, the last one ragged."""
     q, k, v, M = _inputs(5, 64, 8, 3150, 3150, torch.bfloat16)
