@@ -100,7 +100,8 @@ def test_step_in_a_graph():
     (1, 1, 2, 1, 5000, 800),                                                                      # in the merge
 ])
 def test_window_placements_match_dense_attention(B, Hkv, rep, Tq, T, window):
-    """fp32 steps over packed and exact rows, appended ones causal, wherever the plan attends the window."""
+    """fp32 steps over packed and exact rows, appended ones causal, wherever the plan attends the window.  The bar is that of
+    the packed codes; single exact rows are held by test_every_exact_row_counts_once."""
     import kvq
     g = torch.Generator(device="cuda").manual_seed(T + window)
     f32 = torch.float32
@@ -111,3 +112,45 @@ def test_window_placements_match_dense_attention(B, Hkv, rep, Tq, T, window):
     at = torch.arange(T, T + Tq)
     got, want = st.attend(q, 128 ** -0.5, at), st.reference_attend(q, 128 ** -0.5, at)
     assert float((got - want).abs().max()) <= 2e-3                   # the fp32 bar of every decode
+
+
+@pytest.mark.parametrize("B,Hkv,rep,Tq,T,n_exact", [
+    (1, 8, 1, 1, 4096, 16), (1, 8, 1, 1, 4096, 17), (1, 8, 1, 1, 4096, 128), (1, 8, 1, 1, 4096, 129),    # 16-row blocks beside
+    (1, 8, 1, 1, 4240, 272), (1, 8, 1, 1, 4240, 273), (1, 8, 1, 1, 4480, 512), (1, 8, 1, 1, 4481, 513),  # 16 -> 32 rows .. 64
+    (2, 3, 4, 2, 900, 33), (1, 5, 3, 1, 700, 250), (1, 1, 8, 1, 300, 31),
+    (12, 8, 4, 1, 4096, 60), (14, 8, 2, 1, 3000, 101),                                                   # in the packed blocks
+    (16, 8, 4, 1, 2176, 129),                                                                            # beside a class plan
+    (1, 1, 2, 1, 5000, 800), (1, 2, 1, 1, 3000, 1300),                                                   # merge; blocks of their own
+])
+def test_every_exact_row_counts_once(B, Hkv, rep, Tq, T, n_exact):
+    """Queries that lean on the exact rows alone (their keys point along the queries, the packed ones away), each
+    with its own value: a row lost, counted twice or read from elsewhere moves the output by its share of
+    the mass times its distance from the mean, several times the bar.  Against float64 attention over
+    the exact rows; the packed rows' mass is below n_q e^-24."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(n_exact)
+    f32 = torch.float32
+    u = torch.full((128,), 128 ** -0.5, device="cuda")
+    K = 0.02 * _rows(g, B, Hkv, T, 128, dtype=f32) - 12.0 * u
+    V = _rows(g, B, Hkv, T, 128, dtype=f32)
+    W = n_exact - Tq
+    K[:, :, T - W:] += 24.0 * u
+    st = kvq.KIVIState(K, V, window=W, group_k=32, group_v=32, extra=Tq)
+    k1, v1 = 0.02 * _rows(g, B, Hkv, Tq, 128, dtype=f32) + 12.0 * u, _rows(g, B, Hkv, Tq, 128, dtype=f32)
+    at = torch.arange(T, T + Tq)
+    st.append(k1, v1, at)
+    assert st.cache.n_exact == n_exact
+    q = 0.02 * _rows(g, B, Hkv * rep, Tq, 128, dtype=f32) + 1.0 * u
+    got = st.attend(q, 1.0, at).transpose(1, 2).double()                                       # (B, Hq, Tq, d)
+    ke, ve = (torch.cat(x, 2).double().repeat_interleave(rep, 1) for x in ((K[:, :, T - W:], k1), (V[:, :, T - W:], v1)))
+    s = q.double() @ ke.transpose(-1, -2).contiguous()
+    hidden = torch.arange(n_exact, device="cuda")[None, :] > W + torch.arange(Tq, device="cuda")[:, None]
+    p = s.masked_fill(hidden, float("-inf")).softmax(-1)
+    want = p @ ve
+    # what the least of the visible rows moves: p_i |v_i - out| in the channel where it shows most
+    moved = (p[..., None] * (ve[:, :, None] - want[:, :, :, None]).abs()).amax(-1)
+    least = float(moved.masked_fill(hidden, float("inf")).min())
+    # the kernel's own error: logits near 12 to 2^-20, sums of at most 1300 products to 1300 2^-24 of their mean size
+    err = float((got - want).abs().max())
+    print(f"n_exact {n_exact}: err {err:.2e}, least row {least:.2e}", flush=True)
+    assert err <= 0.1 * least
