@@ -254,7 +254,8 @@ def kivi_decode(q: torch.Tensor, scaling: float, cache: PackedKIVICache, *,
 
     With ``q_pos`` (Tq,) int64 and ``cache.exact_pos`` set, exact row i is visible to query t iff
     exact_pos[i] <= q_pos[t] (the causal rule of chunked_attention among appended rows); every
-    packed row is visible.  A ``q_pos`` in host memory goes with the launch by value (no upload).  ``phases`` 1/2 run only the split / merge kernel (timing).
+    packed row is visible.  A ``q_pos`` in host memory goes with the launch by value (no upload; a captured
+    graph keeps those values).  ``phases`` 1/2 run only the split / merge kernel (timing).
 
     ``scores`` (B, Hkv, >= n_q) float32 on the GPU: the step also adds ``score_weight`` times the
     probability mass each packed token received from the query heads of its KV group (the
