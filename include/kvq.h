@@ -151,7 +151,8 @@ int kvq_vmeta_tile(const uint16_t* lo, const uint16_t* scale, int64_t BH, int64_
  *    With a workspace of at least kvq_kivi_score_workspace(...) floats, a scored step's split
  *    kernel also spills its logits (fp32, into the workspace after the partials) and the scores
  *    come from them in one light pass; with kvq_kivi_decode_workspace(...) floats the score pass
- *    reads the keys again.  Both give the same scores bit for bit.
+ *    reads the keys again (unless this step's own partials leave the logits room).  Both give the same
+ *    scores bit for bit.
  * phases (bit mask): 1 = split kernel (partials of the packed splits and the exact rows into the
  *    workspace; with scores and a score workspace, the logits too); 2 = merge kernel (log-sum-exp
  *    merge, output write, and each row's global max/sum into the workspace); 4 = score pass (needs

@@ -25,7 +25,8 @@
 // Both logit passes stream their split's keys through LDS (KeyStream): the four wavefronts of a workgroup hold
 // the operands of 64 rows each and share every key.  What bounds them: the exp2 of every (row, key)
 // pair at a quarter of the vector rate and the products themselves (at 4 x 8 x 65536 bf16 keys and 256 rows
-// each, 137 GFLOP and 0.54 GB a pass: statistics 154 us, columns 153, 131 without the exponentials; a large
+// each, 137 GFLOP and 0.54 GB a pass: statistics 154 us, columns 153 (153 and 152 at best in a trace, 164 and
+// 161 on average over 150 passes), 131 without the exponentials; a large
 // library product reaches 1.26 PFLOP/s here, which is 109 us).  With each wavefront loading its tiles from
 // L2, one ahead, they took 242 and 288.  Eight wavefronts of 32 rows 153 and 157, stages of 128 keys 163
 // and 161.

@@ -50,9 +50,9 @@ def test_split_plan_fills_one_round():
     """Automatic split (16x8 (b, h), 32640 packed + 128 exact tokens, 3 resident blocks per CU on
     256 CUs): 6 packed splits per (b, h) = 768 blocks, one round, so the plan is class-major and the
     128 window rows go to 2 exact-row blocks of 64 rows per (b, h) in the same launch.  Off that
-    one-round shape, exact windows of at most 1024 rows are attended by the merge (no exact-row
-    blocks, no partials); longer ones are blocks of 64 rows dispatched after the packed blocks.  The
-    workspace holds S1 * rows * (d + 2) + 2 * rows floats per (b, h), S1 = exact-row blocks + packed
+    one-round shape, exact windows of at most 1024 rows are attended by the packed blocks or the merge
+    (no partials of their own) unless the packed blocks leave slots for exact-row blocks beside them;
+    longer ones are blocks of 64 rows dispatched after the packed blocks.  The workspace holds S1 * rows * (d + 2) + 2 * rows floats per (b, h), S1 = exact-row blocks + packed
     splits (partials, then each row's max and sum)."""
     from kvq import _lib
     lib = _lib.load()
