@@ -268,18 +268,20 @@ __device__ void exact_block(const DecodeParams& p, int bh, int sidx, float* smem
     u32x4 kw[kW], vw[kW];
     int64_t pos;
   };
-  // loads of row i (clamped to the wavefront's last row, so every load is unconditional)
+  // loads of row i, through buffers that end at the wavefront's last row: every load is unconditional, and rows past
+  // it are zeros (a value row's infinity must not meet their weight of zero)
+  constexpr int kRowBytes = kD * (DT == KVQ_F32 ? 4 : 2);
+  const uint32_t held = static_cast<uint32_t>(w1 * kRowBytes);
+  const __amdgpu_buffer_rsrc_t rk = make_rsrc(static_cast<const uint8_t*>(p.k_exact) + kbase * (kRowBytes / kD), held);
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(static_cast<const uint8_t*>(p.v_exact) + kbase * (kRowBytes / kD), held);
   auto load_rows = [&](int i, Rows& x) {
-    i = min(i, w1 - 1);
-    const int64_t off = (kbase + static_cast<int64_t>(i) * kD + 8 * part) * (DT == KVQ_F32 ? 4 : 2);
-    const u32x4* kp = reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(p.k_exact) + off);
-    const u32x4* vp = reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(p.v_exact) + off);
+    const int off = i * kRowBytes + part * (kRowBytes / 16);
 #pragma unroll
     for (int w = 0; w < kW; ++w) {            // streamed once: non-temporal
-      x.kw[w] = __builtin_nontemporal_load(kp + w);
-      x.vw[w] = __builtin_nontemporal_load(vp + w);
+      x.kw[w] = __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16 * w, 0, 2);
+      x.vw[w] = __builtin_amdgcn_raw_buffer_load_b128(rv, off + 16 * w, 0, 2);
     }
-    x.pos = masked ? p.exact_pos[i] : 0;
+    x.pos = masked ? p.exact_pos[min(i, w1 - 1)] : 0;
   };
   auto to_f32 = [&](const u32x4 (&w)[kW], float (&x)[8]) {
     if constexpr (DT == KVQ_F32) {

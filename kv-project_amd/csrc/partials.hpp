@@ -287,6 +287,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(MergeArgs a) 
 template <int R, int DT, int NS>
 __global__ __launch_bounds__(256) void merge_rows_wave_kernel(MergeArgs a, int n_rows) {
   constexpr int D = 128;
+  constexpr int kLeast = NS == 8 ? 1 : NS == 16 ? 9 : NS == 32 ? 17 : 33;   // the fewest partials it is launched for
   const int row = static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6);
   if (row >= n_rows) return;
   const int lane = threadIdx.x & 63;
@@ -313,8 +314,9 @@ __global__ __launch_bounds__(256) void merge_rows_wave_kernel(MergeArgs a, int n
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));   // 0 past S_all
-    ox = __builtin_fmaf(ws, ov[s].x, ox);
-    oy = __builtin_fmaf(ws, ov[s].y, oy);
+    const bool held = s < kLeast || s < S_all;          // past S_all: the last partial again, its infinities too
+    ox = __builtin_fmaf(ws, held ? ov[s].x : 0.0f, ox);
+    oy = __builtin_fmaf(ws, held ? ov[s].y : 0.0f, oy);
   }
   const int b = bh / a.Hkv, h = bh % a.Hkv;
   const int hq = h * a.rep + r / a.Tq, t = r % a.Tq;

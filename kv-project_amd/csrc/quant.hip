@@ -689,7 +689,7 @@ __global__ __launch_bounds__(256) void kivi_quant_values_p4(
 // A whole context straight into the decode cache (PackedKIVICache's layout, 4 bits, d == 128): every
 // output byte is written once, padding included, so nothing has to be cleared, packed, copied or
 // re-tiled behind these two launches.  Bound by memory: rows in, codes and metadata out.  At
-// 4 x 8 x 32845 bf16 rows a side (0.69 GB) the pair takes 140-142 us, 4.9 TB/s, which a plain 2 GiB copy
+// 4 x 8 x 32845 bf16 rows a side (0.69 GB) the pair takes 140-145 us by box, 4.8-4.9 TB/s, which a plain 2 GiB copy
 // reaches as well; the quantisers, the packed rows' copy into the cache, the value re-tiling and the fills
 // that it replaces, 19 launches, took 595 us.
 

@@ -154,3 +154,21 @@ def test_every_exact_row_counts_once(B, Hkv, rep, Tq, T, n_exact):
     err = float((got - want).abs().max())
     print(f"n_exact {n_exact}: err {err:.2e}, least row {least:.2e}", flush=True)
     assert err <= 0.1 * least
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,n_exact", [(700, 1), (700, 17), (700, 30), (700, 33), (5000, 90), (1400, 1300)])
+def test_infinite_value_of_an_exact_row(T, n_exact, dtype):
+    """An infinity in a visible exact row's value is its channel's output, and no other channel's: lanes that hold no row
+    of a block's last ones, and a merge's slots that hold no partial, must not multiply it by their weight of zero."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(n_exact)
+    for row in {0, n_exact // 2, n_exact - 1}:
+        K, V = _rows(g, 1, 2, T, 128, dtype=dtype), _rows(g, 1, 2, T, 128, dtype=dtype)
+        V[:, :, T - n_exact + row, 7] = float("inf")
+        c = kvq.PackedKIVICache.from_context(K, V, window=n_exact, group_k=32, group_v=32)
+        q = _rows(g, 1, 4, 1, 128, dtype=dtype)
+        few = torch.empty((kvq.workspace_floats(1, 4, 2, 1, 128, c.n_q, 0, 32, 32),), device="cuda")
+        for ws in (None, few)[:1 if n_exact > 1024 else 2]:              # beside the packed blocks, and inside them
+            out = kvq.kivi_decode(q, 0.1, c, workspace=ws)
+            assert torch.isposinf(out[..., 7]).all() and torch.isfinite(out[..., :7]).all() and torch.isfinite(out[..., 8:]).all()
