@@ -425,8 +425,11 @@ __device__ void retained_block(const DecodeParams& p, int bh, int sidx, float* s
     const int u = (x.t < 0 ? 0 : x.t) % 32;
     const int jj = 4 * (u / 16) + (u % 4);
     const int shift = 4 * kNibbleOfSlotD[jj];
-    const float sv = f16_to_f32(static_cast<uint16_t>(x.vmw & 0xffffu));
-    const float lv = f16_to_f32(static_cast<uint16_t>(x.vmw >> 16));
+    // a masked row's values are zeros: what position 0 holds (nothing yet, in a cache without packed rows) may be a
+    // NaN, which its weight of zero would keep
+    const uint32_t vmw = x.t >= 0 ? x.vmw : 0u;
+    const float sv = f16_to_f32(static_cast<uint16_t>(vmw & 0xffffu));
+    const float lv = f16_to_f32(static_cast<uint16_t>(vmw >> 16));
 #pragma unroll
     for (int e = 0; e < 8; ++e) vx[e] = __fadd_rn(__fmul_rn(static_cast<float>((x.vw[e] >> shift) & 15u), sv), lv);
     attend_row<R>(qv, kx, vx, x.t >= 0 ? 0xffffffffu : 0u, m, l, o);

@@ -288,3 +288,24 @@ def test_retained_decode_rejects_bad_inputs():
     idx = torch.zeros((1, 2, 5), dtype=torch.int32, device="cuda")
     with pytest.raises(kvq.KVQError):
         kvq.retained_decode(q, 0.1, cache, idx, workspace=torch.empty((4,), dtype=torch.float32, device="cuda"))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_retained_decode_masked_rows_read_nothing(dtype):
+    """Masked retained positions over a cache without packed rows: whatever its placeholder fields hold, the output is
+    that of the exact rows alone."""
+    import kvq
+    g = torch.Generator(device="cuda").manual_seed(5)
+    k, v = (torch.randn((1, 2, 40, 128), generator=g, device="cuda").to(dtype) for _ in "kv")
+    q = torch.randn((1, 8, 1, 128), generator=g, device="cuda").to(dtype)
+    c = kvq.exact_rows_cache(k, v, 40)
+    idx = torch.tensor([-1, 0, 7, 1 << 30] * 5, dtype=torch.int32, device="cuda").expand(1, 2, 20).contiguous()
+    outs = []
+    for fill in (0, 0xff, 0x7c):                                        # zeros, NaN, infinities among them
+        for f in (c.kc, c.vc, c.k_lo, c.k_sc, c.vmeta):
+            f.view(torch.uint8).fill_(fill)
+        outs.append(kvq.retained_decode(q, 0.1, c, idx))
+    assert torch.isfinite(outs[0].float()).all()
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    want = kvq.kivi_decode(q, 0.1, c)
+    torch.testing.assert_close(outs[0], want, rtol=0, atol=1e-5 if dtype == torch.float32 else 2 ** -8)
