@@ -102,9 +102,13 @@ class DecodeCtl:
 
 
 def _append_takes(c: PackedKIVICache, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """Whether kvq_exact_append takes these rows: on the cache's device, of its dtype and sizes, in 16-byte pieces
-    (every other form is converted and copied by torch)."""
+    """Whether kvq_exact_append takes these rows: on the cache's device, of its dtype and sizes, in 16-byte pieces,
+    into buffers and positions that hold cap_e rows (every other form is converted, copied or refused by torch)."""
     B, H, _, d = c.k_exact.shape
+    pos = c.exact_pos
+    if (c.v_exact.shape != c.k_exact.shape or pos is None or pos.dim() != 1 or pos.numel() < c.cap_e or pos.dtype != torch.int64
+            or not pos.is_contiguous() or pos.device != c.k_exact.device):
+        return False
     es = c.k_exact.element_size()
     t = k.shape[2]
     for x, y in ((k, c.k_exact), (v, c.v_exact)):
