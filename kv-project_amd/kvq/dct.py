@@ -70,8 +70,8 @@ def dct_encode(x: torch.Tensor, for_values: bool = False):
 def _compress_takes(K: torch.Tensor, V: torch.Tensor) -> bool:
     """Whether kvq_dct_compress takes this context as it lies: head_dim 128, K and V alike, rows of 16-byte
     pieces.  Every other form is copied to contiguous blocks and coded a side at a time (dct_encode)."""
-    if (K.shape != V.shape or K.dtype != V.dtype or K.dtype not in _lib.DTYPE_CODE or K.shape[3] != 128
-            or K.numel() == 0 or K.shape[0] * K.shape[1] >= 1 << 24 or K.shape[2] >= 1 << 31):
+    if (K.shape != V.shape or K.dtype != V.dtype or K.device != V.device or K.dtype not in _lib.DTYPE_CODE
+            or K.shape[3] != 128 or K.numel() == 0 or K.shape[0] * K.shape[1] >= 1 << 24 or K.shape[2] >= 1 << 31):
         return False
     es = K.element_size()
     return all(x.stride(3) == 1 and x.data_ptr() % 16 == 0 and not any(s * es % 16 for s in x.stride()[:3]) for x in (K, V))

@@ -28,8 +28,8 @@ def _round_up(x: int, m: int) -> int:
 def _compress_takes(K: torch.Tensor, V: torch.Tensor, group_k: int, group_v: int, cap_t: int) -> bool:
     """Whether kvq_kivi_compress takes this context: head_dim 128, groups of 32, 64 or 128, K and V alike, rows
     of 16-byte pieces that do not overlap.  Every other form is quantised, packed and tiled in separate steps."""
-    if (K.shape != V.shape or K.dtype != V.dtype or K.dtype not in _lib.DTYPE_CODE or K.shape[3] != 128 or K.numel() == 0
-            or group_k not in (32, 64, 128) or group_v not in (32, 64, 128)):
+    if (K.shape != V.shape or K.dtype != V.dtype or K.device != V.device or K.dtype not in _lib.DTYPE_CODE
+            or K.shape[3] != 128 or K.numel() == 0 or group_k not in (32, 64, 128) or group_v not in (32, 64, 128)):
         return False
     B, H, T, d = K.shape
     if B * H >= 1 << 24 or cap_t >= 1 << 31 or B * H * (cap_t // 32) >= 1 << 30:

@@ -57,3 +57,11 @@ def test_positions_too_short_are_refused():
     assert st.cache.exact_pos.tolist() == [1 << 62] * 5 + [5, 6] and st.cache.n_exact == 7
     with pytest.raises(RuntimeError):
         st.append(x, x, torch.tensor([7, 8]))
+
+
+def test_contexts_of_two_devices():
+    """Keys and values of one device only: the kernels read both sides with one device's stream."""
+    from kvq import dct, decode
+    x = torch.zeros(1, 2, 96, 128)
+    assert decode._compress_takes(x, x, 64, 64, 128) and dct._compress_takes(x, x)
+    assert not decode._compress_takes(x, x.to("meta"), 64, 64, 128) and not dct._compress_takes(x, x.to("meta"))
