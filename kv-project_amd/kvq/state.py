@@ -104,17 +104,19 @@ class DecodeCtl:
 def _append_takes(c: PackedKIVICache, k: torch.Tensor, v: torch.Tensor) -> bool:
     """Whether kvq_exact_append takes these rows: on the cache's device, of its dtype and sizes, in 16-byte pieces,
     into buffers and positions that hold cap_e rows (every other form is converted, copied or refused by torch)."""
-    B, H, _, d = c.k_exact.shape
-    pos = c.exact_pos
-    if (c.v_exact.shape != c.k_exact.shape or pos is None or pos.dim() != 1 or pos.numel() < c.cap_e or pos.dtype != torch.int64
-            or not pos.is_contiguous() or pos.device != c.k_exact.device):
+    ke, pos = c.k_exact, c.exact_pos
+    B, H, cap, d = ke.shape
+    es, device, dtype, t = ke.element_size(), ke.device, ke.dtype, k.shape[2]
+    if (pos is None or pos.dtype != torch.int64 or pos.dim() != 1 or pos.shape[0] < cap or pos.device != device
+            or not pos.is_contiguous() or c.v_exact.shape != ke.shape):
         return False
-    es = c.k_exact.element_size()
-    t = k.shape[2]
-    for x, y in ((k, c.k_exact), (v, c.v_exact)):
-        if (x.device != y.device or x.dtype != y.dtype or tuple(x.shape) != (B, H, t, d) or x.stride(3) != 1
-                or x.data_ptr() % 16 or y.data_ptr() % 16 or not y.is_contiguous() or x.requires_grad
-                or any(s * es % 16 for s in x.stride()[:3])):
+    for x, y in ((k, ke), (v, c.v_exact)):
+        if x.shape != (B, H, t, d) or x.dtype != dtype or y.dtype != dtype or x.device != device or y.device != device:
+            return False
+        s0, s1, s2, s3 = x.stride()
+        # one test for three strides: 16 / es is a power of two
+        if (s3 != 1 or (s0 | s1 | s2) * es % 16 or x.data_ptr() % 16 or y.data_ptr() % 16 or not y.is_contiguous()
+                or x.requires_grad):
             return False
     return t > 0 and B * H > 0 and d * es % 16 == 0
 
