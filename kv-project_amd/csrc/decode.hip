@@ -1277,8 +1277,8 @@ inline SplitPlan plan_split(int64_t B, int64_t Hq, int64_t Hkv, int64_t Tq, int6
 // block's stream (split of 2905 packed + 96 exact rows, 8 (b, h), group 32: 8 query rows 11.7 -> 9.1 us,
 // 4 rows 8.1 -> 5.8, 1 row 5.6 -> 4.6; the packed rows alone 7.8, 5.9, 4.6).  Only while the row's partials
 // stay within the one-wavefront merge.  Whole steps of 175 forms that it takes (1 to 64 (b, h), 1 to 8
-// rows, value groups 32 to 128, 66 to 23,000 packed and 1 to 840 exact rows, 16-bit and fp32): 0.62 to
-// 1.003 of the fused pass's time.  Its partials need workspace that the fused pass does not.
+// rows, value groups 32 to 128, 66 to 23,000 packed and 1 to 840 exact rows, 16-bit and fp32): 0.61 to
+// 1.01 of the fused pass's time.  Its partials need workspace that the fused pass does not.
 inline bool place_beside(SplitPlan* sp, int64_t n_exact) {
   if (sp->fused_per == 0) return false;
   const int64_t nb = std::min<int64_t>(sp->room, (n_exact + 15) / 16);

@@ -20,8 +20,8 @@ namespace {
 
 constexpr int kMergeThreadsEx = 256;              // threads of the merge blocks
 // The most partials of a row that one wavefront merges.  At 33, 40 and 48 partials, 1 to 512 (b, h) of 1 to 8 rows,
-// against the workgroup form: a single row 3.9 -> 4.05 us, 2 to 256 rows within 5% (4.1-4.6 us both), from
-// 512 rows on 0.53-0.90 of it (4096 rows of 48: 23.4 -> 16.5).  At 100 partials slower, between not measured.
+// against the workgroup form: a single row 3.9 -> 4.2 us, 2 to 256 rows within 7% (4.1-4.6 us both), from
+// 512 rows on 0.53-0.92 of it (4096 rows of 48: 23.4 -> 16.8).  At 100 partials slower, between not measured.
 constexpr int kWaveMergePartials = 48;
 
 // Exact rows (the residual window, appended tokens) a merge may attend itself instead of reading
